@@ -970,6 +970,7 @@ def test_deposit_mass_matrix_symmetry():
     assert n_checked > 10000
 
 
+@needs_ref
 def test_reference_effective_cutoff_islands():
     """The reference's IntegrateEffectiveCutoff through the harness against
     the closed form Rc_eff = Rc_upper - (allowed width inside the penumbra)

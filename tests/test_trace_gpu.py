@@ -13,6 +13,7 @@ from oracle import oracle as O
 from tests import tracer_setup as TS
 
 pytestmark = pytest.mark.gpu
+needs_ref = pytest.mark.skipif(not O.ref_available(), reason="oracle/_ref not built (no reference tree)")
 
 
 def _oparams(P):
@@ -222,6 +223,7 @@ def test_bracketed_scan_extreme_widths(gpu_ctx, half):
         assert traced.all()
 
 
+@needs_ref
 def test_refine_cutoff_matches_reference_bisection(gpu_ctx):
     """Batched bisection (FP64) vs the reference's RefineCutoffTransition
     compiled from CutoffBandSearch.h, driven by the oracle tracer: the same
@@ -253,6 +255,7 @@ def test_refine_cutoff_matches_reference_bisection(gpu_ctx):
     print(f"refined {len(sel)} upper cutoffs, {int(it.sum())} midpoints")
 
 
+@needs_ref
 def test_penumbra_scan_matches_reference_chain(gpu_ctx):
     """PENUMBRA_SCAN (FP64) for penumbral directions: the GPU chain (full
     scan, band topology, batched refinement of both transitions, batched
