@@ -25,6 +25,7 @@ constexpr int NODE_VALS = 3 + 243;     // per-node J + mass-matrix row block
 constexpr int CELL_STRIDE_MOMENT = 272;  // 17 lines
 constexpr int NODE_STRIDE = 256;         // 16 lines
 constexpr int MAX_SPEC = 8;
+constexpr int64_t PACK_DOUBLES = (int64_t)1 << 23;  // staging of packed J and M columns (64 MiB)
 
 // Device view of the block mesh (leaf blocks of the AMR octree).
 struct MeshView {
@@ -182,6 +183,7 @@ struct amps_ctx {
   // deposit
   double* d_cellpart = nullptr;
   double* d_nodeout = nullptr;
+  double* d_pack = nullptr;    // [PACK_DOUBLES] J or M columns on their way to the host
   int* d_ecsim_nbr = nullptr;  // [nnodes][27] neighbour nodes of the ECSIM stencil, -1 outside
   // ECSIM field equation (ecsim_field.hip)
   uint8_t* d_ecsim_bnd = nullptr;  // [nnodes] 1: corner on the domain boundary

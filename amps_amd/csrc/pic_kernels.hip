@@ -307,6 +307,18 @@ INST_PUSH32(AMPS_MOVER_BORIS, 4)
 // run-length aggregation (ballot + lane masks) so that one atomic serves a
 // whole run of equal keys; deleted particles are dropped.
 // ======================================================================
+// W columns of the [node][NODE_STRIDE] rows as a packed array (n = nodes * W)
+template <int W>
+__global__ __launch_bounds__(256) void k_pack_cols(int64_t n, const double* __restrict__ rows,
+                                                    double* __restrict__ out) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t r = i / W;
+  out[i] = rows[r * NODE_STRIDE + (i - r * W)];
+}
+template __global__ void k_pack_cols<3>(int64_t, const double*, double*);
+template __global__ void k_pack_cols<243>(int64_t, const double*, double*);
+
 __global__ __launch_bounds__(256) void k_fill_int(int* a, int64_t n, int val) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
