@@ -1094,7 +1094,10 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceView a) {
         }
       }
     }
-    if (__ballot(has) == 0ull) break;
+    if (__ballot(has) == 0ull) {
+      if (!BRK || __ballot(!done) == 0ull) break;
+      continue;  // every draw of these rounds was skipped
+    }
     // a wavefront whose lanes all wait for bracket results yields its issue slots
     if (BRK && __ballot(has && !wait) == 0ull) __builtin_amdgcn_s_sleep(64);
     for (int k = 0; k < a.chunk && has && !wait; k++) {
@@ -1180,6 +1183,8 @@ __global__ __launch_bounds__(256) void k_trace_persistent(TraceView a) {
 
 }  // namespace
 
+#include "trace_fast.h"
+
 // =====================================================================
 // host side
 // =====================================================================
@@ -1195,11 +1200,14 @@ struct TraceState {
   int* d_cut = nullptr;
   int* d_pend = nullptr;
   int* d_status = nullptr;
+  int* d_stop = nullptr;
+  int* d_open = nullptr;
+  uint32_t* d_item_steps = nullptr;
   int8_t* d_states = nullptr;
   amps_trace_result* d_out = nullptr;
   amps_trace_exit* d_exits = nullptr;
   size_t b_x0 = 0, b_dir = 0, b_R = 0, b_lo = 0, b_hi = 0, b_cut = 0, b_states = 0, b_out = 0, b_exits = 0;
-  size_t b_pend = 0, b_status = 0;
+  size_t b_pend = 0, b_status = 0, b_stop = 0, b_open = 0, b_item_steps = 0;
   int grid_waves = 0;  // persistent grid size (workgroups); 0 = 8 per CU
   int chunk = 32;      // steps between queue refills
 };
@@ -1219,6 +1227,9 @@ void trace_free(amps_ctx* c) {
   (void)hipFree(t->d_cut);
   (void)hipFree(t->d_pend);
   (void)hipFree(t->d_status);
+  (void)hipFree(t->d_stop);
+  (void)hipFree(t->d_open);
+  (void)hipFree(t->d_item_steps);
   (void)hipFree(t->d_states);
   (void)hipFree(t->d_out);
   (void)hipFree(t->d_exits);
@@ -1309,6 +1320,32 @@ static void launch64(amps_ctx* c, const TraceView& a, dim3 g, dim3 blk) {
   }
 }
 
+// The launches that k_trace_mode covers (trace_fast.h): the FP32 Boris mover
+// and, inside the range of its arithmetic, the FP64 one with the analytic
+// field and the legacy adaptive selector.
+template <class S>
+static void launch_fast(amps_ctx* c, TraceState* t, const typename S::View& v, const TraceView& a, int precision) {
+  ScanWork w;
+  std::memset(&w, 0, sizeof(w));
+  w.chunk = a.chunk, w.nR = a.nR, w.W = a.nbin_item, w.retry = a.P.retry;
+  w.nitems = a.nitems, w.nloc = a.mode == TRACE_MODE_LIST ? 1 : a.nloc;
+  w.inv_nloc = 1.0 / (double)w.nloc;
+  w.queue = a.queue, w.steps_total = a.steps_total;
+  w.x0 = a.x0, w.dir = a.dir, w.R = a.R, w.grid = a.grid, w.lo = a.lo, w.hi = a.hi;
+  w.out = a.out, w.states = a.states, w.cutoff = a.cutoff, w.pend = a.pend, w.status = a.status;
+  w.stop = a.stop, w.item_steps = a.item_steps;
+  if (a.mode == TRACE_MODE_UPPER) w.nitems = a.nloc * a.nR;  // every bin an item, those outside a bracket skipped
+  if (a.mode == TRACE_MODE_BRACKET) {
+    w.nitems = a.nloc * a.nbin_item;  // the rescans are handed out by ticket
+    w.open_list = t->d_open;
+    w.tickets = a.queue + 1, w.n_open = a.queue + 2, w.bracket_left = a.queue + 3;
+  }
+  const int wgs = t->grid_waves > 0 ? t->grid_waves : c->n_cu * fast_wgs_per_cu(a.mode, precision, a.nloc, c->n_cu);
+  launch_mode<S>(c, v, w, a.mode, dim3(wgs));
+  if (a.mode == TRACE_MODE_UPPER)
+    hipLaunchKernelGGL(k_upper_read, dim3((unsigned)((a.nloc + 255) / 256)), dim3(256), 0, c->stream, w);
+}
+
 static int launch(amps_ctx* c, TraceState* t, TraceView& a, int precision) {
   if (precision == AMPS_FP32 && a.P.mover != MV_BORIS && a.P.mover != MV_HC4)
     return fail(AMPS_E_ARG, "trace: the FP32 path runs the BORIS and HC4 movers only");
@@ -1319,7 +1356,35 @@ static int launch(amps_ctx* c, TraceState* t, TraceView& a, int precision) {
     a.mesh = c->mv;
     a.Bm = c->d_Bm;
   }
-  HIP_TRY(hipMemsetAsync(t->d_queue, 0, 8, c->stream));
+  // draws, rescan tickets, opened locations; bracket items outstanding
+  const unsigned long long q0[4] = {0, 0, 0, (unsigned long long)(a.nloc * a.nbin_item)};
+  HIP_TRY(hipMemcpyAsync(t->d_queue, q0, sizeof(q0), hipMemcpyHostToDevice, c->stream));
+  const bool lim = a.P.dist_limiter || a.P.dt_floor;
+  Fast64View V;
+  Fast32View W;
+  bool fast = !a.exits && (a.mode != TRACE_MODE_UPPER || a.item_steps);
+  fast = fast && (precision == AMPS_FP32 ? fast32_view(a, W) : fast64_view(a, V));
+  if (fast) {
+    tbegin(c);
+    const int k = (a.P.outer_sphere ? 2 : 0) + (lim ? 1 : 0);
+    if (precision == AMPS_FP32)
+      switch (k) {
+        case 0: launch_fast<Fast32<false, false>>(c, t, W, a, precision); break;
+        case 1: launch_fast<Fast32<false, true>>(c, t, W, a, precision); break;
+        case 2: launch_fast<Fast32<true, false>>(c, t, W, a, precision); break;
+        default: launch_fast<Fast32<true, true>>(c, t, W, a, precision);
+      }
+    else
+      switch (k) {
+        case 0: launch_fast<Fast64<false, false>>(c, t, {V, a.P}, a, precision); break;
+        case 1: launch_fast<Fast64<false, true>>(c, t, {V, a.P}, a, precision); break;
+        case 2: launch_fast<Fast64<true, false>>(c, t, {V, a.P}, a, precision); break;
+        default: launch_fast<Fast64<true, true>>(c, t, {V, a.P}, a, precision);
+      }
+    HIP_TRY(hipGetLastError());
+    tend(c, AMPS_K_TRACE);
+    return 0;
+  }
   int grid = t->grid_waves;
   if (grid <= 0) {
     hipDeviceProp_t p;
@@ -1819,6 +1884,8 @@ extern "C" int amps_gpu_cutoff_scan(amps_ctx* c, const amps_trace_params* P, int
     // every location starts in its bracket phase with W outstanding bins
     if (int r = ensure((void**)&t->d_pend, &t->b_pend, sizeof(int) * nloc)) return r;
     if (int r = ensure((void**)&t->d_status, &t->b_status, sizeof(int) * nloc)) return r;
+    if (int r = ensure((void**)&t->d_open, &t->b_open, sizeof(int) * nloc)) return r;
+    HIP_TRY(hipMemsetAsync(t->d_open, 0xff, sizeof(int) * nloc, c->stream));
     pend.assign((size_t)nloc, nbin_item);
     HIP_TRY(hipMemcpyAsync(t->d_pend, pend.data(), sizeof(int) * nloc, hipMemcpyHostToDevice, c->stream));
     HIP_TRY(hipMemsetAsync(t->d_status, 0, sizeof(int) * nloc, c->stream));
@@ -1830,6 +1897,14 @@ extern "C" int amps_gpu_cutoff_scan(amps_ctx* c, const amps_trace_params* P, int
   a.nloc = nloc;
   a.pend = t->d_pend;
   a.status = t->d_status;
+  if (mode == AMPS_SCAN_UPPER && nloc * nR <= ((int64_t)1 << 29)) {
+    // every bin an item of its own (trace_fast.h): at most 2 GiB of step counts
+    if (int r = ensure((void**)&t->d_stop, &t->b_stop, sizeof(int) * nloc)) return r;
+    if (int r = ensure((void**)&t->d_item_steps, &t->b_item_steps, sizeof(uint32_t) * nloc * nR)) return r;
+    HIP_TRY(hipMemsetAsync(t->d_stop, 0xff, sizeof(int) * nloc, c->stream));
+    a.stop = t->d_stop;
+    a.item_steps = t->d_item_steps;
+  }
   a.nbin_item = nbin_item;
   a.nR = nR;
   a.x0 = t->d_x0;

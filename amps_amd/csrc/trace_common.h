@@ -35,6 +35,9 @@ struct TraceView {
   int64_t nloc;
   int* pend;
   int* status;
+  // UPPER mode, every bin an item (null: one lane walks a location's bins)
+  int* stop;             // highest not-allowed bin found, -1 none
+  uint32_t* item_steps;  // [nloc][nR]
   // mesh field (field_model 1): the block mesh and the compact interior-cell B
   MeshView mesh;
   const double* Bm;

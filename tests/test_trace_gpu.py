@@ -484,3 +484,96 @@ def test_trap_detector_traces_bitexact(gpu_ctx, mover, policy):
     _same(g, o)
     t = o["termination"]
     assert (t == 2).sum() > 100 and (t == 1).sum() > 10 and (t == 0).sum() > 5
+
+
+def _edge_tasks():
+    """Random trajectories and starts at the edges of the tracer's ranges:
+    inside the inner sphere, outside the box, on an axis, zero and tiny
+    momentum or direction components, a not-a-number."""
+    x, d, R = _random_tasks(1500, 21)
+    re = CU.RE_DIPOLE
+    ex = np.array([[0.0, 0.0, 1.2 * re], [1.2 * re, 0.0, 0.0], [0.5 * re, 0.0, 0.0], [60 * re, 0.0, 0.0],
+                   [1.1 * re, 1e-200, 0.0], [1.2 * re, 0.0, 0.0], [1.1 * re, 0.0, 0.0], [0.0, 1.3 * re, 0.0],
+                   [np.nan, 0.0, 0.0], [1e70, 0.0, 0.0], [1.1 * re, 0.0, 0.0]])
+    ed = np.array([[0.0, 0.0, -1.0], [-1.0, 0.0, 0.0], [0.0, 1.0, 0.0], [1.0, 0.0, 0.0], [0.0, -1.0, 0.0],
+                   [0.0, 0.0, 0.0], [-1.0, 1e-310, 0.0], [0.0, -1e-180, -1.0], [1.0, 0.0, 0.0], [1.0, 0.0, 0.0],
+                   [-1.0, 0.0, 0.0]])
+    eR = np.array([5.0, 5.0, 5.0, 5.0, 2.0, 1.0, 3.0, 3.0, 1.0, 1.0, 1e-120])
+    return np.concatenate([x, ex]), np.concatenate([d, ed]), np.concatenate([R, eR])
+
+
+@pytest.mark.parametrize("kw", [
+    dict(), dict(outer_sphere=True, r_outer_Re=25.0), dict(dist_limiter=False, dt_floor=False),
+    dict(dist_limiter=False, dt_floor=False, outer_sphere=True, r_outer_Re=20.0, max_distance_Re=-1.0, bz_T=-5e-9,
+         tilt_deg=10.0),
+    dict(dt_floor=False, reversed_charge=True), dict(moment_scale=0.0, bz_T=1e-9),
+    dict(moment_scale=0.0, max_time=0.5), dict(moment_scale=1e-30, max_time=0.5, dist_limiter=False),
+    dict(max_time=1e-3, dt_floor=False), dict(max_steps=3, retry=2), dict(dt_trace=1e-6, max_steps=50),
+    dict(r_inner_Re=0.0), dict(adaptive=False), dict(mass_amu=1e-60), dict(charge_e=26, mass_amu=56.0)])
+def test_boris_kernels_agree(gpu_ctx, kw):
+    """The lean Boris kernel (trace_batch) against the general one, which
+    trace_batch_ex runs, over its options and at the edges of its ranges: the
+    same bits in every field."""
+    kw = dict(dict(max_steps=2000, max_time=60.0), **kw)
+    P = CU.legacy_params(**kw)
+    x, d, R = _edge_tasks()
+    print(f"trace options {kw} n={len(R)}", flush=True)
+    a, sa = CU.trace_batch(gpu_ctx, P, x, d, R)
+    b, _, sb = CU.trace_batch_ex(gpu_ctx, P, x, d, R)
+    for f in a.dtype.names:
+        assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype.kind == "f"), f
+    assert sa == sb
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("bracket", [False, True])
+@pytest.mark.parametrize("retry", [0, 2])
+def test_upper_scan_is_the_sequential_one(gpu_ctx, precision, bracket, retry):
+    """AMPS_SCAN_UPPER, whose bins are traced side by side: states, cutoff
+    bins and step total as a downward walk over the trajectories one by one
+    gives them (brackets of different widths, retried terminations)."""
+    P = CU.config2_params()
+    P.max_steps = 3000
+    P.retry = retry
+    pts, lat, lon = CU.config2_points(nlon=9, nlat=7)
+    zen, az = CU.config2_directions(3)
+    dirs = CU.arrival_dirs(pts, zen, az).reshape(-1, 3)
+    x0 = np.repeat(pts, len(zen), axis=0)
+    nR = 24
+    grid = CU.build_search_grid(0.1, 20.0, nR)
+    n = len(x0)
+    lo, hi = np.zeros(n, np.int32), np.full(n, nR - 1, np.int32)
+    if bracket:
+        rng = np.random.default_rng(4)
+        lo = rng.integers(0, nR, n).astype(np.int32)
+        hi = np.minimum(lo + rng.integers(0, 9, n), nR - 1).astype(np.int32)
+    print(f"upper scan precision {precision} bracket {bracket} retry {retry} n={n}", flush=True)
+    st, bins, steps = CU.cutoff_scan(gpu_ctx, P, x0, dirs, grid, mode=CU.SCAN_UPPER, precision=precision,
+                                     lo=lo if bracket else None, hi=hi if bracket else None)
+    r, _ = CU.trace_batch(gpu_ctx, P, np.repeat(x0, nR, axis=0), np.repeat(dirs, nR, axis=0), np.tile(grid, n),
+                          precision=precision)
+    term = r["termination"].reshape(n, nR)
+    first = None
+    if retry:  # the first attempt's steps of the retried trajectories
+        Q = CU.config2_params()
+        Q.max_steps, Q.retry = 3000, 0
+        f, _ = CU.trace_batch(gpu_ctx, Q, np.repeat(x0, nR, axis=0), np.repeat(dirs, nR, axis=0), np.tile(grid, n),
+                              precision=precision)
+        first = np.where(r["retry_count"] > 0, f["steps"], 0).reshape(n, nR)
+    want = np.full((n, nR), -1, np.int8)
+    total = 0
+    for i in range(n):
+        for b in range(hi[i], lo[i] - 1, -1):
+            want[i, b] = 1 if term[i, b] == 0 else (0 if term[i, b] <= 5 else 2)
+            total += int(r["steps"].reshape(n, nR)[i, b]) + (int(first[i, b]) if retry else 0)
+            if want[i, b] != 1:
+                break
+    assert np.array_equal(st, want)
+    assert steps == total
+    for i in range(n):
+        if want[i, hi[i]] != 1:
+            w = -1 if hi[i] == nR - 1 else CU.BIN_ABOVE
+        else:
+            b = int(np.flatnonzero(want[i] == 1)[0])
+            w = CU.BIN_BELOW if b == lo[i] and lo[i] > 0 else b
+        assert bins[i] == w, (i, bins[i], w)
