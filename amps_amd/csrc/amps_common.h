@@ -190,6 +190,7 @@ struct amps_ctx {
   int* d_ecsim_cells8 = nullptr;   // [nnodes][8] cells at node + (ci, cj, ck), ci, cj, ck in {-1, 0}
   int* d_ecsim_noc = nullptr;      // [nblocks][729] node of each block corner
   double* d_ecsim_work = nullptr;  // field vectors, the Krylov basis and reduction partials
+  double* d_ecsim_sym = nullptr;   // the solve's matrix as planes, [14][9][nodes]
   size_t ecsim_work_len = 0;       // doubles allocated at d_ecsim_work
   // deterministic migration: the offsets of the current array layout, keys
   // with many movers, the movers' destinations and source positions, and the

@@ -85,44 +85,41 @@ __global__ __launch_bounds__(256) void k_ecsim_mass(const double* __restrict__ r
   }
 }
 
+__global__ __launch_bounds__(256) void k_ecsim_nbr(int64_t nn, int N, int* __restrict__ nbr) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= nn * 27) return;
+  const int64_t n = i / 27;
+  const int s = (int)(i - n * 27);
+  const int o[3] = {s % 3, (s / 3) % 3, s / 9};
+  int64_t j = n;
+  int64_t g = n, step = 1;
+  bool in = true;
+  for (int d = 0; d < 3; d++) {
+    const int a = o[d] == 0 ? 0 : (o[d] == 1 ? -1 : 1);
+    const int x = (int)(g % N) + a;
+    in = in && x >= 0 && x < N;
+    j += a * step;
+    g /= N;
+    step *= N;
+  }
+  nbr[i] = in ? (int)j : -1;
+}
+
 }  // namespace
 
 namespace amps {
-// neighbour table [nnodes][27] on the level-lmax lattice (-1: outside)
+// neighbour table [nnodes][27] (-1: outside) of a single-level mesh, whose
+// nodes are the points of an N^3 lattice in x, y, z order; built on the
+// device (a search per entry on the host took 1.5 s at 2.15 M nodes)
 int build_nbr(amps_ctx* c) {
   if (c->d_ecsim_nbr) return 0;
-  const int nb = c->mv.nb, lmax = c->mv.lmax;
-  const int64_t S = ((int64_t)1 << lmax) + 1;
   const int64_t nn = c->nnodes;
-  try {
-  std::vector<int64_t> h((size_t)nn, INT64_MAX);
-  for (int b = 0; b < nb; b++) {
-    const int64_t cs = ((int64_t)1 << (lmax - c->h_level[(size_t)b])) / NC;
-    for (int q = 0; q < NCORNER; q++) {
-      int64_t& hn = h[(size_t)c->h_node_of_corner[(size_t)b * NCORNER + q]];
-      hn = std::min(hn, cs);
-    }
-  }
-  const std::vector<int64_t>& keys = c->h_node_keys;
-  std::vector<int> nbr((size_t)nn * 27, -1);
-  static const int A[3] = {0, -1, 1};
-  for (int64_t n = 0; n < nn; n++) {
-    const int64_t k = keys[(size_t)n];
-    const int64_t g[3] = {k % S, (k / S) % S, k / (S * S)};
-    for (int s = 0; s < 27; s++) {
-      const int64_t o[3] = {g[0] + A[s % 3] * h[(size_t)n], g[1] + A[(s / 3) % 3] * h[(size_t)n],
-                            g[2] + A[s / 9] * h[(size_t)n]};
-      if (o[0] < 0 || o[1] < 0 || o[2] < 0 || o[0] >= S || o[1] >= S || o[2] >= S) continue;
-      const int64_t kk = (o[2] * S + o[1]) * S + o[0];
-      const auto it = std::lower_bound(keys.begin(), keys.end(), kk);
-      if (it != keys.end() && *it == kk) nbr[(size_t)n * 27 + s] = (int)(it - keys.begin());
-    }
-  }
-  HIP_TRY(hipMalloc(&c->d_ecsim_nbr, sizeof(int) * std::max<size_t>(27, nbr.size())));
-  HIP_TRY(hipMemcpy(c->d_ecsim_nbr, nbr.data(), sizeof(int) * nbr.size(), hipMemcpyHostToDevice));
-  } catch (const std::bad_alloc&) {
-    return fail(AMPS_E_RANGE, "amps_gpu_ecsim_mass_apply: out of host memory for the neighbour table");
-  }
+  const int N = (NC << c->h_level[0]) + 1;
+  if ((int64_t)N * N * N != nn) return fail(AMPS_E_STATE, "ecsim: the nodes are not a cubic lattice");
+  HIP_TRY(hipMalloc(&c->d_ecsim_nbr, sizeof(int) * std::max<size_t>(27, (size_t)nn * 27)));
+  hipLaunchKernelGGL(k_ecsim_nbr, dim3((unsigned)((nn * 27 + 255) / 256)), dim3(256), 0, c->stream, nn, N,
+                     c->d_ecsim_nbr);
+  HIP_TRY(hipGetLastError());
   return 0;
 }
 

@@ -134,3 +134,43 @@ def test_field_equation_needs_one_level(gpu_ctx):
     st.UpdateJMassMatrix(1e-3, copy_out=False)
     with pytest.raises(L.AmpsGpuError, match="single-level"):
         st.EcsimOperator(st.ecsim_params(1e-3), np.zeros((st.nnodes, 3)))
+
+
+@pytest.mark.parametrize("level,restart,max_iter,kernel", [(0, 1, 30, 2), (0, 3, 200, 0), (1, 9, 200, 1), (3, 25, 60, 2)])
+def test_gmres_packed_operator(gpu_ctx, level, restart, max_iter, kernel):
+    """The solver's packed symmetric operator and its Arnoldi steps: short
+    restarts, an iteration limit that ends the solve, nonzero right-hand sides
+    on the boundary, meshes on both sides of the threads-per-node rule (9^3 to
+    65^3 nodes), M from the exact and the moment deposit.  The reported
+    residual is the node-row operator's to rounding: 1e-12 of |b| covers the
+    243 products a row at condition numbers up to 10."""
+    ppc = 1 if level == 3 else 4
+    gpu_ctx.set_param("deposit_chunks", 4)
+    gpu_ctx.set_param("deposit_kernel", kernel)
+    gpu_ctx.set_param("deposit_exact", 1 if kernel == 1 else 0)
+    try:
+        mesh = M.uniform_mesh(level)
+        E, B = M.corner_fields(mesh)
+        dt = 0.1 / (np.max(np.linalg.norm(B, axis=-1)) / 0.01)
+        st = PicState(mesh, E, B, Species([-1.0, 1.0], [0.01, 1.0], [dt, dt]), ctx=gpu_ctx)
+        st.generate_particles(mesh.ncells * ppc, [0.05, 0.005], seed=level)
+        st.UpdateJMassMatrix(dt, copy_out=False)
+    finally:
+        gpu_ctx.set_param("deposit_exact", 0)
+        gpu_ctx.set_param("deposit_chunks", 4)
+        gpu_ctx.set_param("deposit_kernel", 2)
+        gpu_ctx.set_param("deposit_chunks", 12)
+    dx = mesh.cell_size()[0][0]
+    p = st.ecsim_params(dt, theta=0.5, cDt=2 * dx)
+    b = np.random.default_rng(level).normal(size=(st.nnodes, 3))
+    print(f"packed operator: {st.nnodes} nodes, restart {restart}", flush=True)
+    x, it, rr = st.EcsimSolve(p, b, tol=1e-9, max_iter=max_iter, restart=restart)
+    r = st.EcsimOperator(p, x) - b
+    true = np.linalg.norm(r) / np.linalg.norm(b)
+    assert 0 < it <= max_iter and (rr <= 1e-9 or it == max_iter)
+    assert abs(rr - true) <= 1e-12
+    x2, it2, rr2 = st.EcsimSolve(p, b, tol=1e-9, max_iter=max_iter, restart=restart)
+    assert np.array_equal(x, x2) and it2 == it and rr2 == rr
+    # a zero right-hand side
+    x0, it0, rr0 = st.EcsimSolve(p, np.zeros_like(b), tol=1e-9, max_iter=5, restart=2)
+    assert it0 == 0 and rr0 == 0.0 and not x0.any()
