@@ -79,10 +79,9 @@ struct PushSrc {
 // The migration's classification made by the push (a deterministic step
 // whose arrays have the layout of a previous compaction; lay null: none).
 // lay[] holds that layout's key offsets.  A survivor whose new key's old run
-// holds it (a stayer) sets its bit of the 64-aligned stayer mask word wmask
-// and counts in wcnt and in the push's count[]; a survivor that changes keys
-// (a mover) counts in cursor[] and takes its rank among its new key's movers
-// from that atomic, and is listed at slab[rank * nkeys + key] (rank-major:
+// holds it (a stayer) sets its bit of the 64-aligned stayer mask word wmask;
+// a survivor that changes keys (a mover) counts in cursor[], takes its rank
+// among its new key's movers from that atomic, and is listed at slab[rank * nkeys + key] (rank-major:
 // the first movers of neighbouring cells share cache lines), or, past the
 // slab, as (position, rank) in ovf[] (novf entries).
 constexpr int MIG_SLAB = 16;
@@ -94,7 +93,6 @@ struct PushMig {
   int2* ovf;
   int* novf;
   uint64_t* wmask;
-  int* wcnt;
 };
 
 // Synthetic-population generator arguments (k_generate).
@@ -127,6 +125,7 @@ struct amps_ctx {
   double* d_Bm = nullptr;   // [nb][512][3] Mode3D compact field of interior cells
   bool has_mode3d = false;
   amps::Faces faces{};
+  amps::Faces* d_faces = nullptr;
   int64_t nnodes = 0;
   std::vector<int32_t> h_node_of_corner;
   std::vector<int64_t> h_node_keys;
@@ -164,7 +163,8 @@ struct amps_ctx {
   int* d_ntiles = nullptr;
   int* d_tcount = nullptr;     // per-block tile count / offsets [nb+1]
   int64_t max_tiles = 0;
-  int tile = 8192;
+  int tile = 8192;             // particles per push tile when given, else push_tile()'s rule
+  bool tile_given = false;
   bool offsets_valid = false;  // d_offset describes the current order
   bool tiles_valid = false;    // d_tiles describes the current order
   int dep_nch = 12;            // deposit output chunks per cell (waves per workgroup)
@@ -175,7 +175,7 @@ struct amps_ctx {
   int mig_small = 64;          // movers per key sorted by one lane (more: a workgroup merge sort)
   int dep_waves = 2;           // eight-lanes-per-cell pass: register budget in wavefronts per SIMD (2 or 3)
   int dep_paired = 0;          // matrix-core cell pass: two wavefronts per SIMD in opposite phases
-  int push_waves = 1;          // 4: push kernels built for 4 waves per SIMD (128 VGPRs)
+  int push_waves = 4;          // 4: push kernels built for 4 waves per SIMD (128 VGPRs); 1: unbounded
   int dep_exact = 0;           // 1: unfused mul+add in the deposit (bit-exact order)
   int dep_kernel = 2;          // cell pass: 0 per-lane particle loop, 1 LDS record batches, 2 matrix cores,
                                // 3 eight lanes per cell
@@ -247,6 +247,11 @@ void trace_free(amps_ctx* c);
 void mlp_free(amps_ctx* c);
 // device-wide exclusive scan of n ints in place; total written to total_out
 int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* total_out);
+// the stayers before each mask word; the exclusive scan of the keys' new
+// particle counts (movers in cursor, stayers from the masks of the old runs)
+int scan_masks(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw);
+int scan_keys(amps_ctx* c, const int* cursor, const int* lay, const int* wscan, const uint64_t* wmask, int* offset,
+              int64_t nkeys);
 // ECSIM cell pass with LDS record batches (deposit.hip)
 int launch_deposit_cell_rec(amps_ctx* c, double dt, int nch);
 int launch_deposit_cell_mfma(amps_ctx* c, double dt);

@@ -15,11 +15,11 @@ using namespace amps;
 
 // kernels (pic_kernels.hip)
 template <int MOVER, bool BC, int W>
-__global__ void k_push_f64(MeshView, Faces, Species, const double*, const double*, const Tile*,
+__global__ void k_push_f64(MeshView, const Faces*, Species, const double*, const double*, const Tile*,
                            const int*, int, double, int64_t, double*, double*, const uint8_t*,
                            int*, int8_t*, const double*, int*, PushSrc, PushMig);
 template <int MOVER, int W>
-__global__ void k_push_f32(MeshView, Faces, Species, const double*, const double*, const Tile*,
+__global__ void k_push_f32(MeshView, const Faces*, Species, const double*, const double*, const Tile*,
                            const int*, int, double, int64_t, double*, float*, const uint8_t*, int*,
                            int8_t*, int*, PushSrc, PushMig);
 __global__ void k_fill_int(int*, int64_t, int);
@@ -27,15 +27,15 @@ __global__ void k_count_keys(const int*, const int*, const int8_t*, int*);
 __global__ void k_scatter(const int*, const int*, const int8_t*, const int*, int*, int64_t,
                           const double*, const double*, int, const uint8_t*, const int64_t*,
                           double*, double*, uint8_t*, int*, int64_t*);
-__global__ void k_copy_total(const int*, int*);
-__global__ void k_mig_classify(const int*, const int*, const int8_t*, const int*, int, const int*, int*, int*, int*,
+__global__ void k_mig_finish(int64_t, const int*, int*, int*, int64_t, int*);
+__global__ void k_mig_clear(int64_t, int*, int*, int64_t, uint64_t*, int*, int*);
+__global__ void k_mig_classify(const int*, const int*, const int8_t*, const int*, int, const int*, int*, int*,
                                uint64_t*);
 __global__ void k_mig_order(int64_t, int, int, const int*, const int*, int*, int*, int*, int, const int*,
                             const int*, const uint64_t*, int*);
 __global__ void k_mig_order_slab(int64_t, int, int, const int*, const int*, const int*, int*, int*, int*,
                                  const int*, const int*, const uint64_t*, int*);
 __global__ void k_mig_place(const int*, const int2*, const int*, const int*, const int*, int*);
-__global__ void k_add_ints(int64_t, int*, const int*);
 __global__ void k_mig_order_big(int64_t, int, const int*, const int*, int*, int*, int*, const int*);
 __global__ void k_mig_scatter(const int*, const int*, const int8_t*, const int*, const int*, const uint64_t*,
                               const int*, int64_t, const double*, const double*, int, const uint8_t*,
@@ -43,7 +43,7 @@ __global__ void k_mig_scatter(const int*, const int*, const int8_t*, const int*,
 __global__ void k_mig_dest(const int*, const int*, const int*, const int*, const uint64_t*, int64_t, int*);
 __global__ void k_mig_move(const int*, const int*, int64_t, const double*, const double*, int, const uint8_t*,
                            const int64_t*, const int*, double*, double*, uint8_t*, int64_t*, int*);
-__global__ void k_copy_ints(int64_t, const int*, int*);
+__global__ void k_tiles(int, int, const int*, Tile*, int*);
 __global__ void k_tile_count(int, int, const int*, int*);
 __global__ void k_tile_emit(int, int, const int*, const int*, Tile*, int*);
 template <int NCH, bool EXACT>
@@ -124,6 +124,8 @@ static void free_mesh(amps_ctx* c) {
   (void)hipFree(c->d_dxs);
   (void)hipFree(c->d_leaf);
   (void)hipFree(c->d_blk_lat);
+  (void)hipFree(c->d_faces);
+  c->d_faces = nullptr;
   c->d_blk_lat = nullptr;
   (void)hipFree(c->d_level);
   (void)hipFree(c->d_nbinfo);
@@ -243,6 +245,7 @@ extern "C" int amps_gpu_set_param(amps_ctx* c, const char* name, int64_t value) 
   if (n == "tile") {
     if (value < 64 || value > (1 << 20)) return fail(AMPS_E_ARG, "tile out of range [64, 2^20]");
     c->tile = (int)value;
+    c->tile_given = true;
     c->tiles_valid = false;
   } else if (n == "deposit_chunks") {
     if (!deposit_variant_ok(c->dep_kernel, value))
@@ -485,6 +488,8 @@ extern "C" int amps_gpu_set_mesh(amps_ctx* c, const amps_mesh_desc* desc, const 
   HIP_TRY(hipMalloc(&c->d_dxc, sizeof(double) * 3 * nb));
   HIP_TRY(hipMalloc(&c->d_dxs, sizeof(double) * 3 * nb));
   HIP_TRY(hipMalloc(&c->d_leaf, sizeof(int) * leaf.size()));
+  HIP_TRY(hipMalloc(&c->d_faces, sizeof(Faces)));
+  HIP_TRY(hipMemcpy(c->d_faces, &c->faces, sizeof(Faces), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->d_xmin, xmin.data(), sizeof(double) * 3 * nb, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->d_xmax, xmax.data(), sizeof(double) * 3 * nb, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->d_dxc, dxc.data(), sizeof(double) * 3 * nb, hipMemcpyHostToDevice));
@@ -670,19 +675,40 @@ int amps::alloc_particles(amps_ctx* c, int64_t n) {
   return 0;
 }
 
+// Particles per push workgroup.  Unless the caller set "tile": the largest
+// power of two in [256, 8192] with at least 2,048 tiles, two rounds of the
+// 1,024 workgroups that the push keeps resident.  8,192 at every size left
+// most of the chip idle below 2^24 particles (push in ms with 8192 and with
+// the rule: 16,384 particles 0.072 and 0.023, 2^20 0.151 and 0.068, 2.0 M
+// 0.269 and 0.169, 15.3 M FP32 0.866 and 0.822); from 2^24 on it is the best,
+// since every tile reads its block's 35 KB of fields (2^27: 7.6 ms with 1024,
+// 6.4 with 8192).
+static int push_tile(const amps_ctx* c) {
+  if (c->tile_given) return c->tile;
+  int t = 256;
+  while (t < 8192 && c->cap / (2 * t) >= 2048) t *= 2;
+  return t;
+}
+
 int amps::build_tiles(amps_ctx* c) {
   const int nb = c->mv.nb;
-  const int64_t need = nb + c->cap / c->tile + 2;
+  const int tile = push_tile(c);
+  const int64_t need = nb + c->cap / tile + 2;
   if (need > c->max_tiles) {
     (void)hipFree(c->d_tiles);
     c->d_tiles = nullptr;
     HIP_TRY(hipMalloc(&c->d_tiles, sizeof(Tile) * need));
     c->max_tiles = need;
   }
-  hipLaunchKernelGGL(k_tile_count, dim3((nb + 256) / 256), dim3(256), 0, c->stream, nb, c->tile,
+  if (nb <= 8192) {  // one launch where one workgroup keeps up (5-12 us; three launches above)
+    hipLaunchKernelGGL(k_tiles, dim3(1), dim3(1024), 0, c->stream, nb, tile, c->d_offset, c->d_tiles, c->d_ntiles);
+    c->tiles_valid = true;
+    return AMPS_OK;
+  }
+  hipLaunchKernelGGL(k_tile_count, dim3((nb + 256) / 256), dim3(256), 0, c->stream, nb, tile,
                      c->d_offset, c->d_tcount);
   if (int r = scan_exclusive(c, c->d_tcount, nb + 1, nullptr)) return r;
-  hipLaunchKernelGGL(k_tile_emit, dim3((nb + 256) / 256), dim3(256), 0, c->stream, nb, c->tile,
+  hipLaunchKernelGGL(k_tile_emit, dim3((nb + 256) / 256), dim3(256), 0, c->stream, nb, tile,
                      c->d_offset, c->d_tcount, c->d_tiles, c->d_ntiles);
   c->tiles_valid = true;
   return AMPS_OK;
@@ -810,11 +836,14 @@ extern "C" int amps_gpu_get_particles(amps_ctx* c, double* x, double* v, int32_t
 // ---------------------------------------------------------------------
 // migration
 // ---------------------------------------------------------------------
-// zeroed per-key counters (d_offset) and scatter cursors
-static void clear_counts(amps_ctx* c) {
-  const int64_t nkeys = (int64_t)c->mv.nb * NCELL;
-  hipLaunchKernelGGL(k_fill_int, dim3(1024), dim3(256), 0, c->stream, c->d_offset, nkeys + 1, 0);
-  hipLaunchKernelGGL(k_fill_int, dim3(1024), dim3(256), 0, c->stream, c->d_cursor, nkeys, 0);
+// zeroed counters: per key (d_offset unless classify, whose stayers are
+// counted from the masks), scatter cursors, the stayer masks, the lists
+static void clear_counts(amps_ctx* c, bool classify = false) {
+  const int64_t nkeys = (int64_t)c->mv.nb * NCELL, nw = (c->cap + 255) / 256 * 4;
+  const int64_t most = std::max(nkeys, classify ? nw : 0);
+  hipLaunchKernelGGL(k_mig_clear, dim3((unsigned)std::min<int64_t>(2048, (most + 255) / 256)), dim3(256), 0, c->stream,
+                     nkeys, classify ? nullptr : c->d_offset, c->d_cursor, nw, classify ? c->d_wmask : nullptr,
+                     c->d_mig_slab + nkeys * MIG_SLAB, c->d_big + nkeys);
 }
 
 // counted: the push has already counted the survivors into a cleared d_offset
@@ -823,9 +852,9 @@ static void clear_counts(amps_ctx* c) {
 // (pending_gather): the step's matrix-core cell pass reads the particles
 // through them and the next push moves them as it updates them, so a step
 // writes the particle state once instead of twice.
-// classified: the push also classified the survivors (PushMig): d_offset
-// holds the stayers per key, d_cursor the movers, d_wcnt and d_wmask the
-// stayer counts and masks, the slab and overflow list the movers
+// classified: the push also classified the survivors (PushMig): d_cursor
+// holds the movers per key, d_wmask the stayer masks, the slab and overflow
+// list the movers
 static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, bool classified = false) {
   const int64_t nkeys = (int64_t)c->mv.nb * NCELL;
   const int64_t cap = c->cap;
@@ -836,25 +865,27 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
     hipLaunchKernelGGL(k_count_keys, dim3(gridp), dim3(256), 0, c->stream, c->d_n, c->d_key[a],
                        c->d_code, c->d_offset);
   }
-  if (classified)
-    hipLaunchKernelGGL(k_add_ints, dim3(1024), dim3(256), 0, c->stream, nkeys, c->d_offset, c->d_cursor);
-  if (int r = scan_exclusive(c, c->d_offset, nkeys + 1, nullptr)) return r;
+  const int64_t nw = (int64_t)gridp * 4;
+  if (classified) {
+    if (int r = scan_masks(c, c->d_wmask, c->d_wcnt, nw)) return r;
+    if (int r = scan_keys(c, c->d_cursor, c->d_off_layout, c->d_wcnt, c->d_wmask, c->d_offset, nkeys)) return r;
+  } else {
+    if (int r = scan_exclusive(c, c->d_offset, nkeys + 1, nullptr)) return r;
+  }
   const int vf32 = c->precision == AMPS_FP32 ? 1 : 0;
   if (c->deterministic) {
     // in every key, the particles that stayed in array order, then those that
     // moved in, in array order (every particle a mover when the arrays have no
     // layout of a previous compaction yet, e.g. a generated population)
     const unsigned gridk = (unsigned)((nkeys + 255) / 256);
-    const int64_t nw = (int64_t)gridp * 4;
-    if (!classified)
+    if (!classified) {
       hipLaunchKernelGGL(k_mig_classify, dim3(gridp), dim3(256), 0, c->stream, c->d_n, c->d_key[a], c->d_code,
-                         c->d_off_layout, c->layout_valid ? 1 : 0, c->d_offset, c->d_cursor, c->d_tmpsrc,
-                         c->d_wcnt, c->d_wmask);
-    if (int r = scan_exclusive(c, c->d_wcnt, nw + 1, nullptr)) return r;
+                         c->d_off_layout, c->layout_valid ? 1 : 0, c->d_offset, c->d_cursor, c->d_tmpsrc, c->d_wmask);
+      if (int r = scan_masks(c, c->d_wmask, c->d_wcnt, nw)) return r;
+    }
     if (classified)
       hipLaunchKernelGGL(k_mig_place, dim3(1024), dim3(256), 0, c->stream, c->d_mig_slab + nkeys * MIG_SLAB,
                          c->d_mig_ovf, c->d_key[a], c->d_offset, c->d_cursor, c->d_tmpsrc);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->stream, c->d_big + nkeys, 1, 0);
     // the movers' destinations in dest[] only for the scatter; in a deferred
     // move their source indices are the sorted lists, in place in tmpsrc
     const int write_dest = defer ? 0 : 1;
@@ -884,17 +915,15 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
                        c->d_cursor, cap, c->d_x[a], c->d_v[a], vf32, c->d_spec[a], c->d_id[a], c->d_x[b], c->d_v[b],
                        c->d_spec[b], c->d_key[b], c->d_id[b]);
   }
-  // the new layout, for the next compaction
-  hipLaunchKernelGGL(k_copy_ints, dim3((unsigned)((nkeys + 1 + 255) / 256)), dim3(256), 0, c->stream, nkeys + 1,
-                     c->d_offset, c->d_off_layout);
-  c->layout_valid = true;
-  hipLaunchKernelGGL(k_copy_total, dim3(1), dim3(1), 0, c->stream, c->d_offset + nkeys, c->d_n);
   c->cur = b;
   c->offsets_valid = true;
   // all survivors carry a committed code
   std::swap(c->d_code, c->d_code2);
-  hipLaunchKernelGGL(k_fill_int, dim3(256), dim3(256), 0, c->stream, (int*)c->d_code, (cap + 3) / 4,
-                     0x03030303);
+  // the new layout, for the next compaction, and the codes
+  hipLaunchKernelGGL(k_mig_finish, dim3((unsigned)std::min<int64_t>(2048, (std::max(nkeys, (cap + 3) / 4) + 256) / 256)),
+                     dim3(256), 0, c->stream, nkeys, c->d_offset, c->d_off_layout, c->d_n, (cap + 3) / 4,
+                     (int*)c->d_code);
+  c->layout_valid = true;
   return build_tiles(c);
 }
 
@@ -926,16 +955,16 @@ static int check_mover(const amps_ctx* c, const amps_push_opts* o, const char* w
 }
 
 // count: when non-null, the push also counts the surviving particles per key
-// (the migration's counting pass), into a zeroed array; classify: it also
-// classifies them for the deterministic migration (the stayers alone in
-// count, see PushMig), into zeroed d_cursor, d_wcnt, d_wmask and overflow count
+// (the migration's counting pass), into a zeroed array; classify: instead it
+// classifies them for the deterministic migration (PushMig), into zeroed
+// d_cursor, d_wmask and overflow count
 static int launch_push(amps_ctx* c, const amps_push_opts* o, int* count = nullptr, bool classify = false) {
   const int k = c->cur;
-  PushMig pm = {0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  PushMig pm = {0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   if (classify) {
     const int64_t nkeys = (int64_t)c->mv.nb * NCELL;
     pm = {nkeys, c->d_off_layout, c->d_cursor, c->d_mig_slab, c->d_mig_ovf, c->d_mig_slab + nkeys * MIG_SLAB,
-          c->d_wmask, c->d_wcnt};
+          c->d_wmask};
   }
   const bool w4 = c->push_waves == 4;
   // records the last compaction left in the other buffer: the push reads them
@@ -948,7 +977,7 @@ static int launch_push(amps_ctx* c, const amps_push_opts* o, int* count = nullpt
   }
 #define LAUNCH_PUSH32(MV, W)                                                                              \
   hipLaunchKernelGGL((k_push_f32<MV, W>), dim3((unsigned)c->max_tiles), dim3(256), 0, c->stream, c->mv,     \
-                     c->faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
+                     c->d_faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
                      c->d_x[k], (float*)c->d_v[k], c->d_spec[k], c->d_key[k], c->d_code, count, ps, pm)
   if (c->precision == AMPS_FP32) {
     if (o->mover == AMPS_MOVER_LAPENTA) {
@@ -964,7 +993,7 @@ static int launch_push(amps_ctx* c, const amps_push_opts* o, int* count = nullpt
 #undef LAUNCH_PUSH32
 #define LAUNCH_PUSH64(MV, BCV, W)                                                                       \
   hipLaunchKernelGGL((k_push_f64<MV, BCV, W>), dim3((unsigned)c->max_tiles), dim3(256), 0, c->stream, c->mv,  \
-                     c->faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
+                     c->d_faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
                      c->d_x[k], c->d_v[k], c->d_spec[k], c->d_key[k], c->d_code, c->d_Bc, count, ps, pm)
   const bool bc = c->b_center != 0;
   if (o->mover == AMPS_MOVER_LAPENTA) {
@@ -994,7 +1023,7 @@ extern "C" int amps_gpu_move_particles(amps_ctx* c, const amps_push_opts* o) {
   (void)hipSetDevice(c->device);
   if (o->bc_mode == AMPS_BC_USER)
     if (int r = prepare_exits(c)) return r;
-  if (o->tile > 0 && o->tile != c->tile) {
+  if (o->tile > 0 && (o->tile != c->tile || !c->tile_given)) {
     if (int r = amps_gpu_set_param(c, "tile", o->tile)) return r;
   }
   if (!c->offsets_valid) {
@@ -1002,15 +1031,21 @@ extern "C" int amps_gpu_move_particles(amps_ctx* c, const amps_push_opts* o) {
   } else if (!c->tiles_valid) {
     if (int r = build_tiles(c)) return r;
   }
+  // with the compaction that follows, the push counts for it (as in a step)
+  const bool cls = o->compact && c->deterministic && c->layout_valid;
+  if (o->compact) clear_counts(c, cls);
   tbegin(c);
-  if (int r = launch_push(c, o)) return r;
+  if (int r = launch_push(c, o, o->compact ? c->d_offset : nullptr, cls)) return r;
   tend(c, AMPS_K_PUSH);
   c->offsets_valid = false;
   c->tiles_valid = false;
   if (o->bc_mode == AMPS_BC_USER)
     if (int r = collect_exits(c)) return r;
-  if (o->compact) return amps_gpu_compact(c);
-  return AMPS_OK;
+  if (!o->compact) return AMPS_OK;
+  tbegin(c);
+  const int r = compact_impl(c, true, false, cls);
+  tend(c, AMPS_K_COMPACT);
+  return r;
 }
 
 // ---------------------------------------------------------------------
@@ -1211,14 +1246,7 @@ static int one_step(amps_ctx* c, const amps_push_opts* o, double dt) {
   // and for the deterministic one (the arrays in a compaction's layout)
   // classifies them
   const bool cls = c->deterministic && c->layout_valid;
-  clear_counts(c);
-  if (cls) {
-    const int64_t nkeys = (int64_t)c->mv.nb * NCELL;
-    const int64_t nw = (c->cap + 255) / 256 * 4;
-    hipLaunchKernelGGL(k_fill_int, dim3(1024), dim3(256), 0, c->stream, c->d_wcnt, nw + 1, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1024), dim3(256), 0, c->stream, (int*)c->d_wmask, 2 * nw, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->stream, c->d_mig_slab + nkeys * MIG_SLAB, 1, 0);
-  }
+  clear_counts(c, cls);
   tbegin(c);
   if (int r = launch_push(c, o, c->d_offset, cls)) return r;
   tend(c, AMPS_K_PUSH);
@@ -1245,7 +1273,7 @@ static int run_steps_impl(amps_ctx* c, const amps_push_opts* o, double dt, int64
   (void)hipSetDevice(c->device);
   if (o->bc_mode == AMPS_BC_USER)
     if (int r = prepare_exits(c)) return r;
-  if (o->tile > 0 && o->tile != c->tile)
+  if (o->tile > 0 && (o->tile != c->tile || !c->tile_given))
     if (int r = amps_gpu_set_param(c, "tile", o->tile)) return r;
   if (int r = ensure_deposit_buffers(c)) return r;
   if (!c->offsets_valid)

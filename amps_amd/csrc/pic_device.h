@@ -12,6 +12,56 @@ struct BlockGeom {
   double xmin[3], xmax[3], dxs[3], dxc[3];
 };
 
+// 1 / b to full precision, and a / b with it: the instruction sequence of the
+// compiler's a / b less the operand scaling and special-case fix-up
+// (v_div_scale, v_div_fixup), which are the identity for finite operands
+// within 2^+-700 or so, a zero numerator among them; so the quotients are the
+// same bits, and divisions by one denominator share its reciprocal (3
+// instructions each instead of 11).
+__device__ __forceinline__ double rcp_full(double b) {
+  const double y0 = __builtin_amdgcn_rcp(b);
+  const double y1 = fma(y0, fma(-b, y0, 1.0), y0);
+  return fma(y1, fma(-b, y1, 1.0), y1);
+}
+__device__ __forceinline__ double div_by(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+}
+// 1 / b for b >= 1; beyond the range above the plain division
+__device__ __forceinline__ double recip_from_one(double b) {
+  if (b < 0x1p+600) return div_by(1.0, b, rcp_full(b));
+  return 1.0 / b;
+}
+__device__ __forceinline__ double uniform_f64(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// Reciprocals of the tile's cell sizes (InitStencil's and FindCellIndex's)
+// and of the finest lattice spacing, the same for the whole workgroup.
+struct GeomRcp {
+  double dxs[3], dxc[3], ref[3];
+};
+__device__ __forceinline__ void load_geom_rcp(const MeshView& m, const BlockGeom& g, GeomRcp& r) {
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    r.dxs[d] = uniform_f64(rcp_full(g.dxs[d]));
+    r.dxc[d] = uniform_f64(rcp_full(g.dxc[d]));
+    r.ref[d] = uniform_f64(rcp_full(m.dx_maxref[d]));
+  }
+}
+
+// A species' constants of the push, staged in LDS.
+struct SpeciesPush {
+  double q, mass, dt, qdt_m, q_m;  // qdt_m = (q dt) / mass, q_m = q / mass
+};
+__device__ __forceinline__ void stage_species(const Species& sp, SpeciesPush* s) {
+  if ((int)threadIdx.x < sp.n) {
+    const int i = threadIdx.x;
+    s[i] = {sp.charge[i], sp.mass[i], sp.dt[i], sp.charge[i] * sp.dt[i] / sp.mass[i], sp.charge[i] / sp.mass[i]};
+  }
+}
+
 __device__ __forceinline__ void load_block_geom(const MeshView& m, int b, BlockGeom& g) {
 #pragma unroll
   for (int d = 0; d < 3; d++) {
@@ -67,6 +117,31 @@ __device__ __forceinline__ void corner_stencil(const BlockGeom& g, double x[3], 
   }
 }
 
+// The same with the tile's reciprocals, without the table.
+__device__ __forceinline__ void corner_weights(const BlockGeom& g, const GeomRcp& rc, double x[3], double wn[8],
+                                               int iX[3]) {
+  double f[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    if (fabs(x[d] - g.xmax[d]) < 1e-10 * g.dxs[d]) x[d] = g.xmax[d] - 1e-10 * g.dxs[d];
+    f[d] = div_by(x[d] - g.xmin[d], g.dxs[d], rc.dxs[d]);
+    iX[d] = (int)(f[d]);
+    f[d] -= iX[d];
+  }
+  const double e[3] = {1.0 - f[0], 1.0 - f[1], 1.0 - f[2]};
+  double norm = 0.0;
+#pragma unroll
+  for (int l = 0; l < 8; l++) {
+    wn[l] = ((l >> 2) ? f[0] : e[0]) * (((l >> 1) & 1) ? f[1] : e[1]) * ((l & 1) ? f[2] : e[2]);
+    norm += wn[l];
+  }
+  if (norm > 0.0) {
+    const double r = rcp_full(norm);  // 1 to rounding
+#pragma unroll
+    for (int l = 0; l < 8; l++) wn[l] = div_by(wn[l], norm, r);
+  }
+}
+
 // findTreeNode(int*) as a lookup: the descent of meshAMRgeneric.h:2793-2848
 // returns the leaf containing the lattice point, or NULL outside the root.
 __device__ __forceinline__ int lookup_leaf(const MeshView& m, const int ix[3]) {
@@ -116,10 +191,12 @@ __device__ __forceinline__ void load_block_lat(const MeshView& m, int b, BlockLa
 }
 
 __device__ __forceinline__ int find_block_in(const MeshView& m, const double x[3], const BlockGeom& g,
-                                             const BlockLat& l) {
+                                             const GeomRcp& rc, const BlockLat& l) {
+  // not finite, or beyond div_by's range
+  if (!(fabs(x[0]) + fabs(x[1]) + fabs(x[2]) < 0x1p+900)) return find_block(m, x);
   int ix[3];
 #pragma unroll
-  for (int d = 0; d < 3; d++) ix[d] = (int)floor((x[d] - m.gxmin[d]) / m.dx_maxref[d]);
+  for (int d = 0; d < 3; d++) ix[d] = (int)floor(div_by(x[d] - m.gxmin[d], m.dx_maxref[d], rc.ref[d]));
   bool in = true;
 #pragma unroll
   for (int d = 0; d < 3; d++) in = in && ix[d] >= l.lo[d] && ix[d] < l.hi[d];
@@ -148,14 +225,14 @@ __device__ __forceinline__ int find_cell(const MeshView& m, const double x[3], i
 }
 
 __device__ __forceinline__ int find_cell_in(const MeshView& m, const double x[3], int b, const BlockGeom& g,
-                                            const BlockLat& l) {
+                                            const GeomRcp& rc, const BlockLat& l) {
   if (b != l.b) return find_cell(m, x, b);
   int ijk[3];
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const double xmn = g.xmin[d], xmx = g.xmax[d];
     if ((x[d] < xmn) || (xmx < x[d])) return -1;
-    int i = (int)((x[d] - xmn) / g.dxc[d]);
+    int i = (int)div_by(x[d] - xmn, g.dxc[d], rc.dxc[d]);
     if (i == NC) i = NC - 1;
     ijk[d] = clampi(i, 0, NC - 1);
   }
@@ -166,8 +243,8 @@ __device__ __forceinline__ int find_cell_in(const MeshView& m, const double x[3]
 // (pic_mover_boris.cpp:1088-1375), shared by the FP64 and FP32 pushes.  On
 // entry xInit/vInit hold the start state, xFinal/vFinal the pushed state;
 // xp/vp receive the committed state.
-__device__ __forceinline__ int relocate(const MeshView& m, const Faces& faces, const BlockGeom& g,
-                                        const BlockLat& lat, double dtTotal,
+__device__ __forceinline__ int relocate(const MeshView& m, const Faces* __restrict__ faces, const BlockGeom& g,
+                                        const GeomRcp& rc, const BlockLat& lat, double dtTotal,
                                         int bc_mode, double r_sphere, double xInit[3],
                                         double vInit[3], double xFinal[3], double vFinal[3],
                                         double xp[3], double vp[3], int* blk, int* cell) {
@@ -183,7 +260,7 @@ __device__ __forceinline__ int relocate(const MeshView& m, const Faces& faces, c
     for (int d = 0; d < 3; d++) xp[d] = xFinal[d], vp[d] = vFinal[d];
     return AMPS_CODE_SPHERE;
   }
-  int newNode = find_block_in(m, xFinal, g, lat);
+  int newNode = find_block_in(m, xFinal, g, rc, lat);
   int code = AMPS_CODE_FINISHED;
   if (newNode < 0) {
     if (bc_mode == AMPS_BC_DELETE) {
@@ -196,8 +273,9 @@ __device__ __forceinline__ int relocate(const MeshView& m, const Faces& faces, c
     const double vMiddle[3] = {0.5 * (vInit[0] + vFinal[0]), 0.5 * (vInit[1] + vFinal[1]),
                                0.5 * (vInit[2] + vFinal[2])};
     double dtIntersection = -1.0, r0[3];
+#pragma unroll 1
     for (int nface = 0; nface < 6; nface++) {
-      const Face& F = faces.f[nface];
+      const Face& F = faces->f[nface];
       double cx = 0.0, cv = 0.0;
 #pragma unroll
       for (int d = 0; d < 3; d++) {
@@ -225,7 +303,7 @@ __device__ __forceinline__ int relocate(const MeshView& m, const Faces& faces, c
       for (int d = 0; d < 3; d++) xp[d] = xFinal[d], vp[d] = vFinal[d];
       return AMPS_CODE_LEFT_DOMAIN;
     }
-    const Face& F = faces.f[nIntersectionFace];
+    const Face& F = faces->f[nIntersectionFace];
     const double tVelocityIncrement =
         ((dtIntersection / dtTotal < 1) ? dtIntersection / dtTotal : 1);
 #pragma unroll
@@ -267,7 +345,7 @@ __device__ __forceinline__ int relocate(const MeshView& m, const Faces& faces, c
     for (int d = 0; d < 3; d++) vFinal[d] = vInit[d], xFinal[d] = xInit[d];
     code = AMPS_CODE_REFLECTED;
   }
-  const int c_id = find_cell_in(m, xFinal, newNode, g, lat);
+  const int c_id = find_cell_in(m, xFinal, newNode, g, rc, lat);
   if (c_id < 0) return AMPS_CODE_LEFT_DOMAIN;
   *blk = newNode;
   *cell = c_id;
@@ -285,17 +363,18 @@ static __device__ __noinline__ void center_B(const MeshView& m, const double* __
 // LDS, or with BC the cell-centred B of Bc (the centre-based B mode,
 // :979-1000).  Returns the AMPS_CODE_*; xp/vp hold the committed state.
 template <int MOVER, bool BC = false>
-__device__ __forceinline__ int push_particle(const MeshView& m, const Faces& faces,
-                                             const BlockGeom& g, const BlockLat& lat, const double* sE,
-                                             const double* sB, double q, double mass,
-                                             double dtTotal, int bc_mode, double r_sphere,
+__device__ __forceinline__ int push_particle(const MeshView& m, const Faces* __restrict__ faces,
+                                             const BlockGeom& g, const GeomRcp& rc, const BlockLat& lat,
+                                             const double* sE, const double* sB, const SpeciesPush& sp, int bc_mode,
+                                             double r_sphere,
                                              double xp[3], double vp[3], int* blk, int* cell,
                                              const double* Bc = nullptr) {
   double vInit[3] = {vp[0], vp[1], vp[2]}, xInit[3] = {xp[0], xp[1], xp[2]};
   double vFinal[3], xFinal[3];
-  double wn[8], table[8];
+  double wn[8];
   int iX[3];
-  corner_stencil(g, xInit, wn, table, iX);
+  const double dtTotal = sp.dt;
+  corner_weights(g, rc, xInit, wn, iX);
 #pragma unroll
   for (int d = 0; d < 3; d++) iX[d] = clampi(iX[d], 0, NC - 1);
   double E[3] = {0.0, 0.0, 0.0}, B[3] = {0.0, 0.0, 0.0};
@@ -311,7 +390,7 @@ __device__ __forceinline__ int push_particle(const MeshView& m, const Faces& fac
   if constexpr (BC) center_B(m, Bc, xInit, *blk, B);
   if (MOVER == AMPS_MOVER_LAPENTA) {
     // :1033-1081
-    const double QdT_over_m = q * dtTotal / mass;
+    const double QdT_over_m = sp.qdt_m;
     const double QdT_over_2m = 0.5 * QdT_over_m;
     const double QdT_over_2m_squared = QdT_over_2m * QdT_over_2m;
     double BB[3][3], P[3], alpha[3][3];
@@ -325,7 +404,7 @@ __device__ __forceinline__ int push_particle(const MeshView& m, const Faces& fac
       }
     }
     const double c0 =
-        1.0 / (1.0 + QdT_over_2m_squared * (B[0] * B[0] + B[1] * B[1] + B[2] * B[2]));
+        recip_from_one(1.0 + QdT_over_2m_squared * (B[0] * B[0] + B[1] * B[1] + B[2] * B[2]));
     alpha[0][0] = c0 * (1.0 + BB[0][0]);
     alpha[0][1] = c0 * (-P[2] + BB[0][1]);
     alpha[0][2] = c0 * (P[1] + BB[0][2]);
@@ -346,7 +425,7 @@ __device__ __forceinline__ int push_particle(const MeshView& m, const Faces& fac
     for (int i = 0; i < 3; i++) xFinal[i] = xInit[i] + dtTotal * vFinal[i];
   } else {
     // BorisSplitAcceleration_default :87-98, rotation :253-277
-    const double Charge2Mass = q / mass;
+    const double Charge2Mass = sp.q_m;
     double accl[3], rot[3], u[3], h[3], U[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
@@ -360,16 +439,25 @@ __device__ __forceinline__ int push_particle(const MeshView& m, const Faces& fac
     for (int d = 0; d < 3; d++) h[d] = -dtTempOverTwo * rot[d];
     const double h2 = h[0] * h[0] + h[1] * h[1] + h[2] * h[2];
     const double uh = u[0] * h[0] + u[1] * h[1] + u[2] * h[2];
-    U[0] = ((1 - h2) * u[0] + 2 * (u[1] * h[2] - h[1] * u[2] + uh * h[0])) / (1 + h2);
-    U[1] = ((1 - h2) * u[1] + 2 * (u[2] * h[0] - h[2] * u[0] + uh * h[1])) / (1 + h2);
-    U[2] = ((1 - h2) * u[2] + 2 * (u[0] * h[1] - h[0] * u[1] + uh * h[2])) / (1 + h2);
+    U[0] = (1 - h2) * u[0] + 2 * (u[1] * h[2] - h[1] * u[2] + uh * h[0]);
+    U[1] = (1 - h2) * u[1] + 2 * (u[2] * h[0] - h[2] * u[0] + uh * h[1]);
+    U[2] = (1 - h2) * u[2] + 2 * (u[0] * h[1] - h[0] * u[1] + uh * h[2]);
+    const double o2 = 1 + h2;
+    if (o2 < 0x1p+600 && fabs(U[0]) + fabs(U[1]) + fabs(U[2]) < 0x1p+700) {
+      const double ro = rcp_full(o2);
+#pragma unroll
+      for (int d = 0; d < 3; d++) U[d] = div_by(U[d], o2, ro);
+    } else {
+#pragma unroll
+      for (int d = 0; d < 3; d++) U[d] = U[d] / o2;
+    }
 #pragma unroll
     for (int d = 0; d < 3; d++) vFinal[d] = U[d] + dtTempOverTwo * accl[d];
 #pragma unroll
     for (int d = 0; d < 3; d++) xFinal[d] = xInit[d] + dtTemp * vFinal[d];
   }
 
-  return relocate(m, faces, g, lat, dtTotal, bc_mode, r_sphere, xInit, vInit, xFinal, vFinal, xp, vp, blk,
+  return relocate(m, faces, g, rc, lat, dtTotal, bc_mode, r_sphere, xInit, vInit, xFinal, vFinal, xp, vp, blk,
                   cell);
 }
 
@@ -386,7 +474,7 @@ constexpr double PI_TIMES_2 = 6.283185307179586476925286766559005768394338798750
 // its face table with the spent loop counter).  A reflected particle is
 // committed at the face and the rest of its step dropped (the reference
 // aborts there, :426-432).
-__device__ __forceinline__ int push_particle_rel(const MeshView& m, const Faces& faces, int b0,
+__device__ __forceinline__ int push_particle_rel(const MeshView& m, const Faces* __restrict__ faces, int b0,
                                                  const BlockGeom& g0, const double* sE,
                                                  const double* sB, const double* __restrict__ Eg,
                                                  const double* __restrict__ Bg, double ElectricCharge,
@@ -480,7 +568,7 @@ __device__ __forceinline__ int push_particle_rel(const MeshView& m, const Faces&
 #pragma unroll
       for (int d = 0; d < 3; d++) vEffective[d] = xFinal[d] - xInit[d];
       for (int nface = 0; nface < 6; nface++) {
-        const Face& F = faces.f[nface];
+        const Face& F = faces->f[nface];
         double cx = 0.0, cv = 0.0;
 #pragma unroll
         for (int d = 0; d < 3; d++) {
@@ -508,7 +596,7 @@ __device__ __forceinline__ int push_particle_rel(const MeshView& m, const Faces&
         for (int d = 0; d < 3; d++) xp[d] = xFinal[d], vp[d] = vFinal[d];
         return AMPS_CODE_LEFT_DOMAIN;
       }
-      const Face& F = faces.f[nIntersectionFace];
+      const Face& F = faces->f[nIntersectionFace];
 #pragma unroll
       for (int d = 0; d < 3; d++) {
         xInit[d] += dtIntersection * (xFinal[d] - xInit[d]) - F.norm[d] * m.eps;
@@ -570,8 +658,9 @@ __device__ __forceinline__ int push_particle_rel(const MeshView& m, const Faces&
 // accumulated into the FP64 position, and block/cell location, sphere and
 // boundary handling run on the FP64 position (relocate()).
 template <int MOVER>
-__device__ __forceinline__ int push_particle_f32(const MeshView& m, const Faces& faces,
-                                                 const BlockGeom& g, const BlockLat& lat, const float* sE,
+__device__ __forceinline__ int push_particle_f32(const MeshView& m, const Faces* __restrict__ faces,
+                                                 const BlockGeom& g, const GeomRcp& rc, const BlockLat& lat,
+                                                 const float* sE,
                                                  const float* sB, float q, float mass,
                                                  double dtTotal, int bc_mode, double r_sphere,
                                                  double xp[3], float vf[3], int* blk, int* cell) {
@@ -582,7 +671,7 @@ __device__ __forceinline__ int push_particle_f32(const MeshView& m, const Faces&
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     if (fabs(xInit[d] - g.xmax[d]) < 1e-10 * g.dxs[d]) xInit[d] = g.xmax[d] - 1e-10 * g.dxs[d];
-    const double loc = (xInit[d] - g.xmin[d]) / g.dxs[d];
+    const double loc = div_by(xInit[d] - g.xmin[d], g.dxs[d], rc.dxs[d]);
     iX[d] = (int)loc;
     xl[d] = (float)(loc - iX[d]);
     iX[d] = clampi(iX[d], 0, NC - 1);
@@ -642,7 +731,7 @@ __device__ __forceinline__ int push_particle_f32(const MeshView& m, const Faces&
   for (int d = 0; d < 3; d++) xFinal[d] = xInit[d] + (double)(dt * vF[d]);
   double vo[3];
   const int code =
-      relocate(m, faces, g, lat, dtTotal, bc_mode, r_sphere, xInit, vInit, xFinal, vFinal, xp, vo, blk, cell);
+      relocate(m, faces, g, rc, lat, dtTotal, bc_mode, r_sphere, xInit, vInit, xFinal, vFinal, xp, vo, blk, cell);
 #pragma unroll
   for (int d = 0; d < 3; d++) vf[d] = (float)vo[d];
   return code;

@@ -48,12 +48,10 @@ __device__ __forceinline__ RunInfo wave_runs(bool valid, int k) {
 }
 
 // A pass's movers of the push's classification, listed a pass later, when
-// their rank (the cursor atomic's return, on the run's head lane) has had the
-// next pass's loads to arrive.
+// their rank (the cursor atomic's return) has had the next pass's loads to
+// arrive.
 struct MigPend {
-  int raw;        // the atomic's return (head lanes)
-  int head_lane;  // the lane holding the run's return
-  int off;        // lane - head_lane: the rank within the run
+  int rank;
   int knew;
   int p;
   bool mover;
@@ -62,17 +60,17 @@ struct MigPend {
 // the movers of a pass: each at its rank in its key's slab, or past it in
 // the overflow list (made by every lane of the wavefront)
 __device__ __forceinline__ void mig_list(const PushMig& pm, const MigPend& pd) {
+  if (!__ballot(pd.mover)) return;
   const int lane = __lane_id();
-  const int rank = __shfl(pd.raw, pd.head_lane) + pd.off;
-  const bool ov = pd.mover && rank >= MIG_SLAB;
-  if (pd.mover && !ov) pm.slab[rank * pm.nkeys + pd.knew] = pd.p;
+  const bool ov = pd.mover && pd.rank >= MIG_SLAB;
+  if (pd.mover && !ov) pm.slab[pd.rank * pm.nkeys + pd.knew] = pd.p;
   const uint64_t om = __ballot(ov);
   if (om) {
     const int lead = __ffsll((long long)om) - 1;
     int ob = 0;
     if (lane == lead) ob = atomicAdd(pm.novf, __popcll(om));
     ob = __shfl(ob, lead);
-    if (ov) pm.ovf[ob + __popcll(om & ((1ull << lane) - 1ull))] = make_int2(pd.p, rank);
+    if (ov) pm.ovf[ob + __popcll(om & ((1ull << lane) - 1ull))] = make_int2(pd.p, pd.rank);
   }
 }
 
@@ -81,11 +79,12 @@ __device__ __forceinline__ void mig_list(const PushMig& pm, const MigPend& pd) {
 // pm.lay every survivor counts in count[knew], one atomic per run of equal
 // keys.  With it (the passes 64-aligned, so that a wavefront's pass is one
 // stayer mask word) the push classifies: a stayer (its new key's old run,
-// sLay[] of the tile's block, holds it) counts in count[] and sets its mask
-// bit, stored plainly where the word lies inside the tile and by atomics at
-// the tile's ends, which neighbouring tiles share; a mover takes its rank
-// among its new key's movers from the cursor[] atomic, and the previous
-// pass's movers are listed (mig_list; the last pass's after the loop).
+// sLay[] of the tile's block, holds it) sets its mask bit, stored plainly
+// where the word lies inside the tile and by an atomic at the tile's ends,
+// which neighbouring tiles share; the stayers of a key are counted from the
+// masks afterwards, so they cost no atomic.  A mover takes its rank among its
+// new key's movers from the cursor[] atomic, and the previous pass's movers
+// are listed (mig_list; the last pass's after the loop).
 __device__ __forceinline__ void push_count(int* __restrict__ count, const PushMig& pm, const int* sLay, int b,
                                            int p, int start, int p1, bool alive, int knew, MigPend& pd) {
   if (!pm.lay) {
@@ -93,37 +92,27 @@ __device__ __forceinline__ void push_count(int* __restrict__ count, const PushMi
     if (r.head) atomicAdd(&count[knew], r.len);
     return;
   }
-  const int lane = __lane_id();
   const int cb = knew - b * NCELL;
   const bool stay = alive && cb >= 0 && cb < NCELL && p >= sLay[cb] && p < sLay[cb + 1];
-  const bool mover = alive && !stay;
-  const RunInfo rs = wave_runs(stay, knew);
-  if (rs.head) atomicAdd(&count[knew], rs.len);
   const uint64_t sm = __ballot(stay);
-  if (lane == 0 && sm) {
+  if (__lane_id() == 0 && sm) {
     const int64_t w = (int64_t)p >> 6;  // lane 0 holds the word's first position
-    if ((w << 6) >= start && (w << 6) + 64 <= p1) {
+    if ((w << 6) >= start && (w << 6) + 64 <= p1)
       pm.wmask[w] = sm;
-      pm.wcnt[w] = __popcll(sm);
-    } else {
+    else
       atomicOr((unsigned long long*)(pm.wmask + w), (unsigned long long)sm);
-      atomicAdd(pm.wcnt + w, __popcll(sm));
-    }
   }
   mig_list(pm, pd);
-  const RunInfo rm = wave_runs(mover, knew);
-  pd.raw = 0;
-  if (rm.head) pd.raw = atomicAdd(&pm.cursor[knew], rm.len);
-  pd.head_lane = rm.head_lane;
-  pd.off = lane - rm.head_lane;
+  pd.mover = alive && !stay;
+  pd.rank = 0;
+  if (pd.mover) pd.rank = atomicAdd(&pm.cursor[knew], 1);
   pd.knew = knew;
   pd.p = p;
-  pd.mover = mover;
 }
 
 // W: the occupancy the register allocation aims at (waves per SIMD).
 template <int MOVER, bool BC, int W>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f64(MeshView m, Faces faces, Species sp,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f64(MeshView m, const Faces* __restrict__ faces, Species sp,
                                                    const double* __restrict__ E,
                                                    const double* __restrict__ B,
                                                    const Tile* __restrict__ tiles,
@@ -135,6 +124,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
   __shared__ double sE[NCORNER * 3];
   __shared__ double sB[NCORNER * 3];
   __shared__ int sLay[NCELL + 1];
+  __shared__ SpeciesPush sSp[MAX_SPEC];
   const int t = blockIdx.x;
   if (t >= *ntiles) return;
   const Tile tl = tiles[t];
@@ -145,11 +135,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
     sE[i] = Eb[i];
     sB[i] = Bb[i];
   }
+  stage_species(sp, sSp);
   if (pm.lay)
     for (int i = threadIdx.x; i <= NCELL; i += blockDim.x) sLay[i] = pm.lay[(int64_t)b * NCELL + i];
   __syncthreads();
   BlockGeom g;
   load_block_geom(m, b, g);
+  GeomRcp rc;
+  load_geom_rcp(m, g, rc);
   BlockLat lat;
   load_block_lat(m, b, lat);
   const int p1 = tl.start + tl.count;
@@ -158,7 +151,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
   // 64-aligned when the push classifies.  Where the next pass reads (the last
   // compaction's source index) is loaded a pass ahead.
   const int pa = pm.lay ? (tl.start & ~63) : tl.start;
-  MigPend pd = {0, 0, 0, 0, 0, false};
+  MigPend pd = {0, 0, 0, false};
   const int pf = pa + (int)threadIdx.x;
   int qn = (ps.src && pf >= tl.start && pf < p1) ? ps.src[pf] : 0;
   for (int p0 = pa; p0 < p1; p0 += blockDim.x) {
@@ -182,11 +175,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
     int nb_out = b, cell_out = 0;
     int c;
     if constexpr (MOVER == AMPS_MOVER_RELATIVISTIC)
-      c = push_particle_rel(m, faces, b, g, sE, sB, E, B, sp.charge[s], sp.mass[s], sp.dt[s], bc_mode,
-                            r_sphere, xp, vp, &nb_out, &cell_out);
+      c = push_particle_rel(m, faces, b, g, sE, sB, E, B, sSp[s].q, sSp[s].mass, sSp[s].dt, bc_mode, r_sphere, xp,
+                            vp, &nb_out, &cell_out);
     else
-      c = push_particle<MOVER, BC>(m, faces, g, lat, sE, sB, sp.charge[s], sp.mass[s], sp.dt[s], bc_mode,
-                                   r_sphere, xp, vp, &nb_out, &cell_out, Bc);
+      c = push_particle<MOVER, BC>(m, faces, g, rc, lat, sE, sB, sSp[s], bc_mode, r_sphere, xp, vp, &nb_out,
+                                   &cell_out, Bc);
     x[p] = xp[0];
     x[cap + p] = xp[1];
     x[2 * cap + p] = xp[2];
@@ -206,7 +199,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
 }
 
 #define INST_PUSH64(MV, BCV, W)                                                                  \
-  template __global__ void k_push_f64<MV, BCV, W>(MeshView, Faces, Species, const double*, const double*, \
+  template __global__ void k_push_f64<MV, BCV, W>(MeshView, const Faces*, Species, const double*, const double*, \
                                                   const Tile*, const int*, int, double, int64_t, double*, \
                                                   double*, const uint8_t*, int*, int8_t*, const double*, int*, \
                                                   PushSrc, PushMig);
@@ -221,7 +214,7 @@ INST_PUSH64(AMPS_MOVER_BORIS, true, 1)
 // FP32 push: float E/B stencil in LDS (17.5 KB), float velocities, FP64
 // positions.
 template <int MOVER, int W>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f32(MeshView m, Faces faces, Species sp,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f32(MeshView m, const Faces* __restrict__ faces, Species sp,
                                                    const double* __restrict__ E,
                                                    const double* __restrict__ B,
                                                    const Tile* __restrict__ tiles,
@@ -233,6 +226,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
   __shared__ float sE[NCORNER * 3];
   __shared__ float sB[NCORNER * 3];
   __shared__ int sLay[NCELL + 1];
+  __shared__ SpeciesPush sSp[MAX_SPEC];
   const int t = blockIdx.x;
   if (t >= *ntiles) return;
   const Tile tl = tiles[t];
@@ -243,16 +237,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
     sE[i] = (float)Eb[i];
     sB[i] = (float)Bb[i];
   }
+  stage_species(sp, sSp);
   if (pm.lay)
     for (int i = threadIdx.x; i <= NCELL; i += blockDim.x) sLay[i] = pm.lay[(int64_t)b * NCELL + i];
   __syncthreads();
   BlockGeom g;
   load_block_geom(m, b, g);
+  GeomRcp rc;
+  load_geom_rcp(m, g, rc);
   BlockLat lat;
   load_block_lat(m, b, lat);
   const int p1 = tl.start + tl.count;
   const int pa = pm.lay ? (tl.start & ~63) : tl.start;
-  MigPend pd = {0, 0, 0, 0, 0, false};
+  MigPend pd = {0, 0, 0, false};
   const int pf = pa + (int)threadIdx.x;
   int qn = (ps.src && pf >= tl.start && pf < p1) ? ps.src[pf] : 0;
   for (int p0 = pa; p0 < p1; p0 += blockDim.x) {
@@ -273,8 +270,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
       ps.id_out[p] = ps.id[q];
     }
     int nb_out = b, cell_out = 0;
-    const int c = push_particle_f32<MOVER>(m, faces, g, lat, sE, sB, (float)sp.charge[s], (float)sp.mass[s],
-                                           sp.dt[s], bc_mode, r_sphere, xp, vp, &nb_out, &cell_out);
+    const int c = push_particle_f32<MOVER>(m, faces, g, rc, lat, sE, sB, (float)sSp[s].q, (float)sSp[s].mass,
+                                           sSp[s].dt, bc_mode, r_sphere, xp, vp, &nb_out, &cell_out);
     x[p] = xp[0];
     x[cap + p] = xp[1];
     x[2 * cap + p] = xp[2];
@@ -293,7 +290,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
 }
 
 #define INST_PUSH32(MV, W)                                                                        \
-  template __global__ void k_push_f32<MV, W>(MeshView, Faces, Species, const double*, const double*, \
+  template __global__ void k_push_f32<MV, W>(MeshView, const Faces*, Species, const double*, const double*, \
                                              const Tile*, const int*, int, double, int64_t, double*,  \
                                              float*, const uint8_t*, int*, int8_t*, int*, PushSrc,   \
                                              PushMig);
@@ -392,8 +389,7 @@ __global__ __launch_bounds__(256) void k_scatter(const int* __restrict__ n_dev,
 __global__ __launch_bounds__(256) void k_mig_classify(const int* __restrict__ n_dev, const int* __restrict__ key,
                                                        const int8_t* __restrict__ code, const int* __restrict__ lay,
                                                        int has_layout, const int* __restrict__ offset, int* cursor,
-                                                       int* __restrict__ tmpsrc, int* __restrict__ wcnt,
-                                                       uint64_t* __restrict__ wmask) {
+                                                       int* __restrict__ tmpsrc, uint64_t* __restrict__ wmask) {
   const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int n = *n_dev;
   const bool valid = (p < n) && alive_code(code[p]);
@@ -405,10 +401,7 @@ __global__ __launch_bounds__(256) void k_mig_classify(const int* __restrict__ n_
   int base = 0;
   if (ru.head) base = atomicAdd(&cursor[k], ru.len);
   base = __shfl(base, ru.head_lane);
-  if (__lane_id() == 0) {
-    wcnt[p >> 6] = __popcll(m);
-    wmask[p >> 6] = m;
-  }
+  if (__lane_id() == 0) wmask[p >> 6] = m;
   if (mover) tmpsrc[(int64_t)offset[k + 1] - 1 - (base + (__lane_id() - ru.head_lane))] = (int)p;
 }
 
@@ -423,12 +416,6 @@ __global__ __launch_bounds__(256) void k_mig_place(const int* __restrict__ novf,
     const int k = key[e.x];
     tmpsrc[(int64_t)offset[k + 1] - cursor[k] + e.y] = e.x;
   }
-}
-
-// a[i] += b[i]
-__global__ __launch_bounds__(256) void k_add_ints(int64_t n, int* __restrict__ a, const int* __restrict__ b) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    a[i] += b[i];
 }
 
 // the destination base of key k's stayers: its new offset less the stayers
@@ -491,9 +478,13 @@ __global__ __launch_bounds__(256) void k_mig_order(int64_t nkeys, int small, int
   sort_movers(q, m, d0, write_dest, dest);
 }
 
-// The same for movers the push listed (PushMig): the key's lane places its
-// slab entries beside the entries k_mig_place put past them (rank r at
-// d0 + r) and sorts them, or past `small` lists the key for k_mig_order_big.
+// The same for movers the push listed (PushMig).  Up to MIG_SLAB of them the
+// key's lane sorts in its column of LDS as it reads them from the slab
+// (rank-major: coalesced) and writes out in order; more (or more than
+// `small`) are put beside the entries k_mig_place put past the slab, and the
+// key is listed for k_mig_order_big.  Sorting in place in memory took 81 us a
+// step on the two-level mesh (2.0 M particles, CFL 0.2), a chain of dependent
+// accesses of the lane with the most movers.
 __global__ __launch_bounds__(256) void k_mig_order_slab(int64_t nkeys, int small, int write_dest,
                                                          const int* __restrict__ slab,
                                                          const int* __restrict__ offset,
@@ -502,19 +493,37 @@ __global__ __launch_bounds__(256) void k_mig_order_slab(int64_t nkeys, int small
                                                          const int* __restrict__ lay, const int* __restrict__ wscan,
                                                          const uint64_t* __restrict__ wmask,
                                                          int* __restrict__ kbase) {
+  __shared__ int col[MIG_SLAB][256];
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (k >= nkeys) return;
   key_base(k, offset, lay, wscan, wmask, kbase);
   const int m = cursor[k];
   if (m == 0) return;
   const int d0 = offset[k + 1] - m;
-  const int ms = min(m, MIG_SLAB);
-  for (int j = 0; j < ms; j++) tmpsrc[d0 + j] = slab[j * nkeys + k];
-  if (m > small) {
+  if (m > small || m > MIG_SLAB) {
+    const int ms = min(m, MIG_SLAB);
+    for (int j = 0; j < ms; j++) tmpsrc[d0 + j] = slab[j * nkeys + k];
     big[atomicAdd(&big[nkeys], 1)] = (int)k;
     return;
   }
-  sort_movers(tmpsrc + d0, m, d0, write_dest, dest);
+  const int t = threadIdx.x;
+  for (int j0 = 0; j0 < m; j0 += 4) {
+    int v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = j0 + q < m ? slab[(j0 + q) * nkeys + k] : 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (j0 + q >= m) break;
+      int i = j0 + q;
+      for (; i > 0 && col[i - 1][t] > v[q]; i--) col[i][t] = col[i - 1][t];
+      col[i][t] = v[q];
+    }
+  }
+  for (int j = 0; j < m; j++) {
+    const int v = col[j][t];
+    tmpsrc[d0 + j] = v;
+    if (write_dest) dest[v] = d0 + j;
+  }
 }
 
 // number of entries of the ascending run r[0, n) below t
@@ -531,9 +540,11 @@ __device__ __forceinline__ int count_below(const int* r, int n, int t) {
 }
 
 // the keys with many movers, one workgroup each (a grid-stride loop over the
-// list): a bottom-up merge sort of the distinct source positions, every
+// list): up to RANK_SORT of them from LDS, every element's place the number of
+// smaller ones (the positions are distinct); above that a bottom-up merge sort of the distinct source positions, every
 // element placed by a binary search in the partner run, ping-ponging between
 // tmpsrc and a spare array of the same size; the sorted run ends in tmpsrc
+constexpr int RANK_SORT = 1024;
 __global__ __launch_bounds__(256) void k_mig_order_big(int64_t nkeys, int write_dest,
                                                         const int* __restrict__ offset,
                                                         const int* __restrict__ cursor, int* tmpsrc, int* spare,
@@ -545,6 +556,24 @@ __global__ __launch_bounds__(256) void k_mig_order_big(int64_t nkeys, int write_
     const int d0 = offset[k + 1] - m;
     int* src = tmpsrc + d0;
     int* dst = spare + d0;
+    if (m <= RANK_SORT) {
+      __shared__ __align__(16) int v[RANK_SORT];
+      const int m4 = (m + 3) & ~3;
+      for (int i = threadIdx.x; i < m4; i += blockDim.x) v[i] = i < m ? src[i] : 0x7fffffff;
+      __syncthreads();
+      for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        const int t = v[i];
+        int below = 0;
+        for (int j = 0; j < m4; j += 4) {
+          const int4 q = *(const int4*)(v + j);
+          below += (q.x < t) + (q.y < t) + (q.z < t) + (q.w < t);
+        }
+        src[below] = t;
+        if (write_dest) dest[t] = d0 + below;
+      }
+      __syncthreads();
+      continue;
+    }
     for (int w = 1; w < m; w *= 2) {
       for (int i = threadIdx.x; i < m; i += blockDim.x) {
         const int r = i / w, s = (r >> 1) * 2 * w;
@@ -681,12 +710,64 @@ __global__ __launch_bounds__(256) void k_mig_scatter(const int* __restrict__ n_d
   ib[d] = ia[p];
 }
 
-__global__ __launch_bounds__(256) void k_copy_ints(int64_t n, const int* __restrict__ src, int* __restrict__ dst) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
+// The end of a compaction: the new layout and particle count for the next
+// one, and every survivor's code committed.
+__global__ __launch_bounds__(256) void k_mig_finish(int64_t nkeys, const int* __restrict__ offset, int* __restrict__ lay,
+                                                     int* __restrict__ n_dev, int64_t ncode4, int* __restrict__ code) {
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = i0; i <= nkeys; i += st) lay[i] = offset[i];
+  for (int64_t i = i0; i < ncode4; i += st) code[i] = 0x03030303;
+  if (i0 == 0) *n_dev = offset[nkeys];
 }
 
-__global__ void k_copy_total(const int* __restrict__ src, int* dst) { *dst = *src; }
+// What a step's counting starts from: zeroed counters (count null: not used),
+// stayer masks (wmask null likewise) and list lengths.
+__global__ __launch_bounds__(256) void k_mig_clear(int64_t nkeys, int* __restrict__ count, int* __restrict__ cursor,
+                                                    int64_t nw, uint64_t* __restrict__ wmask, int* __restrict__ novf,
+                                                    int* __restrict__ nbig) {
+  const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = i0; i < nkeys; i += st) {
+    cursor[i] = 0;
+    if (count) count[i] = 0;
+  }
+  if (wmask)
+    for (int64_t i = i0; i < nw; i += st) wmask[i] = 0;
+  if (i0 == 0) {
+    if (count) count[nkeys] = 0;
+    *novf = 0;
+    *nbig = 0;
+  }
+}
+
+// The push tiles in one workgroup (meshes of up to TILE_WG blocks): counts,
+// their scan and the tiles.
+constexpr int TILE_WG = 8192;
+__global__ __launch_bounds__(1024) void k_tiles(int nb, int T, const int* __restrict__ offset, Tile* tiles,
+                                                int* ntiles) {
+  __shared__ int s[16];
+  const int per = (nb + 1023) / 1024;
+  const int b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
+  int tot = 0;
+  for (int b = b0; b < b1; b++) tot += (offset[(b + 1) * NCELL] - offset[b * NCELL] + T - 1) / T;
+  int incl = tot;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(incl, off);
+    if (lane >= off) incl += t;
+  }
+  if (lane == 63) s[w] = incl;
+  __syncthreads();
+  int at = incl - tot;
+#pragma unroll
+  for (int q = 0; q < 16; q++)
+    if (q < w) at += s[q];
+  if (threadIdx.x == 1023) *ntiles = at + tot;
+  for (int b = b0; b < b1; b++) {
+    const int start = offset[b * NCELL], cnt = offset[(b + 1) * NCELL] - start;
+    for (int t = 0; t < cnt; t += T) tiles[at++] = Tile{b, start + t, min(T, cnt - t), 0};
+  }
+}
 
 // tiles of at most T particles, never straddling a block
 __global__ __launch_bounds__(256) void k_tile_count(int nb, int T, const int* __restrict__ offset,
@@ -726,27 +807,60 @@ constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 8;
 constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_tile(int* data, int64_t n, int* sums) {
-  __shared__ int s[SCAN_BLOCK];
+// What a scan reads: an array, the stayer counts of the mask words, or the
+// new particle count of every key (its movers and its stayers).
+struct ScanArray {
+  const int* a;
+  __device__ int at(int64_t i) const { return a[i]; }
+};
+struct ScanMasks {
+  const uint64_t* m;
+  int64_t nw;
+  __device__ int at(int64_t i) const { return i < nw ? __popcll(m[i]) : 0; }
+};
+struct ScanKeys {
+  const int *cursor, *lay, *wscan;
+  const uint64_t* wmask;
+  int64_t nkeys;
+  // stayers before position q
+  __device__ int before(int q) const {
+    const int w = q >> 6, r = q & 63;
+    return wscan[w] + (r ? __popcll(wmask[w] & ((1ull << r) - 1ull)) : 0);
+  }
+  // a key's stayers are the mask bits of its old run
+  __device__ int at(int64_t k) const {
+    if (k >= nkeys) return 0;
+    const int q0 = lay[k], q1 = lay[k + 1];
+    return cursor[k] + (q1 > q0 ? before(q1) - before(q0) : 0);
+  }
+};
+
+template <class IN>
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_tile(IN in, int* data, int64_t n, int* sums) {
+  __shared__ int s[SCAN_BLOCK / 64];
   const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
   int vals[SCAN_ITEMS];
   int tot = 0;
 #pragma unroll
   for (int i = 0; i < SCAN_ITEMS; i++) {
     const int64_t j = base + i;
-    vals[i] = (j < n) ? data[j] : 0;
+    vals[i] = (j < n) ? in.at(j) : 0;
     tot += vals[i];
   }
-  s[threadIdx.x] = tot;
-  __syncthreads();
-  for (int off = 1; off < SCAN_BLOCK; off <<= 1) {
-    int t = (threadIdx.x >= off) ? s[threadIdx.x - off] : 0;
-    __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
+  int incl = tot;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(incl, off);
+    if (lane >= off) incl += t;
   }
-  int run = s[threadIdx.x] - tot;  // exclusive prefix of this thread
-  if (threadIdx.x == SCAN_BLOCK - 1) sums[blockIdx.x] = s[threadIdx.x];
+  if (lane == 63) s[w] = incl;
+  __syncthreads();
+  int run = incl - tot;  // exclusive prefix of this thread
+#pragma unroll
+  for (int q = 0; q < SCAN_BLOCK / 64; q++)
+    if (q < w) run += s[q];
+  if (threadIdx.x == SCAN_BLOCK - 1) sums[blockIdx.x] = run + tot;
 #pragma unroll
   for (int i = 0; i < SCAN_ITEMS; i++) {
     const int64_t j = base + i;
@@ -755,9 +869,23 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_tile(int* data, int64_t n, 
   }
 }
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add(int* data, int64_t n,
-                                                          const int* __restrict__ sums) {
-  const int add = sums[blockIdx.x];
+// sums: the scanned tile totals, or with raw the totals, of which every
+// workgroup sums the preceding ones itself
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add(int* data, int64_t n, const int* __restrict__ sums, int raw) {
+  __shared__ int s[SCAN_BLOCK / 64];
+  int add;
+  if (raw) {
+    int v = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += SCAN_BLOCK) v += sums[i];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    add = 0;
+#pragma unroll
+    for (int q = 0; q < SCAN_BLOCK / 64; q++) add += s[q];
+  } else {
+    add = sums[blockIdx.x];
+  }
   const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
   for (int i = threadIdx.x; i < SCAN_TILE; i += SCAN_BLOCK) {
     const int64_t j = base + i;
@@ -766,19 +894,22 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add(int* data, int64_t n,
 }
 
 namespace amps {
-static int scan_rec(amps_ctx* c, int* data, int64_t n, int* tmp) {
+// up to this many tiles (4 M entries) every workgroup of the second pass sums
+// the tile totals before its own; above, they are scanned
+constexpr int64_t SCAN_RAW = 2048;
+
+template <class IN>
+static void scan_rec(amps_ctx* c, IN in, int* data, int64_t n, int* tmp) {
   const int64_t nt = (n + SCAN_TILE - 1) / SCAN_TILE;
-  hipLaunchKernelGGL(k_scan_tile, dim3((unsigned)nt), dim3(SCAN_BLOCK), 0, c->stream, data, n, tmp);
+  hipLaunchKernelGGL(k_scan_tile<IN>, dim3((unsigned)nt), dim3(SCAN_BLOCK), 0, c->stream, in, data, n, tmp);
   if (nt > 1) {
-    int r = scan_rec(c, tmp, nt, tmp + nt);
-    if (r) return r;
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nt), dim3(SCAN_BLOCK), 0, c->stream, data, n,
-                       tmp);
+    if (nt > SCAN_RAW) scan_rec(c, ScanArray{tmp}, tmp, nt, tmp + nt);
+    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nt), dim3(SCAN_BLOCK), 0, c->stream, data, n, tmp,
+                       nt > SCAN_RAW ? 0 : 1);
   }
-  return 0;
 }
 
-int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* /*total_out*/) {
+static int scan_space(amps_ctx* c, int64_t n) {
   // temporary space: sum over levels of ceil(n / TILE^k) < n/(TILE-1) + levels
   int64_t need = 0, m = n;
   while (m > 1) {
@@ -792,7 +923,23 @@ int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* /*total_out*/) {
     HIP_TRY(hipMalloc(&c->d_scan_tmp, sizeof(int) * need));
     c->scan_tmp_len = need;
   }
-  return scan_rec(c, data, n, c->d_scan_tmp);
+  return 0;
+}
+int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* /*total_out*/) {
+  if (int r = scan_space(c, n)) return r;
+  scan_rec(c, ScanArray{data}, data, n, c->d_scan_tmp);
+  return 0;
+}
+int scan_masks(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw) {
+  if (int r = scan_space(c, nw + 1)) return r;
+  scan_rec(c, ScanMasks{wmask, nw}, wscan, nw + 1, c->d_scan_tmp);
+  return 0;
+}
+int scan_keys(amps_ctx* c, const int* cursor, const int* lay, const int* wscan, const uint64_t* wmask, int* offset,
+              int64_t nkeys) {
+  if (int r = scan_space(c, nkeys + 1)) return r;
+  scan_rec(c, ScanKeys{cursor, lay, wscan, wmask, nkeys}, offset, nkeys + 1, c->d_scan_tmp);
+  return 0;
 }
 }  // namespace amps
 

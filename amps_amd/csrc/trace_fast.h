@@ -28,13 +28,6 @@
 
 namespace {
 
-// 1 / b to full precision (the refined reciprocal of the division sequence)
-__device__ __forceinline__ double rcp_full(double b) {
-  const double y0 = __builtin_amdgcn_rcp(b);
-  const double y1 = fma(y0, fma(-b, y0, 1.0), y0);
-  return fma(y1, fma(-b, y1, 1.0), y1);
-}
-
 template <bool IEEE>
 struct Arith {
   static __device__ __forceinline__ double rcp(double b) { return IEEE ? 0.0 : rcp_full(b); }

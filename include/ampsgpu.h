@@ -77,7 +77,7 @@ int amps_gpu_device_info(amps_ctx* ctx, char* name, int* n_cu, int64_t* hbm_byte
  * repeated runs give the same layout and bit-identical deposits; 0: the
  * order in which the atomics of the scatter land), "migration_sort_small"
  * (1..64, default 64: cells receiving more movers than this are ordered by a
- * workgroup merge sort instead of one lane), "deposit_paired"
+ * workgroup instead of one lane), "deposit_paired"
  * (kernel 2: 1 two wavefronts per SIMD in opposite VALU/MFMA phases,
  * 0 (default): one phase sequence per wavefront), "node_batch"
  * (1..64 consecutive nodes per wavefront in the deposit node gather,
@@ -87,7 +87,7 @@ int amps_gpu_device_info(amps_ctx* ctx, char* name, int* n_cu, int64_t* hbm_byte
  * each node's inputs through shared memory with run-wise loads; 0: one
  * gathered load per output value),
  * "push_waves" (1: push kernels with the compiler's register allocation,
- * 4: held to 128 registers for four wavefronts per SIMD),
+ * 4 (default): held to 128 registers for four wavefronts per SIMD),
  * "b_center" (1: the FP64 Lapenta/Boris movers and the deposit take B from
  * the cell-centred field of amps_gpu_set_center_fields, the centre-based B
  * mode _PIC_FIELD_SOLVER_B_MODE_; 0 (default): B at the corners),

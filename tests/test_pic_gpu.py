@@ -250,6 +250,63 @@ def test_migration_order_is_deterministic(gpu_ctx, small):
         gpu_ctx.set_param("migration_sort_small", 64)
 
 
+@pytest.mark.parametrize("tile", [None, 256, 8192])
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+def test_migration_arrival_counts_at_the_sort_limits(tile, precision):
+    """Cells taking 1 .. 3000 arrivals, on both sides of every limit of the
+    arrival sorts (16 listed by the push, 64 by one lane, 1024 ranked in
+    LDS, the merge sort above), among resting particles and some that leave:
+    the push with the compaction in the same call against the push and a
+    separate compaction, with the push's own tiles and given ones, and the
+    layout the arrays themselves determine."""
+    mesh = M.uniform_mesh(1)
+    E, B = M.corner_fields(mesh)
+    E, B = np.zeros_like(E), np.zeros_like(B)
+    sp = Species([-1.0, 1.0], [1.0, 1.0], [0.125, 0.125])
+    counts = [1, 2, 15, 16, 17, 63, 64, 65, 255, 256, 1023, 1024, 1025, 3000]
+    rng = np.random.default_rng(17)
+    nbg, ngone = 9000, 500
+    lo, hi = mesh.xmin, mesh.xmax
+    n = nbg + ngone + sum(counts)
+    x = lo + (hi - lo) * rng.uniform(0.02, 0.98, (3, n)).T
+    v = np.zeros((n, 3))
+    v[nbg:nbg + ngone, 0] = 40.0 * (hi[0] - lo[0])  # out through the wall
+    o = nbg + ngone
+    h = (hi - lo) / 16
+    for j, m in enumerate(counts):  # the centre of a cell of its own
+        tgt = lo + (np.array([j + 1, 15 - j, (5 * j) % 16]) + 0.5) * h
+        v[o:o + m] = (tgt - x[o:o + m]) / 0.125
+        o += m
+    mix = rng.permutation(n)
+    x, v = np.ascontiguousarray(x[mix].T), np.ascontiguousarray(v[mix].T)
+    blk = mesh.locate(x.T)
+    p = M.Particles(x, v, np.arange(n) % 2, blk, M.cell_of(mesh, x, blk))
+    ctx = L.Context(0)  # its own: a tile once given stays
+    if tile:
+        ctx.set_param("tile", tile)
+    st = PicState(mesh, E, B, sp, ctx=ctx)
+    st.set_particles(p, precision=precision)
+    a, _ = st.get_particles()
+    st.MoveParticles(mover=L.MOVER_BORIS, bc_mode=L.BC_DELETE, compact=True)
+    b, _ = st.get_particles()
+    st.set_particles(p, precision=precision)
+    st.MoveParticles(mover=L.MOVER_BORIS, bc_mode=L.BC_DELETE, compact=False)
+    st.compact()
+    c, _ = st.get_particles()
+    ctx.close()
+    for k in ("id", "x", "v", "blk", "cell", "spec"):
+        assert np.array_equal(getattr(b, k), getattr(c, k)), k
+    pos = np.full(n, -1)
+    pos[a.id] = np.arange(a.n)
+    old = pos[b.id]
+    ka = a.blk.astype(np.int64) * 512 + a.cell
+    kb = b.blk.astype(np.int64) * 512 + b.cell
+    mover = kb != ka[old]
+    assert np.array_equal(np.lexsort((old, mover, kb)), np.arange(b.n))
+    per_key = np.bincount(kb[mover], minlength=mesh.ncells)
+    assert b.n == n - ngone and per_key.max() > 1024 and (per_key > 16).sum() >= 10
+
+
 @pytest.mark.parametrize("small,kernel", [(64, 2), (1, 2), (64, 1)])
 def test_step_migration_order_with_crowded_arrivals(gpu_ctx, small, kernel):
     """The same layout from the step's own migration, whose push classifies
