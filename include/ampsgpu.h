@@ -62,7 +62,9 @@ int amps_gpu_synchronize(amps_ctx* ctx);
 int amps_gpu_device_info(amps_ctx* ctx, char* name, int* n_cu, int64_t* hbm_bytes);
 
 /* Tuning parameters (no reference counterpart; set by the autotuner):
- * "tile" (particles per push workgroup, 64..2^20), "deposit_chunks"
+ * "tile" (particles per push workgroup, 64..2^20; until set, the largest
+ * power of two from 256 to 8192 of which the capacity holds 2,048),
+ * "deposit_chunks"
  * (waves per deposit workgroup: 2,3,4,6 for kernel 0, 4,6,12 for kernels 1
  * and 2; particles per cell per record batch, 4 or 8, for kernel 3),
  * "deposit_exact" (0/1: unfused mul+add in the deposit accumulation

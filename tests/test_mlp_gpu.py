@@ -94,3 +94,51 @@ def test_training_step_follows_new_data(gpu_ctx):
     assert steps == 1
     want, _, _ = MO.adam_step(th.astype(np.float64), 0, 0, g.astype(np.float64), 1, lr=1e-3)
     assert np.allclose(th1, want, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 65, 4 * 16 * 3 * 256 + 21])
+def test_forward_at_tile_edges(gpu_ctx, n):
+    """Fewer samples than a wavefront's 16, one more than a tile, and more
+    than one pass of the resident grid (4 x 3 wavefronts on 256 units): the
+    values of the same samples do not depend on their place.  The tolerance
+    is that of test_forward_matches_reference."""
+    th = MO.init_params(3).astype(np.float32)
+    sur = Surrogate(gpu_ctx, theta=th)
+    X, _ = _data(1000)
+    big = np.resize(X, (n, 6))
+    y = sur.predict(big)
+    yr = _rounded_forward(th.astype(np.float64), X.astype(np.float64))
+    assert y.shape == (n,)
+    assert np.abs(y - np.resize(yr, n)).max() <= 2e-3 * np.abs(yr).max()
+    assert np.array_equal(y, np.resize(sur.predict(X), n))
+
+
+@pytest.mark.parametrize("n", [64, 192, 4032])
+def test_gradient_at_partial_counts(gpu_ctx, n):
+    """2, 6 and 126 gradient partials: fewer than, and no multiple of, the
+    wavefronts that sum them (the tolerance of test_gradient_matches_reference)."""
+    th = MO.init_params(4).astype(np.float32)
+    sur = Surrogate(gpu_ctx, theta=th)
+    X, t = _data(4096, 1)
+    sur.set_data(X, t)
+    g, loss = sur.grad(n)
+    L64, g64 = MO.loss_and_grad(th.astype(np.float64), X[:n].astype(np.float64), t[:n].astype(np.float64))
+    assert abs(loss - L64) <= 2e-2 * L64
+    for o, m in ((0, 768), (768, 128), (896, 16384), (17280, 128), (17408, 128), (17536, 1)):
+        assert np.linalg.norm(g[o:o + m] - g64[o:o + m]) <= 5e-2 * np.linalg.norm(g64[o:o + m]), o
+
+
+@pytest.mark.parametrize("n", [24, 100])
+def test_batches_wrap_at_the_data_s_end(gpu_ctx, n):
+    """Batches of 64 over n rows run into the start of the data, also inside a
+    workgroup's rows and more than once in a batch: the same parameters as
+    from the rows written out."""
+    th = MO.init_params(7).astype(np.float32)
+    X, t = _data(n, 5)
+    out = []
+    for data in ((X, t), (np.resize(X, (3 * 64, 6)), np.resize(t, 3 * 64))):
+        sur = Surrogate(gpu_ctx, theta=th)
+        sur.set_data(*data)
+        sur.train(3, batch=64, lr=1e-3)
+        out.append(sur.params()[0])
+    assert np.array_equal(out[0], out[1])
