@@ -15,19 +15,32 @@
 // registers, with the parts of the 16 x 32 result outside these blocks unused.
 //
 // One workgroup per 4x4x4 sub-tile of a block; wavefront w takes the 16
-// cells of z-layer w.  Its cells' particles are consecutive runs of the
-// key-sorted arrays; the wavefront walks their concatenation 64 particles at a
+// cells of z-layer w (8 or 4 cells a wavefront, and fewer layers a workgroup, on
+// meshes of few blocks).  Its cells' particles are consecutive runs of the
+// key-sorted arrays; the wavefront walks their concatenation, each cell's run
+// rounded up to whole steps of 4, 64 places at a
 // time: each lane turns one particle into its operand record (corner stencil,
 // B from the sub-tile's corners staged in LDS, alpha, alpha v) in LDS, then the
 // wavefront issues the MFMA steps cell by cell and writes a finished cell's
-// 267 values (J[8][3] / V, then M[27][9]) to its partial-sum record.  The next
-// chunk's particles are loaded while the current one is accumulated.
+// 267 values (J[8][3] / V, then M[27][9]) to its partial-sum record.  The
+// particles of the next two chunks, and the source indices of the one after,
+// are loaded while the current one is accumulated.
+//
+// What bounds it: the issue slots of a SIMD's two wavefronts (80 KB of LDS a
+// workgroup).  With counters (15.3 M particles, before): MFMA 38 % and other
+// vector instructions 31 % of the cycles, LDS 47 % busy.  So the inner loop is
+// kept to the products and five address increments per four steps, with two
+// steps to an LDS read; 2^27 particles on 7,456 blocks 6.37 -> 5.88 ms, 15.3 M
+// in FP32 0.69 -> 0.62.  Three wavefronts per SIMD (records written in
+// halves of 32 particles, 47 KB) took 8.6 ms: the halves double the record stores.
 //
 // PAIRED: eight wavefronts, two per SIMD (a z-layer's two row pairs), run
 // in opposite phases locked by workgroup barriers: while one builds the
 // records of its next chunk (VALU), the other issues the matrix products of
 // its current one (MFMA), so the two units overlap instead of taking turns.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "amps_common.h"
 #include "center_device.h"
@@ -67,7 +80,8 @@ constexpr int waves_of() { return PAIRED ? 8 : 4; }
 
 // VF32: FP32 velocities (widened when the record is built, not at the load:
 // a conversion there would wait for the prefetched data)
-template <bool BC, bool PAIRED, bool FUSED, bool VF32>
+// NCW: cells per wavefront, 16 (a z-layer of the sub-tile), 8 or 4
+template <bool BC, bool PAIRED, bool FUSED, bool VF32, int NCW>
 __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(MeshView m, Species sp, double dtTotal,
                                                                  const double* __restrict__ B,
                                                                  const int* __restrict__ offset,
@@ -80,27 +94,28 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
                                                                  const double* __restrict__ Bc,
                                                                  const int* __restrict__ src) {
   constexpr int MW = waves_of<PAIRED>();
-  constexpr int NCW = PAIRED ? 8 : 16;  // cells per wavefront
-  __shared__ double sB[125 * 3];
-  // 8 doubles of padding: the operand loads run up to two steps (8
+  constexpr int WPL = 16 / NCW, LZ = MW / WPL;  // wavefronts per layer, layers per workgroup
+  constexpr int TPB = 4 * (NC / LZ);            // workgroups per block
+  __shared__ double sB[25 * (LZ + 1) * 3];
+  // 16 doubles of padding: the operand loads run up to four steps (16
   // particles) past a segment's last particle, and are not used there
-  __shared__ double rec[MW][NFLD * FS + 8];
-  __shared__ double sconst[MAX_SPEC][3];  // chargeQ, QdT_over_2m, matrixConst
+  __shared__ double rec[MW][NFLD * FS + 16];
+  __shared__ double sconst[MAX_SPEC + 1][3];  // chargeQ, QdT_over_2m, matrixConst; the last: an empty place
   __shared__ int sfirst[MW][NCW], scum[MW][NCW + 1];
-  __shared__ double sstage[MW][CS];  // a finished cell's record, written out in full lines
+  __shared__ __align__(16) double sstage[MW][CS + 2];  // a finished cell's record, written out in full lines, and a spare place
   __shared__ int smaxchunks;
-  const int tile = xcd_tile();  // the 8 sub-tiles of a block on one XCD
-  const int b = tile >> 3;
-  const int st = tile & 7;
-  const int sx = (st & 1) * 4, sy = ((st >> 1) & 1) * 4, sz = (st >> 2) * 4;
+  const int tile = xcd_tile();  // the workgroups of a block on one XCD
+  const int b = tile / TPB;
+  const int st = tile % TPB;
+  const int sx = (st & 1) * 4, sy = ((st >> 1) & 1) * 4, sz = (st >> 2) * LZ;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // wavefront w: z-layer w % 4, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
-  const int zc = sz + (w & 3);
-  const int row0 = PAIRED ? 2 * (w >> 2) : 0;
+  // wavefront w: layer w / WPL, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
+  const int zl = w / WPL, zc = sz + zl;
+  const int row0 = (w % WPL) * (NCW / 4);
   const int keybase = b * NCELL;
   if constexpr (!BC) {
     const double* Bb = B + (size_t)b * NCORNER * 3;
-    for (int i = threadIdx.x; i < 125 * 3; i += blockDim.x) {
+    for (int i = threadIdx.x; i < 25 * (LZ + 1) * 3; i += blockDim.x) {
       const int cidx = i / 3, d = i % 3;
       const int a0 = cidx % 5, a1 = (cidx / 5) % 5, a2 = cidx / 25;
       sB[i] = Bb[3 * ((sx + a0) + NN * ((sy + a1) + NN * (sz + a2))) + d];
@@ -125,12 +140,17 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     sconst[s][1] = QdT_over_2m;
     sconst[s][2] = chargeQ * QdT_over_2m / CellVolume;
   }
+  if (threadIdx.x < 3) sconst[MAX_SPEC][threadIdx.x] = 0.0;
   auto cellkey = [&](int c) { return keybase + (sx + (c & 3)) + NC * ((sy + row0 + (c >> 2)) + NC * zc); };
-  // this wavefront's cells: first particle, running counts
+  // this wavefront's cells: first particle, running counts, each rounded up to
+  // whole steps of 4 particles
+  int cntk = 0;
   {
     // counts of lanes' cells, then an inclusive scan across the lanes
     const int ck = cellkey(lane < NCW ? lane : 0);
-    const int o0 = offset[ck], cnt = lane < NCW ? offset[ck + 1] - o0 : 0;
+    const int o0 = offset[ck];
+    cntk = lane < NCW ? offset[ck + 1] - o0 : 0;
+    const int cnt = (cntk + 3) & ~3;
     int incl = cnt;
 #pragma unroll
     for (int d = 1; d < NCW; d <<= 1) {
@@ -165,7 +185,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     }
   }
   const int oa = (F_A + j) * FS, o0a = f0a * FS, o0b = f0b * FS, o1a = f1a * FS, o1b = f1b * FS;
-  // destinations of the 8 accumulator values; -1: unused.  v_mfma_f64_16x16x4f64
+  // destinations of the 8 accumulator values; CS: unused.  v_mfma_f64_16x16x4f64
   // holds A[i][k] in lane i + 16k, B[k][j] in lane j + 16k and D[i][j] in
   // lane 16 (i % 4) + j, accumulator register i / 4.
   double* S = sstage[w];
@@ -175,7 +195,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int i = slot + 4 * r, col = 16 * T + j;
-      int o = -1;
+      int o = CS;  // not kept
       if (i < 9 && col < 27) {
         o = 24 + 9 * (i + 9 * (col / 9)) + col % 9;
       } else if (i >= 9 && i < 15 && col >= 27 && col < 31) {
@@ -198,9 +218,16 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   // from a position in the concatenation to the particle's index
   const int cumk = lane < NCW ? cum[lane] : 0;
   const int dk = lane < NCW ? sfirst[w][lane] - cum[lane] : 0;
-  // the particles at positions pbase + lane (called by the whole wavefront):
-  // a position's cell is the last one that starts at or before it
-  auto fetch = [&](int pbase, Pre& n) {
+  const int endk = cumk + cntk;  // and where its particles end
+  // where the particle at position pbase + lane is (called by the whole
+  // wavefront): a position's cell is the last one that starts at or before it.
+  // FUSED: the particles are still where the last compaction found them,
+  // particle p of the new order at src[p]; that load is a chunk ahead of the
+  // ones that need it, so that no wavefront waits for it.
+  struct Idx {
+    int q, c;  // q < 0: an empty place, up to three at the end of a cell
+  };
+  auto index = [&](int pbase, Idx& ix) {
     const int pos = pbase + lane;
     int c = __popcll(__ballot(lane >= 1 && lane < NCW && cumk <= pbase));
     uint64_t starts = __ballot(lane >= 1 && lane < NCW && cumk > pbase && cumk <= pbase + 63);
@@ -210,11 +237,18 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
       c += (pos >= __builtin_amdgcn_readlane(cumk, k)) ? 1 : 0;
     }
     const int p = pos + __shfl(dk, c, 64);
-    if (pos < total) {
-      n.c = c;
-      // FUSED: the particles are still where the last compaction found
-      // them, particle p of the new order at src[p]
-      const int q = FUSED ? src[p] : p;
+    ix.c = c;
+    ix.q = -1;
+    if (pos < __shfl(endk, c, 64)) ix.q = FUSED ? src[p] : p;
+  };
+  auto fetch = [&](const Idx& ix, Pre& n) {
+    const int q = ix.q;
+    n.c = ix.c;
+    // an empty place: no charge, so that its record adds zeros
+    n.s = MAX_SPEC;
+#pragma unroll
+    for (int d = 0; d < 3; d++) n.x[d] = g.xmin[d], n.v[d] = 0.0, n.vf[d] = 0.f;
+    if (q >= 0) {
       n.x[0] = x[q], n.x[1] = x[cap + q], n.x[2] = x[2 * cap + q];
       if constexpr (VF32) {
         const float* vf = (const float*)v;
@@ -234,23 +268,28 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     const int key = cellkey(c);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      if (oidx[r] >= 0) S[oidx[r]] = C0[r];
-      if (oidx[4 + r] >= 0) S[oidx[4 + r]] = C1[r];
+      S[oidx[r]] = C0[r];
+      S[oidx[4 + r]] = C1[r];
     }
     C0 = dbl4{0.0, 0.0, 0.0, 0.0};
     C1 = C0;
     wave_lds_sync();
     // 2176 bytes from a 128-byte boundary: every store covers whole lines
-    double* dst = cellpart + (size_t)key * CS;
+    double2* dst = (double2*)(cellpart + (size_t)key * CS);
 #pragma unroll
-    for (int i = lane; i < CS; i += 64) dst[i] = S[i];
+    for (int i = 0; i < CS / 2; i += 64)
+      if (i + lane < CS / 2) dst[i + lane] = ((const double2*)S)[i + lane];
     wave_lds_sync();
   };
   // cells with no particles before the first particle
   while (cur < NCW && uniform(cum[cur + 1]) == 0) flush(cur++);
 
-  fetch(0, n1);
-  fetch(64, n2);
+  Idx ix = {0, 0}, ix2 = {0, 0};
+  index(0, ix);
+  index(64, ix2);
+  fetch(ix, n1);
+  fetch(ix2, n2);
+  index(128, ix);
   // the records of the chunk starting at particle base (VALU) from its
   // particles in nb; the particles two chunks ahead are then loaded into nb
   // (chunks alternate between n1 and n2)
@@ -286,9 +325,9 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
         double lxy[4];
 #pragma unroll
         for (int l = 0; l < 4; l++) lxy[l] = Lf[l >> 1] * Lf[2 + (l & 1)];
-        // the cell's lower corner in the staged 5 x 5 x 5 corners; corner l
+        // the cell's lower corner in the staged corners; corner l
         // at a fixed offset from it
-        const double* sBc = sB + 3 * ((nc & 3) + 5 * (row0 + (nc >> 2)) + 25 * (w & 3));
+        const double* sBc = sB + 3 * ((nc & 3) + 5 * (row0 + (nc >> 2)) + 25 * zl);
 #pragma unroll
         for (int l = 0; l < 8; l++) {
           const double wl = lxy[l >> 1] * Lf[4 + (l & 1)];
@@ -351,7 +390,8 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
         for (int by = 0; by < 2; by++) FLD(F_WYZ + by + 2 * bz) = Lf[2 + by] * Lf[4 + bz];
 #undef FLD
     }
-    fetch(base + 128, nb);  // in flight while two chunks are accumulated
+    fetch(ix, nb);  // in flight while two chunks are accumulated
+    index(base + 192, ix);
   };
   // the matrix products of that chunk, cell by cell, and the finished cells' records
   auto accumulate = [&](int base) {
@@ -360,62 +400,62 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     while (q < cend) {
       const int ce = uniform(cum[cur + 1]);
       const int se = ce < cend ? ce : cend;
-      // full steps of 4 particles, the operands of step t + 1 loaded while step t runs
+      // steps of 4 particles
       const int nfull = (se - q) >> 2;
       const double* R = R0 + (q - base + slot);
       if (nfull > 0) {
-        // the raw operands of two steps in flight ahead of the products (the
-        // LDS latency under load exceeds one step's two MFMAs); the factors
-        // are multiplied just before use
+        // the raw operands of four steps in flight ahead of the products (the
+        // LDS latency under load exceeds one step's two MFMAs), two steps to
+        // a ds_read2_b64; the factors are multiplied just before use.  The five
+        // running LDS addresses are opaque to the compiler, which otherwise adds
+        // a common offset to each of them again for every pair of steps: vector
+        // instructions and MFMAs share the issue slots that bound this pass.
         struct Ops {
-          double a, x0, y0, x1, y1;
+          double a[2], x0[2], y0[2], x1[2], y1[2];
         };
-        // one pointer per operand field, advanced by two steps per iteration
-        const double *Ra = R + oa, *Rx0 = R + o0a, *Ry0 = R + o0b, *Rx1 = R + o1a, *Ry1 = R + o1b;
+        typedef const __attribute__((address_space(3))) double* lds_t;
+        unsigned pA = (unsigned)(size_t)(lds_t)(R + oa), pX0 = (unsigned)(size_t)(lds_t)(R + o0a),
+                 pY0 = (unsigned)(size_t)(lds_t)(R + o0b), pX1 = (unsigned)(size_t)(lds_t)(R + o1a),
+                 pY1 = (unsigned)(size_t)(lds_t)(R + o1b);
         auto ld = [&](int k, Ops& o) {
-          o.a = Ra[k];
-          o.x0 = Rx0[k];
-          o.y0 = Ry0[k];
-          o.x1 = Rx1[k];
-          o.y1 = Ry1[k];
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            o.a[i] = ((lds_t)(size_t)pA)[k + 4 * i];
+            o.x0[i] = ((lds_t)(size_t)pX0)[k + 4 * i];
+            o.y0[i] = ((lds_t)(size_t)pY0)[k + 4 * i];
+            o.x1[i] = ((lds_t)(size_t)pX1)[k + 4 * i];
+            o.y1[i] = ((lds_t)(size_t)pY1)[k + 4 * i];
+          }
         };
-        auto step = [&](const Ops& o) {
-          const double b0 = o.x0 * o.y0, b1 = o.x1 * o.y1;
-          C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a, b0, C0, 0, 0, 0);
-          C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a, b1, C1, 0, 0, 0);
+        auto step = [&](const Ops& o, int i) {
+          const double b0 = o.x0[i] * o.y0[i], b1 = o.x1[i] * o.y1[i];
+          C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[i], b0, C0, 0, 0, 0);
+          C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[i], b1, C1, 0, 0, 0);
         };
-        // two operand sets, unrolled by two so that neither is copied while
-        // its loads are in flight; each is reloaded right after its products
-        // (the loads of the two steps past the last one read records past
-        // the segment, inside rec[], and are not used)
+        // two operand sets, each reloaded right after its products (the loads
+        // of the four steps past the last one read records past the segment,
+        // inside rec[], and are not used)
         Ops pa, pb;
         ld(0, pa);
-        ld(4, pb);
+        ld(8, pb);
         __builtin_amdgcn_sched_barrier(0);
-        int t = 0;
-        for (; t + 1 < nfull; t += 2) {
+        int t = nfull;
+        for (; t >= 4; t -= 4) {
           // the scheduling barriers keep each reload where it is issued
-          step(pa);
-          Ra += 8, Rx0 += 8, Ry0 += 8, Rx1 += 8, Ry1 += 8;
+          step(pa, 0);
+          step(pa, 1);
+          pA += 128, pX0 += 128, pY0 += 128, pX1 += 128, pY1 += 128;
+          asm volatile("" : "+v"(pA), "+v"(pX0), "+v"(pY0), "+v"(pX1), "+v"(pY1));
           ld(0, pa);
           __builtin_amdgcn_sched_barrier(0);
-          step(pb);
-          ld(4, pb);
+          step(pb, 0);
+          step(pb, 1);
+          ld(8, pb);
           __builtin_amdgcn_sched_barrier(0);
         }
-        if (t < nfull) step(pa);
-        R += 4 * nfull;
-      }
-      if (q + 4 * nfull < se) {
-        // the cell's last 1-3 particles in this chunk: the other slots add zero
-        double a = 0.0, b0 = 0.0, b1 = 0.0;
-        if (q + 4 * nfull + slot < se) {
-          a = R[oa];
-          b0 = R[o0a] * R[o0b];
-          b1 = R[o1a] * R[o1b];
-        }
-        C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, C0, 0, 0, 0);
-        C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, C1, 0, 0, 0);
+        if (t >= 1) step(pa, 0);
+        if (t >= 2) step(pa, 1);
+        if (t >= 3) step(pb, 0);
       }
       q = se;
       if (q == ce) {
@@ -461,13 +501,14 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   }
 }
 
-template <bool BC, bool PAIRED, bool FUSED, bool VF32>
+template <bool BC, bool PAIRED, bool FUSED, bool VF32, int NCW>
 void launch(amps_ctx* c, double dt) {
   const int k = c->cur;
   // FUSED: the particles are read from the previous buffer through the
   // migration's source indices
   const int r = FUSED ? 1 - k : k;
-  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32>), dim3((unsigned)c->mv.nb * 8),
+  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32, NCW>),
+                     dim3((unsigned)c->mv.nb * (32 / waves_of<PAIRED>() * (16 / NCW))),
                      dim3(64 * waves_of<PAIRED>()), 0, c->stream, c->mv, c->sp, dt, c->d_B, c->d_offset, c->cap,
                      c->d_x[r], c->d_v[r], c->precision == AMPS_FP32 ? 1 : 0, c->d_spec[r], c->d_cellpart, c->d_Bc,
                      c->d_tmpsrc);
@@ -475,7 +516,28 @@ void launch(amps_ctx* c, double dt) {
 
 template <bool BC, bool PAIRED, bool FUSED>
 void launch_v(amps_ctx* c, double dt, bool vf32) {
-  vf32 ? launch<BC, PAIRED, FUSED, true>(c, dt) : launch<BC, PAIRED, FUSED, false>(c, dt);
+  auto go = [&](auto ncw) {
+    constexpr int N = decltype(ncw)::value;
+    vf32 ? launch<BC, PAIRED, FUSED, true, N>(c, dt) : launch<BC, PAIRED, FUSED, false, N>(c, dt);
+  };
+  if constexpr (PAIRED) {
+    go(std::integral_constant<int, 8>());
+  } else if constexpr (BC) {
+    go(std::integral_constant<int, 16>());
+  } else {
+    // fewer cells per wavefront where 16 would not give the chip its 8
+    // wavefronts per CU: 8 blocks take 21, 13.6 and 10.5 us with 16, 8 and 4;
+    // at 64 blocks (one round of wavefronts) 16 is ahead, 40.9, 42.7 and
+    // 46.5 us, and on 7,456 blocks 5.88, 6.11 and 6.84 ms: each wavefront
+    // pays once for its first loads
+    const int64_t waves = (int64_t)c->mv.nb * 32, resident = (int64_t)c->n_cu * 8;
+    if (waves >= resident)
+      go(std::integral_constant<int, 16>());
+    else if (2 * waves >= resident)
+      go(std::integral_constant<int, 8>());
+    else
+      go(std::integral_constant<int, 4>());
+  }
 }
 
 }  // namespace

@@ -546,6 +546,50 @@ def test_deposit_ragged_cells(gpu_ctx, kernel, paired, nch):
     assert np.all(Mm[zero] == 0) and np.all(J[zero] == 0)
 
 
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("nblocks", [8, 36, 64])
+def test_deposit_cells_per_wavefront(gpu_ctx, nblocks, precision):
+    """Meshes on which the matrix-core pass gives a wavefront 4, 8 and 16
+    cells, every cell count from 0 to 7 and around the 64-particle chunk
+    (empty places at the cells' ends): against the oracle on the same
+    particles, the bound of test_deposit_ragged_cells, and after a step's own
+    migration (sources through its indices) as after a plain one."""
+    mesh = M.uniform_mesh(2 if nblocks == 64 else 1)
+    if nblocks == 36:
+        lv, ijk = M.refine(mesh.level, mesh.ijk, lambda lev, i, j, k: i == 0)
+        mesh = M.BlockMesh(lv, ijk, lmax=mesh.lmax)
+    assert mesh.nblocks == nblocks
+    E, B = M.corner_fields(mesh)
+    dt = 0.05
+    sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
+    full = M.per_cell_particles(mesh, [35, 35], [0.05, 0.005], drift=(0.01, 0.0, 0.0))
+    key = full.blk.astype(np.int64) * 512 + full.cell
+    order = np.argsort(key, kind="stable")
+    rank = np.empty(full.n, np.int64)
+    rank[order] = np.arange(full.n) - np.searchsorted(key[order], key[order])
+    want = np.array([0, 1, 2, 3, 4, 5, 7, 63, 64, 65, 70])[np.arange(mesh.ncells) % 11]
+    parts = full.take(np.flatnonzero(rank < want[key]))
+    st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+    st.set_particles(parts, precision=precision)
+    set_deposit_variant(gpu_ctx, 2, 12)
+    try:
+        J, Mm = st.UpdateJMassMatrix(dt)
+        g, _ = st.get_particles()
+        om = O.Mesh(mesh)
+        noc, keys = om.build_nodes()
+        Jo, Mo = O.deposit(om, B, sp, dt, g, noc, len(keys))
+        for a, b in ((J, Jo), (Mm, Mo)):
+            assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1)).all()
+        if nblocks != 36:  # J and M on the device are read through the mass term, single-level meshes only
+            probe = np.random.default_rng(3).standard_normal((len(keys), 3))
+            st.run_steps(1, dt, use_graph=False)  # its deposit reads through the source indices
+            fused = st.MassMatrixApply(probe, 1.0)
+            st.UpdateJMassMatrix(dt, copy_out=False)
+            assert np.abs(fused).max() > 0 and np.array_equal(fused, st.MassMatrixApply(probe, 1.0))
+    finally:
+        set_deposit_variant(gpu_ctx, 1, 6)
+
+
 def test_deposit_after_push_and_migration(gpu_ctx, dep_case):
     mesh, E, B, parts, sp, dt = dep_case
     st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
