@@ -183,6 +183,8 @@ struct amps_ctx {
   // deposit
   double* d_cellpart = nullptr;
   double* d_nodeout = nullptr;
+  char* h_pin = nullptr;       // pinned slots of the copies to and from the caller's arrays
+  hipEvent_t pin_ev[8] = {};   // their last use
   double* d_pack = nullptr;    // [PACK_DOUBLES] J or M columns on their way to the host
   int* d_ecsim_nbr = nullptr;  // [nnodes][27] neighbour nodes of the ECSIM stencil, -1 outside
   // ECSIM field equation (ecsim_field.hip)
@@ -245,6 +247,10 @@ void tend(amps_ctx* c, int k);
 // per-feature state release (trace.hip, mlp.hip)
 void trace_free(amps_ctx* c);
 void mlp_free(amps_ctx* c);
+void host_copy_init(amps_ctx* c);
+void host_copy_free(amps_ctx* c);
+int copy_to_host(amps_ctx* c, void* dst, const void* src, size_t bytes);
+int copy_to_device(amps_ctx* c, void* dst, const void* src, size_t bytes);
 // device-wide exclusive scan of n ints in place; total written to total_out
 int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* total_out);
 // the stayers before each mask word; the exclusive scan of the keys' new

@@ -56,6 +56,8 @@ __global__ void k_generate(MeshView, GenArgs, int64_t, double*, double*, uint8_t
 __global__ void k_copy_probe(const float4*, float4*, int64_t);
 template <int W>
 __global__ void k_pack_cols(int64_t, const double*, double*);
+__global__ void k_host_columns(int64_t, const uint8_t*, const int*, const int8_t*, int*);
+__global__ void k_widen_planes(int64_t, int64_t, const float*, double*);
 namespace amps {
 int upload_inv_index_matrix(hipStream_t s);
 }
@@ -186,6 +188,7 @@ extern "C" int amps_gpu_create(int device, amps_ctx** out) {
   HIP_TRY(hipMalloc(&c->d_ntiles, sizeof(int) * 4));
   if (int r = upload_inv_index_matrix(c->stream)) return r;
   HIP_TRY(hipStreamSynchronize(c->stream));
+  host_copy_init(c);
   *out = c;
   return AMPS_OK;
 }
@@ -199,6 +202,7 @@ extern "C" int amps_gpu_destroy(amps_ctx* c) {
   trace_free(c);
   mlp_free(c);
   exits_free(c);
+  host_copy_free(c);
   (void)hipFree(c->d_n);
   (void)hipFree(c->d_ntiles);
   (void)hipFree(c->d_tiles);
@@ -623,8 +627,8 @@ extern "C" int amps_gpu_set_fields(amps_ctx* c, const double* E, const double* B
   const size_t nbytes = sizeof(double) * (size_t)c->mv.nb * NCORNER * 3;
   if (!c->d_E) HIP_TRY(hipMalloc(&c->d_E, nbytes));
   if (!c->d_B) HIP_TRY(hipMalloc(&c->d_B, nbytes));
-  HIP_TRY(hipMemcpyAsync(c->d_E, E, nbytes, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->d_B, B, nbytes, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, c->d_E, E, nbytes)) return r;
+  if (int r = copy_to_device(c, c->d_B, B, nbytes)) return r;
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->has_fields = true;
   return AMPS_OK;
@@ -798,38 +802,34 @@ extern "C" int amps_gpu_get_particles(amps_ctx* c, double* x, double* v, int32_t
   if (n == 0) return AMPS_OK;
   const int64_t cap = c->cap;
   const int k = c->cur;
+  auto planes = [&](double* out, const double* in, int64_t stride) {
+    if (stride == n) return copy_to_host(c, out, in, sizeof(double) * 3 * n);
+    for (int d = 0; d < 3; d++)
+      if (int r = copy_to_host(c, out + d * n, in + d * stride, sizeof(double) * n)) return r;
+    return 0;
+  };
+  // what the host's layout widens or splits is written out on the device, into
+  // the position buffer that the next compaction fills (24 bytes a particle)
+  double* wide = c->d_x[1 - k];
+  const dim3 grid((unsigned)((n + 255) / 256));
   if (x)
-    for (int d = 0; d < 3; d++)
-      HIP_TRY(hipMemcpy(x + d * n, c->d_x[k] + d * cap, sizeof(double) * n, hipMemcpyDeviceToHost));
+    if (int r = planes(x, c->d_x[k], cap)) return r;
   if (v && c->precision == AMPS_FP32) {
-    std::vector<float> f((size_t)n);
-    for (int d = 0; d < 3; d++) {
-      HIP_TRY(hipMemcpy(f.data(), (const float*)c->d_v[k] + d * cap, sizeof(float) * n, hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < n; i++) v[d * n + i] = f[(size_t)i];
-    }
+    hipLaunchKernelGGL(k_widen_planes, grid, dim3(256), 0, c->stream, n, cap, (const float*)c->d_v[k], wide);
+    HIP_TRY(hipGetLastError());
+    if (int r = planes(v, wide, n)) return r;
   } else if (v) {
-    for (int d = 0; d < 3; d++)
-      HIP_TRY(hipMemcpy(v + d * n, c->d_v[k] + d * cap, sizeof(double) * n, hipMemcpyDeviceToHost));
+    if (int r = planes(v, c->d_v[k], cap)) return r;
   }
-  if (spec) {
-    std::vector<uint8_t> s((size_t)n);
-    HIP_TRY(hipMemcpy(s.data(), c->d_spec[k], n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) spec[i] = s[(size_t)i];
-  }
-  if (blk || cell) {
-    std::vector<int> kk((size_t)n);
-    HIP_TRY(hipMemcpy(kk.data(), c->d_key[k], sizeof(int) * n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) {
-      if (blk) blk[i] = kk[(size_t)i] / NCELL;
-      if (cell) cell[i] = kk[(size_t)i] % NCELL;
-    }
-  }
-  if (id) HIP_TRY(hipMemcpy(id, c->d_id[k], sizeof(int64_t) * n, hipMemcpyDeviceToHost));
-  if (code) {
-    std::vector<int8_t> s((size_t)n);
-    HIP_TRY(hipMemcpy(s.data(), c->d_code, n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) code[i] = s[(size_t)i];
-  }
+  int* w = (int*)wide;  // spec, blk, cell, code of n each
+  hipLaunchKernelGGL(k_host_columns, grid, dim3(256), 0, c->stream, n, c->d_spec[k], c->d_key[k], c->d_code, w);
+  HIP_TRY(hipGetLastError());
+  int32_t* out[4] = {spec, blk, cell, code};
+  for (int q = 0; q < 4; q++)
+    if (out[q])
+      if (int r = copy_to_host(c, out[q], w + q * n, sizeof(int) * n)) return r;
+  if (id)
+    if (int r = copy_to_host(c, id, c->d_id[k], sizeof(int64_t) * n)) return r;
   return AMPS_OK;
 }
 
@@ -1136,7 +1136,7 @@ static int copy_node_cols(amps_ctx* c, int col, double* out) {
     hipLaunchKernelGGL((k_pack_cols<W>), dim3((unsigned)((n * W + 255) / 256)), dim3(256), 0, c->stream, n * W,
                        c->d_nodeout + n0 * NODE_STRIDE + col, c->d_pack);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out + n0 * W, c->d_pack, sizeof(double) * n * W, hipMemcpyDeviceToHost, c->stream));
+    if (int r = copy_to_host(c, out + n0 * W, c->d_pack, sizeof(double) * n * W)) return r;
   }
   return 0;
 }
@@ -1160,7 +1160,6 @@ extern "C" int amps_gpu_update_j_mass_matrix(amps_ctx* c, double dt, double* J_o
     if (int r = copy_node_cols<3>(c, 0, J_out)) return r;
   if (M_out)
     if (int r = copy_node_cols<243>(c, 3, M_out)) return r;
-  if (J_out || M_out) HIP_TRY(hipStreamSynchronize(c->stream));
   return AMPS_OK;
 }
 

@@ -949,15 +949,14 @@ extern "C" int amps_gpu_ecsim_operator(amps_ctx* c, const amps_ecsim_params* p, 
   Work W;
   if (int r = prepare(c, p, 0, &W, "amps_gpu_ecsim_operator")) return r;
   const size_t n3 = 3 * (size_t)c->nnodes;
-  HIP_TRY(hipMemcpyAsync(W.x, x, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, W.x, x, sizeof(double) * n3)) return r;
   for (int i = 0; i < reps; i++) {
     tbegin(c);
     launch_op(c, W, fpdt_of(p), W.x, W.w);
     tend(c, AMPS_K_ECSIM);
   }
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(y, W.w, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (int r = copy_to_host(c, y, W.w, sizeof(double) * n3)) return r;
   return AMPS_OK;
 }
 
@@ -968,14 +967,13 @@ extern "C" int amps_gpu_ecsim_rhs(amps_ctx* c, const amps_ecsim_params* p, const
   if (int r = prepare(c, p, 0, &W, "amps_gpu_ecsim_rhs")) return r;
   const int64_t nn = c->nnodes;
   const size_t n3 = 3 * (size_t)nn, c3 = 3 * (size_t)c->mv.nb * NCELL;
-  HIP_TRY(hipMemcpyAsync(W.En, E_n, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(W.Bc, B_c, sizeof(double) * c3, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, W.En, E_n, sizeof(double) * n3)) return r;
+  if (int r = copy_to_device(c, W.Bc, B_c, sizeof(double) * c3)) return r;
   hipLaunchKernelGGL(k_ecsim_rhs, dim3((unsigned)((((nn + 7) / 8) + 7) / 8 * 8)), dim3(256), 0, c->stream, nn, c->d_nodeout, c->d_ecsim_nbr,
                      c->d_ecsim_bnd, c->d_ecsim_cells8, W.C, p->dt, p->theta, p->E_conv, p->B_conv, W.En, W.Bc,
                      W.rhs);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(rhs, W.rhs, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (int r = copy_to_host(c, rhs, W.rhs, sizeof(double) * n3)) return r;
   return AMPS_OK;
 }
 
@@ -988,12 +986,11 @@ extern "C" int amps_gpu_ecsim_solve(amps_ctx* c, const amps_ecsim_params* p, con
   Work W;
   if (int r = prepare(c, p, restart, &W, "amps_gpu_ecsim_solve")) return r;
   const size_t n3 = 3 * (size_t)c->nnodes;
-  HIP_TRY(hipMemcpyAsync(W.rhs, rhs, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, W.rhs, rhs, sizeof(double) * n3)) return r;
   int it = 0;
   double rr = 0.0;
   if (int r = gmres(c, W, fpdt_of(p), tol, max_iter, restart, true, &it, &rr)) return r;
-  HIP_TRY(hipMemcpyAsync(dE, W.x, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (int r = copy_to_host(c, dE, W.x, sizeof(double) * n3)) return r;
   *iters = it;
   *rel_residual = rr;
   return AMPS_OK;
@@ -1006,8 +1003,8 @@ extern "C" int amps_gpu_ecsim_update_b(amps_ctx* c, const amps_ecsim_params* p, 
   if (int r = prepare(c, p, 0, &W, "amps_gpu_ecsim_update_b")) return r;
   const size_t n3 = 3 * (size_t)c->nnodes;
   const int64_t ncell = (int64_t)c->mv.nb * NCELL;
-  HIP_TRY(hipMemcpyAsync(W.Eth, E_theta, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(W.Bc, B_c, sizeof(double) * 3 * ncell, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, W.Eth, E_theta, sizeof(double) * n3)) return r;
+  if (int r = copy_to_device(c, W.Bc, B_c, sizeof(double) * 3 * ncell)) return r;
   double dx[3];
   cell_size(c, dx);
   double c4[3];
@@ -1015,8 +1012,7 @@ extern "C" int amps_gpu_ecsim_update_b(amps_ctx* c, const amps_ecsim_params* p, 
   hipLaunchKernelGGL(k_ecsim_update_b, grid_of(ncell), dim3(256), 0, c->stream, ncell, c->d_ecsim_noc, W.Eth,
                      W.Bc, c4[0], c4[1], c4[2], p->E_conv, p->B_conv, W.Bout);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(B_out, W.Bout, sizeof(double) * 3 * ncell, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (int r = copy_to_host(c, B_out, W.Bout, sizeof(double) * 3 * ncell)) return r;
   return AMPS_OK;
 }
 
@@ -1031,8 +1027,8 @@ extern "C" int amps_gpu_ecsim_time_step(amps_ctx* c, const amps_ecsim_params* p,
   const int64_t nn = c->nnodes;
   const size_t n3 = 3 * (size_t)nn;
   const int64_t ncell = (int64_t)c->mv.nb * NCELL;
-  HIP_TRY(hipMemcpyAsync(W.En, E, sizeof(double) * n3, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(W.Bc, B_c, sizeof(double) * 3 * ncell, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, W.En, E, sizeof(double) * n3)) return r;
+  if (int r = copy_to_device(c, W.Bc, B_c, sizeof(double) * 3 * ncell)) return r;
   // right-hand side, GMRES, E^{n+theta} and E^{n+1}, B^{n+1}
   hipLaunchKernelGGL(k_ecsim_rhs, dim3((unsigned)((((nn + 7) / 8) + 7) / 8 * 8)), dim3(256), 0, c->stream, nn, c->d_nodeout, c->d_ecsim_nbr,
                      c->d_ecsim_bnd, c->d_ecsim_cells8, W.C, p->dt, p->theta, p->E_conv, p->B_conv, W.En, W.Bc,
@@ -1049,10 +1045,10 @@ extern "C" int amps_gpu_ecsim_time_step(amps_ctx* c, const amps_ecsim_params* p,
   hipLaunchKernelGGL(k_ecsim_update_b, grid_of(ncell), dim3(256), 0, c->stream, ncell, c->d_ecsim_noc, W.Eth,
                      W.Bc, c4[0], c4[1], c4[2], p->E_conv, p->B_conv, W.Bout);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(E, W.E1, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-  if (E_theta) HIP_TRY(hipMemcpyAsync(E_theta, W.Eth, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipMemcpyAsync(B_c, W.Bout, sizeof(double) * 3 * ncell, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (int r = copy_to_host(c, E, W.E1, sizeof(double) * n3)) return r;
+  if (E_theta)
+    if (int r = copy_to_host(c, E_theta, W.Eth, sizeof(double) * n3)) return r;
+  if (int r = copy_to_host(c, B_c, W.Bout, sizeof(double) * 3 * ncell)) return r;
   *iters = it;
   *rel_residual = rr;
   return AMPS_OK;

@@ -730,12 +730,10 @@ extern "C" int amps_gpu_mlp_predict(amps_ctx* c, int64_t n, const float* X, floa
     HIP_TRY(hipMalloc(&s->qy, sizeof(float) * n));
     s->qcap = n;
   }
-  HIP_TRY(hipMemcpyAsync(s->qX, X, sizeof(float) * DIN * n, hipMemcpyHostToDevice, c->stream));
+  if (int r = copy_to_device(c, s->qX, X, sizeof(float) * DIN * n)) return r;
   tbegin(c);
   hipLaunchKernelGGL(k_mlp_forward, dim3(forward_wgs(c, n)), dim3(256), 0, c->stream, view(s), s->qX, n, s->qy);
   HIP_TRY(hipGetLastError());
   tend(c, AMPS_K_MLP);
-  HIP_TRY(hipMemcpyAsync(y, s->qy, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return AMPS_OK;
+  return copy_to_host(c, y, s->qy, sizeof(float) * n);
 }

@@ -97,6 +97,14 @@ __global__ __launch_bounds__(256) void k_export(int64_t n, Layout L, const int* 
   if (L.w_off >= 0) put_f64<ALIGNED>(rec, L.w_off, 1.0);
 }
 
+// the number of particles of every cell in restart order (block-major, then
+// 64 i + 8 j + k); one thread per cell
+__global__ __launch_bounds__(256) void k_rank_counts(const int* __restrict__ offset, int* __restrict__ counts) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t k = i / NCELL * NCELL + cell_of_rank((int)(i % NCELL));
+  counts[i] = offset[k + 1] - offset[k];
+}
+
 // record e (restart order) -> its device position
 template <bool ALIGNED>
 __global__ __launch_bounds__(256) void k_import(int64_t n, Layout L, int64_t nseg, const int64_t* __restrict__ rbase,
@@ -164,21 +172,28 @@ extern "C" int amps_gpu_get_particles_restart(amps_ctx* c, const amps_aos_layout
   if (n_records) *n_records = n;
   const int nb = c->mv.nb;
   const int64_t nkeys = (int64_t)nb * NCELL;
-  std::vector<int> off((size_t)nkeys + 1, 0);
-  if (n > 0) HIP_TRY(hipMemcpy(off.data(), c->d_offset, sizeof(int) * (nkeys + 1), hipMemcpyDeviceToHost));
-  // restart-order counts and prefix (block-major, then 64 i + 8 j + k)
-  std::vector<int64_t> rb((size_t)nkeys + 1, 0), rbase_key((size_t)nkeys, 0);
-  for (int b = 0; b < nb; b++)
-    for (int r = 0; r < NCELL; r++) {
-      const int64_t k = (int64_t)b * NCELL + cell_of_rank(r);
-      const int cnt = off[(size_t)k + 1] - off[(size_t)k];
-      if (counts) counts[(size_t)b * NCELL + r] = cnt;
-      rb[(size_t)b * NCELL + r + 1] = rb[(size_t)b * NCELL + r] + cnt;
-    }
+  std::vector<int> own;
+  if (!counts && records && n > 0) {
+    own.resize((size_t)nkeys);
+    counts = own.data();
+  }
+  if (counts && n > 0) {
+    // the cursors of a compaction, idle between calls
+    hipLaunchKernelGGL(k_rank_counts, dim3((unsigned)(nkeys / 256)), dim3(256), 0, c->stream, c->d_offset, c->d_cursor);
+    HIP_TRY(hipGetLastError());
+    if (int r = copy_to_host(c, counts, c->d_cursor, sizeof(int) * nkeys)) return r;
+  } else if (counts) {
+    std::fill(counts, counts + nkeys, 0);
+  }
   if (!records || n == 0) return AMPS_OK;
   if (cap_records < n) return fail(AMPS_E_RANGE, "amps_gpu_get_particles_restart: record buffer too small");
-  for (int b = 0; b < nb; b++)
-    for (int cc = 0; cc < NCELL; cc++) rbase_key[(size_t)b * NCELL + restart_rank(cc)] = rb[(size_t)b * NCELL + restart_rank(cc)];
+  // the first record of every (block, restart rank)
+  std::vector<int64_t> rbase_key((size_t)nkeys);
+  int64_t first = 0;
+  for (int64_t i = 0; i < nkeys; i++) {
+    rbase_key[(size_t)i] = first;
+    first += counts[i];
+  }
   int64_t* d_rb = nullptr;
   unsigned char* d_out = nullptr;
   HIP_TRY(hipMalloc(&d_rb, sizeof(int64_t) * nkeys));
@@ -195,11 +210,10 @@ extern "C" int amps_gpu_get_particles_restart(amps_ctx* c, const amps_aos_layout
     hipLaunchKernelGGL(k_export<false>, grid, dim3(256), 0, c->stream, n, L, c->d_key[k], c->d_offset, d_rb,
                        c->d_x[k], c->d_v[k], vf32, c->d_spec[k], c->cap, d_out);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(records, d_out, (size_t)n * L.bytes, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  const int r = copy_to_host(c, records, d_out, (size_t)n * L.bytes);
   (void)hipFree(d_rb);
   (void)hipFree(d_out);
-  return AMPS_OK;
+  return r;
 }
 
 extern "C" int amps_gpu_set_particles_restart(amps_ctx* c, const amps_aos_layout* layout, const int32_t* counts,

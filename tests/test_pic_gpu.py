@@ -784,6 +784,34 @@ def test_push_fp32_error_against_fp64_oracle(gpu_ctx, mover):
     assert abs(g.n - o.n) <= max(2, o.n // 5000)
 
 
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("n", [1, 131071, 131073, 600001])
+def test_particles_to_the_host(gpu_ctx, n, precision):
+    """Columns on both sides of the size from which a copy goes through the
+    pinned slots (1 MiB: 131,072 doubles, or twice as many ints) and of
+    several chunks with a ragged last one: what was set comes back, and the
+    cells' numbers in restart order are those of the columns."""
+    import ctypes
+
+    mesh = M.uniform_mesh(2)
+    E, B = M.corner_fields(mesh)
+    p = M.uniform_particles(mesh, n, 0.1)
+    p.spec = (np.arange(n) % 2).astype(np.int32)
+    st = PicState(mesh, E, B, Species([-1.0, 1.0], [1.0, 2.0], [0.01, 0.01]), ctx=gpu_ctx)
+    st.set_particles(p, precision=precision)
+    g, code = st.get_particles()
+    g, code = _by_id(g, code)
+    v = p.v.astype(np.float32).astype(np.float64) if precision == L.FP32 else p.v
+    assert np.array_equal(g.id, p.id) and np.array_equal(g.x, p.x) and np.array_equal(g.v, v)
+    assert np.array_equal(g.spec, p.spec) and np.array_equal(g.blk, p.blk) and np.array_equal(g.cell, p.cell)
+    counts, m = np.zeros((mesh.nblocks, 512), np.int32), ctypes.c_int64()
+    L.check(st.lib.amps_gpu_get_particles_restart(gpu_ctx.h, ctypes.byref(L.aos_layout_aligned()),
+                                                  L._ptr(counts, ctypes.c_int32), None, 0, ctypes.byref(m)))
+    i, j, k = p.cell % 8, p.cell // 8 % 8, p.cell // 64
+    want = np.bincount(p.blk.astype(np.int64) * 512 + 64 * i + 8 * j + k, minlength=mesh.ncells)
+    assert m.value == n and np.array_equal(counts.ravel(), want)
+
+
 @pytest.mark.parametrize("layout_name,weight", [("aligned", False), ("aligned", True), ("packed", True)])
 def test_restart_records_round_trip(gpu_ctx, layout_name, weight):
     """ParticleBuffer records in restart order: the export follows
