@@ -181,6 +181,7 @@ struct amps_ctx {
                                // 3 eight lanes per cell
   int b_center = 0;            // 1: B from the cell-centred field (mover and deposit)
   // deposit
+  int* d_crowd = nullptr;      // crowded sub-tiles: count, list [2 n_cu], a byte per sub-tile
   double* d_cellpart = nullptr;
   double* d_nodeout = nullptr;
   char* h_pin = nullptr;       // pinned slots of the copies to and from the caller's arrays

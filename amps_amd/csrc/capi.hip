@@ -50,8 +50,8 @@ template <int NCH, bool EXACT>
 __global__ void k_deposit_cell(MeshView, Species, double, const double*, const int*, int64_t,
                                const double*, const double*, int, const uint8_t*, double*);
 template <bool MOMENT>
-__global__ void k_deposit_node(int64_t, int, const int*, const int*, const double*, double*);
-__global__ void k_deposit_node_staged(int64_t, int, const int*, const int*, const double*, double*);
+__global__ void k_deposit_node(int64_t, int, const int*, const int*, const double*, double*, int*);
+__global__ void k_deposit_node_staged(int64_t, int, const int*, const int*, const double*, double*, int*);
 __global__ void k_generate(MeshView, GenArgs, int64_t, double*, double*, uint8_t*, int*, int64_t*, int8_t*);
 __global__ void k_copy_probe(const float4*, float4*, int64_t);
 template <int W>
@@ -152,6 +152,8 @@ static void free_mesh(amps_ctx* c) {
   (void)hipFree(c->d_cursor);
   (void)hipFree(c->d_tcount);
   (void)hipFree(c->d_cellpart);
+  (void)hipFree(c->d_crowd);
+  c->d_crowd = nullptr;
   (void)hipFree(c->d_nodeout);
   (void)hipFree(c->d_pack);
   c->d_pack = nullptr;
@@ -1098,13 +1100,13 @@ static int launch_deposit(amps_ctx* c, double dt) {
   // the record-batched and matrix-core cell passes write the moment form unless bit-exact
   if (c->dep_kernel >= 1 && !c->dep_exact && c->node_staged)
     hipLaunchKernelGGL(k_deposit_node_staged, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout, c->d_crowd);
   else if (c->dep_kernel >= 1 && !c->dep_exact)
     hipLaunchKernelGGL(k_deposit_node<true>, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout, c->d_crowd);
   else
     hipLaunchKernelGGL(k_deposit_node<false>, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8, c->d_cellpart, c->d_nodeout);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8, c->d_cellpart, c->d_nodeout, c->d_crowd);
   HIP_TRY(hipGetLastError());
   tend(c, AMPS_K_DEPOSIT_NODE);
   return 0;
@@ -1118,6 +1120,10 @@ static int ensure_deposit_buffers(amps_ctx* c) {
     HIP_TRY(hipMalloc(&c->d_cellpart, sizeof(double) * n));
     HIP_TRY(hipMemset(c->d_cellpart + (size_t)c->zero_rec * CELL_STRIDE_MOMENT, 0,
                       sizeof(double) * CELL_STRIDE_MOMENT));
+  }
+  if (!c->d_crowd) {
+    HIP_TRY(hipMalloc(&c->d_crowd, sizeof(int) * (1 + 2 * (size_t)c->n_cu) + (size_t)c->mv.nb * 8));
+    HIP_TRY(hipMemset(c->d_crowd, 0, sizeof(int)));
   }
   if (!c->d_nodeout) HIP_TRY(hipMalloc(&c->d_nodeout, sizeof(double) * (size_t)c->nnodes * NODE_STRIDE));
   return 0;

@@ -40,8 +40,6 @@
 // its current one (MFMA), so the two units overlap instead of taking turns.
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 #include "amps_common.h"
 #include "center_device.h"
 #include "pic_device.h"
@@ -80,8 +78,41 @@ constexpr int waves_of() { return PAIRED ? 8 : 4; }
 
 // VF32: FP32 velocities (widened when the record is built, not at the load:
 // a conversion there would wait for the prefetched data)
-// NCW: cells per wavefront, 16 (a z-layer of the sub-tile), 8 or 4
-template <bool BC, bool PAIRED, bool FUSED, bool VF32, int NCW>
+// How the cells are split: ncw cells per wavefront; with `extra` workgroups
+// (four per list entry) in front of the others, the crowded sub-tiles take
+// one workgroup per layer and 4 cells per wavefront.
+struct Split {
+  int ncw, extra;
+  int* count;  // crowded sub-tiles; the node gather clears it for the next pass
+  const int* list;
+  const uint8_t* crowded;  // per sub-tile
+};
+
+// The crowded sub-tiles, those with more particles than an equal share of
+// all of them for each workgroup the chip holds (so at most that many), which
+// alone would outlast the rest, and twice the mean (64 blocks are one
+// workgroup each: splitting those above the mean took 60 us instead of 41).
+// With drifted electrons standing at the walls (1,000 steps on the two-level
+// mesh, 2.0 M particles) the pass took 429 us, with the split 163, 131 at the
+// start of the run; the list takes 4.7 us.
+// 16 lanes a sub-tile, one row of 4 cells each.
+__global__ __launch_bounds__(256) void k_crowded(int ntiles, int64_t nkeys, int slots, const int* __restrict__ offset,
+                                                  int* __restrict__ count, int* __restrict__ list,
+                                                  uint8_t* __restrict__ crowded) {
+  const int t = blockIdx.x * 16 + (threadIdx.x >> 4), r = threadIdx.x & 15;
+  if (t >= ntiles) return;
+  const int st = t & 7, x = (st & 1) * 4, y = ((st >> 1) & 1) * 4 + (r & 3), z = (st >> 2) * 4 + (r >> 2);
+  const int k = (t >> 3) * NCELL + x + NC * (y + NC * z);
+  int n = offset[k + 4] - offset[k];
+  for (int d = 1; d < 16; d <<= 1) n += __shfl_xor(n, d);
+  if (r) return;
+  const int64_t total = offset[nkeys];
+  const bool c = (int64_t)n * slots > total && (int64_t)n * ntiles > 2 * total;
+  crowded[t] = c;
+  if (c) list[atomicAdd(count, 1)] = t;
+}
+
+template <bool BC, bool PAIRED, bool FUSED, bool VF32>
 __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(MeshView m, Species sp, double dtTotal,
                                                                  const double* __restrict__ B,
                                                                  const int* __restrict__ offset,
@@ -92,30 +123,47 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
                                                                  const uint8_t* __restrict__ spec,
                                                                  double* __restrict__ cellpart,
                                                                  const double* __restrict__ Bc,
-                                                                 const int* __restrict__ src) {
+                                                                 const int* __restrict__ src, Split sp4) {
   constexpr int MW = waves_of<PAIRED>();
-  constexpr int WPL = 16 / NCW, LZ = MW / WPL;  // wavefronts per layer, layers per workgroup
-  constexpr int TPB = 4 * (NC / LZ);            // workgroups per block
-  __shared__ double sB[25 * (LZ + 1) * 3];
+  constexpr int MCW = PAIRED ? 8 : 16;  // most cells per wavefront
+  __shared__ double sB[125 * 3];
   // 16 doubles of padding: the operand loads run up to four steps (16
   // particles) past a segment's last particle, and are not used there
   __shared__ double rec[MW][NFLD * FS + 16];
   __shared__ double sconst[MAX_SPEC + 1][3];  // chargeQ, QdT_over_2m, matrixConst; the last: an empty place
-  __shared__ int sfirst[MW][NCW], scum[MW][NCW + 1];
+  __shared__ int sfirst[MW][MCW], scum[MW][MCW + 1];
   __shared__ __align__(16) double sstage[MW][CS + 2];  // a finished cell's record, written out in full lines, and a spare place
   __shared__ int smaxchunks;
-  const int tile = xcd_tile();  // the workgroups of a block on one XCD
-  const int b = tile / TPB;
-  const int st = tile % TPB;
-  const int sx = (st & 1) * 4, sy = ((st >> 1) & 1) * 4, sz = (st >> 2) * LZ;
+  // cells per wavefront, wavefronts per layer, layers per workgroup
+  int ncw = PAIRED ? 8 : BC ? 16 : sp4.ncw;
+  int wpl = 16 / ncw, lz = MW / wpl;
+  int b, st, sz;
+  if (!PAIRED && !BC && (int)blockIdx.x < sp4.extra) {
+    // a layer of a crowded sub-tile
+    if ((int)blockIdx.x >= 4 * sp4.count[0]) return;
+    const int tile = sp4.list[blockIdx.x >> 2];
+    ncw = 4, wpl = 4, lz = 1;
+    b = tile >> 3, st = tile & 7;
+    sz = (st >> 2) * 4 + (blockIdx.x & 3);
+  } else {
+    // the workgroups of a block on one XCD
+    const int extra = PAIRED || BC ? 0 : sp4.extra;
+    const int bi = blockIdx.x - extra, ng = gridDim.x - extra;
+    const int tile = (bi % N_XCD) * (ng / N_XCD) + bi / N_XCD;
+    if (extra && sp4.crowded[tile]) return;
+    const int tpb = 4 * (NC / lz);  // workgroups per block
+    b = tile / tpb, st = tile % tpb;
+    sz = (st >> 2) * lz;
+  }
+  const int sx = (st & 1) * 4, sy = ((st >> 1) & 1) * 4;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // wavefront w: layer w / WPL, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
-  const int zl = w / WPL, zc = sz + zl;
-  const int row0 = (w % WPL) * (NCW / 4);
+  // wavefront w: layer w / wpl, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
+  const int zl = uniform(w / wpl), zc = sz + zl;
+  const int row0 = uniform((w % wpl) * (ncw / 4));
   const int keybase = b * NCELL;
   if constexpr (!BC) {
     const double* Bb = B + (size_t)b * NCORNER * 3;
-    for (int i = threadIdx.x; i < 25 * (LZ + 1) * 3; i += blockDim.x) {
+    for (int i = threadIdx.x; i < 75 * (lz + 1); i += blockDim.x) {
       const int cidx = i / 3, d = i % 3;
       const int a0 = cidx % 5, a1 = (cidx / 5) % 5, a2 = cidx / 25;
       sB[i] = Bb[3 * ((sx + a0) + NN * ((sy + a1) + NN * (sz + a2))) + d];
@@ -147,26 +195,26 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   int cntk = 0;
   {
     // counts of lanes' cells, then an inclusive scan across the lanes
-    const int ck = cellkey(lane < NCW ? lane : 0);
+    const int ck = cellkey(lane < ncw ? lane : 0);
     const int o0 = offset[ck];
-    cntk = lane < NCW ? offset[ck + 1] - o0 : 0;
+    cntk = lane < ncw ? offset[ck + 1] - o0 : 0;
     const int cnt = (cntk + 3) & ~3;
     int incl = cnt;
 #pragma unroll
-    for (int d = 1; d < NCW; d <<= 1) {
+    for (int d = 1; d < MCW; d <<= 1) {
       const int t = __shfl_up(incl, d, 64);
       if (lane >= d) incl += t;
     }
-    if (lane < NCW) {
+    if (lane < ncw) {
       sfirst[w][lane] = o0;
       scum[w][lane] = incl - cnt;
     }
-    if (lane == NCW - 1) scum[w][NCW] = incl;
+    if (lane == ncw - 1) scum[w][ncw] = incl;
   }
   if (threadIdx.x == 0) smaxchunks = 0;
   __syncthreads();
   const int* cum = scum[w];
-  const int total = uniform(cum[NCW]);
+  const int total = uniform(cum[ncw]);
   double* R0 = rec[w];
 
   // operand selectors of this lane: A row ia = j and B columns j, 16 + j of particle slot lane / 16
@@ -214,10 +262,10 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     float vf[3];
     int s, c;
   };
-  // lane k < NCW: where cell k starts in the concatenation, and the offset
+  // lane k < ncw: where cell k starts in the concatenation, and the offset
   // from a position in the concatenation to the particle's index
-  const int cumk = lane < NCW ? cum[lane] : 0;
-  const int dk = lane < NCW ? sfirst[w][lane] - cum[lane] : 0;
+  const int cumk = lane < ncw ? cum[lane] : 0;
+  const int dk = lane < ncw ? sfirst[w][lane] - cum[lane] : 0;
   const int endk = cumk + cntk;  // and where its particles end
   // where the particle at position pbase + lane is (called by the whole
   // wavefront): a position's cell is the last one that starts at or before it.
@@ -229,8 +277,8 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   };
   auto index = [&](int pbase, Idx& ix) {
     const int pos = pbase + lane;
-    int c = __popcll(__ballot(lane >= 1 && lane < NCW && cumk <= pbase));
-    uint64_t starts = __ballot(lane >= 1 && lane < NCW && cumk > pbase && cumk <= pbase + 63);
+    int c = __popcll(__ballot(lane >= 1 && lane < ncw && cumk <= pbase));
+    uint64_t starts = __ballot(lane >= 1 && lane < ncw && cumk > pbase && cumk <= pbase + 63);
     while (starts) {
       const int k = __builtin_ctzll(starts);
       starts &= starts - 1;
@@ -282,7 +330,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     wave_lds_sync();
   };
   // cells with no particles before the first particle
-  while (cur < NCW && uniform(cum[cur + 1]) == 0) flush(cur++);
+  while (cur < ncw && uniform(cum[cur + 1]) == 0) flush(cur++);
 
   Idx ix = {0, 0}, ix2 = {0, 0};
   index(0, ix);
@@ -460,7 +508,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
       q = se;
       if (q == ce) {
         flush(cur++);
-        while (cur < NCW && uniform(cum[cur + 1]) == q) flush(cur++);  // empty cells
+        while (cur < ncw && uniform(cum[cur + 1]) == q) flush(cur++);  // empty cells
       }
     }
   };
@@ -501,43 +549,41 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   }
 }
 
-template <bool BC, bool PAIRED, bool FUSED, bool VF32, int NCW>
-void launch(amps_ctx* c, double dt) {
+template <bool BC, bool PAIRED, bool FUSED, bool VF32>
+void launch(amps_ctx* c, double dt, const Split& sp4) {
   const int k = c->cur;
   // FUSED: the particles are read from the previous buffer through the
   // migration's source indices
   const int r = FUSED ? 1 - k : k;
-  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32, NCW>),
-                     dim3((unsigned)c->mv.nb * (32 / waves_of<PAIRED>() * (16 / NCW))),
-                     dim3(64 * waves_of<PAIRED>()), 0, c->stream, c->mv, c->sp, dt, c->d_B, c->d_offset, c->cap,
-                     c->d_x[r], c->d_v[r], c->precision == AMPS_FP32 ? 1 : 0, c->d_spec[r], c->d_cellpart, c->d_Bc,
-                     c->d_tmpsrc);
+  const unsigned grid = (unsigned)(c->mv.nb * (PAIRED || BC ? 8 : 8 * (16 / sp4.ncw)) + sp4.extra);
+  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32>), dim3(grid), dim3(64 * waves_of<PAIRED>()), 0,
+                     c->stream, c->mv, c->sp, dt, c->d_B, c->d_offset, c->cap, c->d_x[r], c->d_v[r],
+                     c->precision == AMPS_FP32 ? 1 : 0, c->d_spec[r], c->d_cellpart, c->d_Bc, c->d_tmpsrc, sp4);
 }
 
 template <bool BC, bool PAIRED, bool FUSED>
 void launch_v(amps_ctx* c, double dt, bool vf32) {
-  auto go = [&](auto ncw) {
-    constexpr int N = decltype(ncw)::value;
-    vf32 ? launch<BC, PAIRED, FUSED, true, N>(c, dt) : launch<BC, PAIRED, FUSED, false, N>(c, dt);
-  };
-  if constexpr (PAIRED) {
-    go(std::integral_constant<int, 8>());
-  } else if constexpr (BC) {
-    go(std::integral_constant<int, 16>());
-  } else {
+  Split s = {16, 0, nullptr, nullptr, nullptr};
+  if constexpr (!PAIRED && !BC) {
     // fewer cells per wavefront where 16 would not give the chip its 8
-    // wavefronts per CU: 8 blocks take 21, 13.6 and 10.5 us with 16, 8 and 4;
-    // at 64 blocks (one round of wavefronts) 16 is ahead, 40.9, 42.7 and
-    // 46.5 us, and on 7,456 blocks 5.88, 6.11 and 6.84 ms: each wavefront
-    // pays once for its first loads
+    // wavefronts per CU (two workgroups): 8 blocks take 21, 13.6 and 10.5 us
+    // with 16, 8 and 4; at 64 blocks (one round of wavefronts) 16 is ahead,
+    // 40.9, 42.7 and 46.5 us, and on 7,456 blocks 5.88, 6.11 and 6.84 ms: each
+    // wavefront pays once for its first loads
     const int64_t waves = (int64_t)c->mv.nb * 32, resident = (int64_t)c->n_cu * 8;
-    if (waves >= resident)
-      go(std::integral_constant<int, 16>());
-    else if (2 * waves >= resident)
-      go(std::integral_constant<int, 8>());
-    else
-      go(std::integral_constant<int, 4>());
+    s.ncw = waves >= resident ? 16 : 2 * waves >= resident ? 8 : 4;
+    if (s.ncw == 16) {
+      const int slots = 2 * c->n_cu, nt = c->mv.nb * 8;
+      s.extra = 4 * slots;
+      s.count = c->d_crowd;
+      s.list = c->d_crowd + 1;
+      s.crowded = (const uint8_t*)(c->d_crowd + 1 + slots);
+      hipLaunchKernelGGL(k_crowded, dim3((unsigned)((nt + 15) / 16)), dim3(256), 0, c->stream, nt,
+                         (int64_t)c->mv.nb * NCELL, slots, c->d_offset, s.count, c->d_crowd + 1,
+                         (uint8_t*)(c->d_crowd + 1 + slots));
+    }
   }
+  vf32 ? launch<BC, PAIRED, FUSED, true>(c, dt, s) : launch<BC, PAIRED, FUSED, false>(c, dt, s);
 }
 
 }  // namespace

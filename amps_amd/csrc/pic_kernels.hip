@@ -1045,7 +1045,8 @@ __global__ __launch_bounds__(256) void k_deposit_node(int64_t nnodes, int npw,
                                                        const int* __restrict__ node_order,
                                                        const int* __restrict__ inc8,
                                                        const double* __restrict__ cellpart,
-                                                       double* __restrict__ nodeout) {
+                                                       double* __restrict__ nodeout, int* clear) {
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // the cell pass's list, done with
   constexpr int STRIDE = MOMENT ? CELL_STRIDE_MOMENT : CELL_VALS;
   __shared__ __align__(16) short soff[8][256];
   static_assert(sizeof(soff) == 256 * 16, "one 16-byte row per thread");
@@ -1099,8 +1100,8 @@ __global__ __launch_bounds__(256) void k_deposit_node(int64_t nnodes, int npw,
   }
 }
 
-template __global__ void k_deposit_node<false>(int64_t, int, const int*, const int*, const double*, double*);
-template __global__ void k_deposit_node<true>(int64_t, int, const int*, const int*, const double*, double*);
+template __global__ void k_deposit_node<false>(int64_t, int, const int*, const int*, const double*, double*, int*);
+template __global__ void k_deposit_node<true>(int64_t, int, const int*, const int*, const double*, double*, int*);
 
 // Node gather for the moment record, staged.  The incidence rows come in
 // octant order (slot t: the cell on the node's side (t & 1, t >> 1 & 1,
@@ -1128,7 +1129,8 @@ __global__ __launch_bounds__(256) void k_deposit_node_staged(int64_t nnodes, int
                                                              const int* __restrict__ node_order,
                                                              const int* __restrict__ inc8,
                                                              const double* __restrict__ cellpart,
-                                                             double* __restrict__ nodeout) {
+                                                             double* __restrict__ nodeout, int* clear) {
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // the cell pass's list, done with
   __shared__ double G[4][8 * NODE_G + 1];  // the gathered values, then a zero
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;

@@ -590,6 +590,41 @@ def test_deposit_cells_per_wavefront(gpu_ctx, nblocks, precision):
         set_deposit_variant(gpu_ctx, 1, 6)
 
 
+@pytest.mark.parametrize("crowds", [1, 3, 20])
+def test_deposit_crowded_subtiles(gpu_ctx, crowds):
+    """Sub-tiles that hold more than an equal share of the particles, whose
+    layers go to workgroups of their own, beside ones that don't: J and M
+    against the oracle (the bound of test_deposit_ragged_cells), twice (the
+    list is cleared in between), and after the crowd has gone."""
+    mesh = M.central_octant_mesh()
+    E, B = M.corner_fields(mesh)
+    dt = 0.05
+    sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
+    base = M.per_cell_particles(mesh, [2, 2], [0.05, 0.005], drift=(0.01, 0.0, 0.0))
+    key = base.blk.astype(np.int64) * 512 + base.cell
+    rng = np.random.default_rng(5)
+    crowd = rng.choice(mesh.ncells, crowds, replace=False)
+    times = np.where(np.isin(key, crowd), 700, 1)
+    many = base.take(np.repeat(np.arange(base.n), times))
+    many.id = np.arange(many.n)
+    many.v *= rng.uniform(0.5, 1.5, many.n)
+    om = O.Mesh(mesh)
+    noc, keys = om.build_nodes()
+    set_deposit_variant(gpu_ctx, 2, 12)
+    try:
+        for parts in (many, many, base):
+            st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+            st.set_particles(parts)
+            for _ in range(2):
+                J, Mm = st.UpdateJMassMatrix(dt)
+            g, _ = st.get_particles()
+            Jo, Mo = O.deposit(om, B, sp, dt, g, noc, len(keys))
+            for a, b in ((J, Jo), (Mm, Mo)):
+                assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1)).all()
+    finally:
+        set_deposit_variant(gpu_ctx, 1, 6)
+
+
 def test_deposit_after_push_and_migration(gpu_ctx, dep_case):
     mesh, E, B, parts, sp, dt = dep_case
     st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
