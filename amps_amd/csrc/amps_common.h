@@ -257,6 +257,9 @@ int scan_exclusive(amps_ctx* c, int* data, int64_t n, int* total_out);
 // the stayers before each mask word; the exclusive scan of the keys' new
 // particle counts (movers in cursor, stayers from the masks of the old runs)
 int scan_masks(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw);
+bool scan_small_ok(int64_t nw, int64_t nkeys);
+void scan_small(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw, const int* cursor, const int* lay,
+                int* offset, int64_t nkeys, int tile);
 int scan_keys(amps_ctx* c, const int* cursor, const int* lay, const int* wscan, const uint64_t* wmask, int* offset,
               int64_t nkeys);
 // ECSIM cell pass with LDS record batches (deposit.hip)

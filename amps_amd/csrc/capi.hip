@@ -34,8 +34,8 @@ __global__ void k_mig_classify(const int*, const int*, const int8_t*, const int*
 __global__ void k_mig_order(int64_t, int, int, const int*, const int*, int*, int*, int*, int, const int*,
                             const int*, const uint64_t*, int*);
 __global__ void k_mig_order_slab(int64_t, int, int, const int*, const int*, const int*, int*, int*, int*,
-                                 const int*, const int*, const uint64_t*, int*);
-__global__ void k_mig_place(const int*, const int2*, const int*, const int*, const int*, int*);
+                                 const int*, const int*, const uint64_t*, int*,
+                                 unsigned, const int*, const int2*, const int*);
 __global__ void k_mig_order_big(int64_t, int, const int*, const int*, int*, int*, int*, const int*);
 __global__ void k_mig_scatter(const int*, const int*, const int8_t*, const int*, const int*, const uint64_t*,
                               const int*, int64_t, const double*, const double*, int, const uint8_t*,
@@ -696,16 +696,21 @@ static int push_tile(const amps_ctx* c) {
   return t;
 }
 
-int amps::build_tiles(amps_ctx* c) {
-  const int nb = c->mv.nb;
-  const int tile = push_tile(c);
-  const int64_t need = nb + c->cap / tile + 2;
+static int ensure_tiles(amps_ctx* c) {
+  const int64_t need = c->mv.nb + c->cap / push_tile(c) + 2;
   if (need > c->max_tiles) {
     (void)hipFree(c->d_tiles);
     c->d_tiles = nullptr;
     HIP_TRY(hipMalloc(&c->d_tiles, sizeof(Tile) * need));
     c->max_tiles = need;
   }
+  return 0;
+}
+
+int amps::build_tiles(amps_ctx* c) {
+  const int nb = c->mv.nb;
+  const int tile = push_tile(c);
+  if (int r = ensure_tiles(c)) return r;
   if (nb <= 8192) {  // one launch where one workgroup keeps up (5-12 us; three launches above)
     hipLaunchKernelGGL(k_tiles, dim3(1), dim3(1024), 0, c->stream, nb, tile, c->d_offset, c->d_tiles, c->d_ntiles);
     c->tiles_valid = true;
@@ -868,7 +873,12 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
                        c->d_code, c->d_offset);
   }
   const int64_t nw = (int64_t)gridp * 4;
-  if (classified) {
+  // small runs: both scans and the push tiles in one launch
+  const bool small = classified && scan_small_ok(nw, nkeys);
+  if (small) {
+    if (int r = ensure_tiles(c)) return r;
+    scan_small(c, c->d_wmask, c->d_wcnt, nw, c->d_cursor, c->d_off_layout, c->d_offset, nkeys, push_tile(c));
+  } else if (classified) {
     if (int r = scan_masks(c, c->d_wmask, c->d_wcnt, nw)) return r;
     if (int r = scan_keys(c, c->d_cursor, c->d_off_layout, c->d_wcnt, c->d_wmask, c->d_offset, nkeys)) return r;
   } else {
@@ -885,16 +895,15 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
                          c->d_off_layout, c->layout_valid ? 1 : 0, c->d_offset, c->d_cursor, c->d_tmpsrc, c->d_wmask);
       if (int r = scan_masks(c, c->d_wmask, c->d_wcnt, nw)) return r;
     }
-    if (classified)
-      hipLaunchKernelGGL(k_mig_place, dim3(1024), dim3(256), 0, c->stream, c->d_mig_slab + nkeys * MIG_SLAB,
-                         c->d_mig_ovf, c->d_key[a], c->d_offset, c->d_cursor, c->d_tmpsrc);
     // the movers' destinations in dest[] only for the scatter; in a deferred
     // move their source indices are the sorted lists, in place in tmpsrc
     const int write_dest = defer ? 0 : 1;
     if (classified)
-      hipLaunchKernelGGL(k_mig_order_slab, dim3(gridk), dim3(256), 0, c->stream, nkeys, c->mig_small, write_dest,
+      hipLaunchKernelGGL(k_mig_order_slab, dim3(gridk + std::min(1024u, gridp)), dim3(256), 0, c->stream, nkeys,
+                         c->mig_small, write_dest,
                          c->d_mig_slab, c->d_offset, c->d_cursor, c->d_tmpsrc, c->d_dest, c->d_big, c->d_off_layout,
-                         c->d_wcnt, c->d_wmask, c->d_kbase);
+                         c->d_wcnt, c->d_wmask, c->d_kbase, gridk, c->d_mig_slab + nkeys * MIG_SLAB, c->d_mig_ovf,
+                         c->d_key[a]);
     else
       hipLaunchKernelGGL(k_mig_order, dim3(gridk), dim3(256), 0, c->stream, nkeys, c->mig_small, write_dest,
                          c->d_offset, c->d_cursor, c->d_tmpsrc, c->d_dest, c->d_big, c->layout_valid ? 1 : 0,
@@ -926,6 +935,10 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
                      dim3(256), 0, c->stream, nkeys, c->d_offset, c->d_off_layout, c->d_n, (cap + 3) / 4,
                      (int*)c->d_code);
   c->layout_valid = true;
+  if (small) {
+    c->tiles_valid = true;
+    return 0;
+  }
   return build_tiles(c);
 }
 

@@ -427,19 +427,6 @@ __global__ __launch_bounds__(256) void k_mig_classify(const int* __restrict__ n_
   if (mover) tmpsrc[(int64_t)offset[k + 1] - 1 - (base + (__lane_id() - ru.head_lane))] = (int)p;
 }
 
-// the movers the push listed past its slab: rank r of key k's m movers at
-// offset[k + 1] - m + r of tmpsrc (the key's movers in rank order)
-__global__ __launch_bounds__(256) void k_mig_place(const int* __restrict__ novf, const int2* __restrict__ ovf,
-                                                    const int* __restrict__ key, const int* __restrict__ offset,
-                                                    const int* __restrict__ cursor, int* __restrict__ tmpsrc) {
-  const int n = *novf;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const int2 e = ovf[i];
-    const int k = key[e.x];
-    tmpsrc[(int64_t)offset[k + 1] - cursor[k] + e.y] = e.x;
-  }
-}
-
 // the destination base of key k's stayers: its new offset less the stayers
 // (of any key) before its old run (a key with an empty old run has none)
 __device__ __forceinline__ void key_base(int64_t k, const int* __restrict__ offset, const int* __restrict__ lay,
@@ -503,8 +490,10 @@ __global__ __launch_bounds__(256) void k_mig_order(int64_t nkeys, int small, int
 // The same for movers the push listed (PushMig).  Up to MIG_SLAB of them the
 // key's lane sorts in its column of LDS as it reads them from the slab
 // (rank-major: coalesced) and writes out in order; more (or more than
-// `small`) are put beside the entries k_mig_place put past the slab, and the
-// key is listed for k_mig_order_big.  Sorting in place in memory took 81 us a
+// `small`) are put beside the entries past the slab, and the
+// key is listed for k_mig_order_big.  The workgroups from kwgs on put those
+// entries in place: rank r of key k's m movers at offset[k + 1] - m + r of
+// tmpsrc.  Sorting in place in memory took 81 us a
 // step on the two-level mesh (2.0 M particles, CFL 0.2), a chain of dependent
 // accesses of the lane with the most movers.
 __global__ __launch_bounds__(256) void k_mig_order_slab(int64_t nkeys, int small, int write_dest,
@@ -514,8 +503,20 @@ __global__ __launch_bounds__(256) void k_mig_order_slab(int64_t nkeys, int small
                                                          int* __restrict__ dest, int* __restrict__ big,
                                                          const int* __restrict__ lay, const int* __restrict__ wscan,
                                                          const uint64_t* __restrict__ wmask,
-                                                         int* __restrict__ kbase) {
+                                                         int* __restrict__ kbase, unsigned kwgs,
+                                                         const int* __restrict__ novf, const int2* __restrict__ ovf,
+                                                         const int* __restrict__ key) {
   __shared__ int col[MIG_SLAB][256];
+  if (blockIdx.x >= kwgs) {
+    const int n = *novf;
+    for (int64_t i = (blockIdx.x - kwgs) * (int64_t)blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)(gridDim.x - kwgs) * blockDim.x) {
+      const int2 e = ovf[i];
+      const int k = key[e.x];
+      tmpsrc[(int64_t)offset[k + 1] - cursor[k] + e.y] = e.x;
+    }
+    return;
+  }
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (k >= nkeys) return;
   key_base(k, offset, lay, wscan, wmask, kbase);
@@ -764,31 +765,40 @@ __global__ __launch_bounds__(256) void k_mig_clear(int64_t nkeys, int* __restric
 // The push tiles in one workgroup (meshes of up to TILE_WG blocks): counts,
 // their scan and the tiles.
 constexpr int TILE_WG = 8192;
-__global__ __launch_bounds__(1024) void k_tiles(int nb, int T, const int* __restrict__ offset, Tile* tiles,
-                                                int* ntiles) {
-  __shared__ int s[16];
-  const int per = (nb + 1023) / 1024;
-  const int b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
-  int tot = 0;
-  for (int b = b0; b < b1; b++) tot += (offset[(b + 1) * NCELL] - offset[b * NCELL] + T - 1) / T;
-  int incl = tot;
+// exclusive prefix of v over the workgroup's 1,024 threads
+__device__ __forceinline__ int wg_prefix(int v, int* s) {
+  int incl = v;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     const int t = __shfl_up(incl, off);
     if (lane >= off) incl += t;
   }
+  __syncthreads();  // s may still be read from the call before
   if (lane == 63) s[w] = incl;
   __syncthreads();
-  int at = incl - tot;
+  int at = incl - v;
 #pragma unroll
   for (int q = 0; q < 16; q++)
     if (q < w) at += s[q];
+  return at;
+}
+__device__ __forceinline__ void make_tiles(int nb, int T, const int* offset, Tile* tiles, int* ntiles, int* s) {
+  const int per = (nb + 1023) / 1024;
+  const int b0 = min(nb, (int)threadIdx.x * per), b1 = min(nb, b0 + per);
+  int tot = 0;
+  for (int b = b0; b < b1; b++) tot += (offset[(b + 1) * NCELL] - offset[b * NCELL] + T - 1) / T;
+  int at = wg_prefix(tot, s);
   if (threadIdx.x == 1023) *ntiles = at + tot;
   for (int b = b0; b < b1; b++) {
     const int start = offset[b * NCELL], cnt = offset[(b + 1) * NCELL] - start;
     for (int t = 0; t < cnt; t += T) tiles[at++] = Tile{b, start + t, min(T, cnt - t), 0};
   }
+}
+__global__ __launch_bounds__(1024) void k_tiles(int nb, int T, const int* __restrict__ offset, Tile* tiles,
+                                                int* ntiles) {
+  __shared__ int s[16];
+  make_tiles(nb, T, offset, tiles, ntiles, s);
 }
 
 // tiles of at most T particles, never straddling a block
@@ -891,6 +901,34 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_tile(IN in, int* data, int6
   }
 }
 
+// A small migration's scans and push tiles in one workgroup: the mask words,
+// then the keys, eight of each a thread at most.  Launches of a few
+// microseconds each are what such a step is made of: 16.6 us in four of them.
+__global__ __launch_bounds__(1024) void k_scan_small(ScanMasks masks, int* wscan, int nwords, ScanKeys keys, int* offset,
+                                                     int nb, int T, Tile* tiles, int* ntiles) {
+  __shared__ int s[16];
+  auto scan = [&](auto in, int* data, int n) {
+    const int per = (n + 1023) / 1024, i0 = threadIdx.x * per;
+    int v[8], tot = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[i] = i < per && i0 + i < n ? in.at(i0 + i) : 0;
+      tot += v[i];
+    }
+    int run = wg_prefix(tot, s);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (i < per && i0 + i < n) data[i0 + i] = run;
+      run += v[i];
+    }
+    __threadfence_block();
+    __syncthreads();  // the workgroup's own stores are read next
+  };
+  scan(masks, wscan, nwords);
+  scan(keys, offset, (int)keys.nkeys + 1);
+  make_tiles(nb, T, offset, tiles, ntiles, s);
+}
+
 // sums: the scanned tile totals, or with raw the totals, of which every
 // workgroup sums the preceding ones itself
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add(int* data, int64_t n, const int* __restrict__ sums, int raw) {
@@ -956,6 +994,12 @@ int scan_masks(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw) {
   if (int r = scan_space(c, nw + 1)) return r;
   scan_rec(c, ScanMasks{wmask, nw}, wscan, nw + 1, c->d_scan_tmp);
   return 0;
+}
+bool scan_small_ok(int64_t nw, int64_t nkeys) { return nw < 8192 && nkeys < 8192; }
+void scan_small(amps_ctx* c, const uint64_t* wmask, int* wscan, int64_t nw, const int* cursor, const int* lay,
+                int* offset, int64_t nkeys, int tile) {
+  hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, c->stream, ScanMasks{wmask, nw}, wscan, (int)nw + 1,
+                     ScanKeys{cursor, lay, wscan, wmask, nkeys}, offset, c->mv.nb, tile, c->d_tiles, c->d_ntiles);
 }
 int scan_keys(amps_ctx* c, const int* cursor, const int* lay, const int* wscan, const uint64_t* wmask, int* offset,
               int64_t nkeys) {
