@@ -212,7 +212,10 @@ INST_PUSH64(AMPS_MOVER_LAPENTA, true, 1)
 INST_PUSH64(AMPS_MOVER_BORIS, true, 1)
 
 // FP32 push: float E/B stencil in LDS (17.5 KB), float velocities, FP64
-// positions.
+// positions.  Bound by the latency of its loads at four wavefronts per SIMD, so
+// a pass loads the next one's particles ahead: 15.3 M particles 0.66 -> 0.60 ms.
+// The FP64 push has no registers left for that: at 128 it spills (2^27
+// particles 5.4 -> 7.0 ms), and with three wavefronts it takes 5.9.
 template <int MOVER, int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f32(MeshView m, const Faces* __restrict__ faces, Species sp,
                                                    const double* __restrict__ E,
@@ -252,22 +255,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
   MigPend pd = {0, 0, 0, false};
   const int pf = pa + (int)threadIdx.x;
   int qn = (ps.src && pf >= tl.start && pf < p1) ? ps.src[pf] : 0;
+  const double* xr = ps.src ? ps.x : x;
+  const float* vr = ps.src ? (const float*)ps.v : v;
+  double nx[3] = {0, 0, 0};
+  float nv[3] = {0, 0, 0};
+  int ns = 0;
+  int64_t nid = 0;
+  auto load = [&](int p) {
+    if (p >= tl.start && p < p1) {
+      const int q = ps.src ? qn : p;
+      nx[0] = xr[q], nx[1] = xr[cap + q], nx[2] = xr[2 * cap + q];
+      nv[0] = vr[q], nv[1] = vr[cap + q], nv[2] = vr[2 * cap + q];
+      ns = ps.src ? ps.spec[q] : spec[p];
+      if (ps.src) nid = ps.id[q];
+    }
+    if (ps.src && p + (int)blockDim.x < p1) qn = ps.src[p + blockDim.x];
+  };
+  load(pf);
   for (int p0 = pa; p0 < p1; p0 += blockDim.x) {
     const int p = p0 + threadIdx.x;
     bool alive = false;
     int knew = -1;
-    const int qs = qn;
-    if (ps.src && p + (int)blockDim.x < p1) qn = ps.src[p + blockDim.x];
+    double xp[3] = {nx[0], nx[1], nx[2]};
+    float vp[3] = {nv[0], nv[1], nv[2]};
+    const int s = ns;
+    const int64_t id = nid;
+    load(p + (int)blockDim.x);
     if (p >= tl.start && p < p1) {
-    const int q = ps.src ? qs : p;
-    const double* xr = ps.src ? ps.x : x;
-    const float* vr = ps.src ? (const float*)ps.v : v;
-    double xp[3] = {xr[q], xr[cap + q], xr[2 * cap + q]};
-    float vp[3] = {vr[q], vr[cap + q], vr[2 * cap + q]};
-    const int s = ps.src ? ps.spec[q] : spec[p];
     if (ps.src) {
       ps.spec_out[p] = (uint8_t)s;
-      ps.id_out[p] = ps.id[q];
+      ps.id_out[p] = id;
     }
     int nb_out = b, cell_out = 0;
     const int c = push_particle_f32<MOVER>(m, faces, g, rc, lat, sE, sB, (float)sSp[s].q, (float)sSp[s].mass,
@@ -564,9 +581,11 @@ __device__ __forceinline__ int count_below(const int* r, int n, int t) {
 
 // the keys with many movers, one workgroup each (a grid-stride loop over the
 // list): up to RANK_SORT of them from LDS, every element's place the number of
-// smaller ones (the positions are distinct); above that a bottom-up merge sort of the distinct source positions, every
-// element placed by a binary search in the partner run, ping-ponging between
-// tmpsrc and a spare array of the same size; the sorted run ends in tmpsrc
+// smaller ones (the positions are distinct); above that a bottom-up merge sort,
+// every element placed by a binary search in the partner run, ping-ponging
+// between tmpsrc and a spare array of the same size; the sorted run ends in
+// tmpsrc.  The merge sort's passes over memory took 20 us and more for a few
+// hundred arrivals, the ranks 2 to 11 us a launch on the two-level mesh.
 constexpr int RANK_SORT = 1024;
 __global__ __launch_bounds__(256) void k_mig_order_big(int64_t nkeys, int write_dest,
                                                         const int* __restrict__ offset,
