@@ -990,6 +990,7 @@ def test_reference_effective_cutoff_islands():
     assert un and c == -1.0
 
 
+@needs_ref
 def test_reference_refine_cutoff_threshold():
     """The reference's RefineCutoffTransition through the harness: a sharp
     threshold is bracketed to max(1e-3, 1e-6 R) from the allowed side, in
