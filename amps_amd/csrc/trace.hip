@@ -1208,7 +1208,7 @@ struct TraceState {
   amps_trace_exit* d_exits = nullptr;
   size_t b_x0 = 0, b_dir = 0, b_R = 0, b_lo = 0, b_hi = 0, b_cut = 0, b_states = 0, b_out = 0, b_exits = 0;
   size_t b_pend = 0, b_status = 0, b_stop = 0, b_open = 0, b_item_steps = 0;
-  int grid_waves = 0;  // persistent grid size (workgroups); 0 = 8 per CU
+  int grid_waves = 0;  // persistent grid size (workgroups); 0 = 8 per CU, 1 or 2 for the Boris kernels
   int chunk = 32;      // steps between queue refills
 };
 
@@ -1340,7 +1340,12 @@ static void launch_fast(amps_ctx* c, TraceState* t, const typename S::View& v, c
     w.open_list = t->d_open;
     w.tickets = a.queue + 1, w.n_open = a.queue + 2, w.bracket_left = a.queue + 3;
   }
-  const int wgs = t->grid_waves > 0 ? t->grid_waves : c->n_cu * fast_wgs_per_cu(a.mode, precision, a.nloc, c->n_cu);
+  // a grid size that was set is a bound here: it is tuned on one mode and kept
+  // for all, and these kernels only lose above their own (full FP64 map, 142
+  // ms with 512 workgroups, 178 with 1,024; bracketed, 145 with 256, 309 with
+  // 1,024, in FP32 338)
+  const int own = c->n_cu * fast_wgs_per_cu(a.mode, precision, a.nloc, c->n_cu);
+  const int wgs = t->grid_waves > 0 ? std::min(t->grid_waves, own) : own;
   launch_mode<S>(c, v, w, a.mode, dim3(wgs));
   if (a.mode == TRACE_MODE_UPPER)
     hipLaunchKernelGGL(k_upper_read, dim3((unsigned)((a.nloc + 255) / 256)), dim3(256), 0, c->stream, w);

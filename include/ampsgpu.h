@@ -542,7 +542,8 @@ int amps_gpu_local_dirs(int64_t npts, const double* x0, int32_t ndir, const doub
  * lon_deg[p], lat_deg[p].  Host code. */
 int amps_gpu_local_dirs_paired(int64_t n, const double* x0, const double* lon_deg, const double* lat_deg,
                                double* dirs);
-/* Tracer tuning (autotuner): "workgroups" (persistent grid, 0 = 8 per CU),
+/* Tracer tuning (autotuner): "workgroups" (persistent grid, 0 = 8 per CU; the
+ * Boris kernels take at most their own 1 or 2 per CU),
  * "chunk" (steps between work-queue refills). */
 int amps_gpu_trace_set_param(amps_ctx* ctx, const char* name, int64_t value);
 
