@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -186,6 +187,8 @@ struct amps_ctx {
   double* d_nodeout = nullptr;
   char* h_pin = nullptr;       // pinned slots of the copies to and from the caller's arrays
   hipEvent_t pin_ev[8] = {};   // their last use
+  std::mutex pin_mutex;        // held by the copy that uses them
+  std::mutex get_mutex;        // held by amps_gpu_get_particles, which writes scratch
   double* d_pack = nullptr;    // [PACK_DOUBLES] J or M columns on their way to the host
   int* d_ecsim_nbr = nullptr;  // [nnodes][27] neighbour nodes of the ECSIM stencil, -1 outside
   // ECSIM field equation (ecsim_field.hip)

@@ -804,6 +804,7 @@ extern "C" int64_t amps_gpu_particle_count(amps_ctx* c) {
 extern "C" int amps_gpu_get_particles(amps_ctx* c, double* x, double* v, int32_t* spec,
                                       int32_t* blk, int32_t* cell, int64_t* id, int32_t* code) {
   if (!c) return fail(AMPS_E_ARG, "null context");
+  const std::lock_guard<std::mutex> lock(c->get_mutex);
   const int64_t n = amps_gpu_particle_count(c);
   if (n < 0) return fail(AMPS_E_HIP, "amps_gpu_get_particles: cannot read the particle count");
   if (n == 0) return AMPS_OK;

@@ -107,9 +107,13 @@ __global__ __launch_bounds__(256) void k_crowded(int ntiles, int64_t nkeys, int 
   for (int d = 1; d < 16; d <<= 1) n += __shfl_xor(n, d);
   if (r) return;
   const int64_t total = offset[nkeys];
-  const bool c = (int64_t)n * slots > total && (int64_t)n * ntiles > 2 * total;
+  bool c = (int64_t)n * slots > total && (int64_t)n * ntiles > 2 * total;
+  if (c) {
+    const int at = atomicAdd(count, 1);
+    c = at < slots;  // always, unless a pass before was cut off by an error
+    if (c) list[at] = t;
+  }
   crowded[t] = c;
-  if (c) list[atomicAdd(count, 1)] = t;
 }
 
 template <bool BC, bool PAIRED, bool FUSED, bool VF32>
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   int b, st, sz;
   if (!PAIRED && !BC && (int)blockIdx.x < sp4.extra) {
     // a layer of a crowded sub-tile
-    if ((int)blockIdx.x >= 4 * sp4.count[0]) return;
+    if ((int)(blockIdx.x >> 2) >= sp4.count[0]) return;
     const int tile = sp4.list[blockIdx.x >> 2];
     ncw = 4, wpl = 4, lz = 1;
     b = tile >> 3, st = tile & 7;

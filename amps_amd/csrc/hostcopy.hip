@@ -10,7 +10,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
+#include <functional>
+#include <mutex>
 #include <thread>
 
 #include "amps_common.h"
@@ -79,6 +81,7 @@ int copy(amps_ctx* c, void* dst, const void* src, size_t bytes, bool to_host) {
     if (to_host) HIP_TRY(hipStreamSynchronize(c->stream));  // a pageable source is read before the return
     return 0;
   }
+  const std::lock_guard<std::mutex> lock(c->pin_mutex);  // one call at a time on the slots
   Job j{c, (char*)dst, (const char*)src, bytes, 0, to_host};
   // at least two chunks a thread, whole pages
   j.chunk = std::min(SLOT_BYTES, ((bytes + SLOTS - 1) / SLOTS + 4095) / 4096 * 4096);
@@ -86,7 +89,7 @@ int copy(amps_ctx* c, void* dst, const void* src, size_t bytes, bool to_host) {
   for (int t = 1; t < THREADS; t++) {
     try {
       th[t - 1] = std::thread(work, std::ref(j), t);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {
       break;  // no more threads: the ones there are take all chunks
     }
   }

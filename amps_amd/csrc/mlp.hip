@@ -49,8 +49,8 @@ __device__ __forceinline__ float bf_hi(unsigned u) { return __uint_as_float(u & 
 // Phi(z) = (1 + erf(z / sqrt 2)) / 2 and E = exp(-z^2 / 2), which the
 // derivative of GELU uses too.  Below |z| = 1.25, 1/2 + z S(z^2); above,
 // the tail q = E t P(t) with t = 1 / (1 + 0.3 |z|), for z > 0 as 1 - q (the
-// form of Hastings' rational approximations to erfc).  S and P are fits of my
-// own, weighted to the least largest error in Phi and in q / E: 5e-11 and 1.6e-7
+// form of Hastings' rational approximations to erfc).  S and P were fitted
+// for this, to the least largest error in Phi and in q / E: 5e-11 and 1.6e-7
 // of q, below FP32 rounding, and the tail keeps its relative precision, which
 // 1 + erf loses: over |z| <= 12 the largest errors are 7.3e-8 in Phi and 3.8e-7
 // in GELU, where erff's were 7.5e-8 and 4.5e-7.  GELU is what bounds inference
