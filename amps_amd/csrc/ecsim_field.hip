@@ -493,7 +493,9 @@ __global__ __launch_bounds__(RED_THREADS) void k_gs_resid(int64_t n, const doubl
 }
 
 // The norm of a cycle's first residual.  what 0: of b (the first cycle), 1:
-// of a later cycle's, 2: of the final solution (into last).
+// of a later cycle's, 2: of the final solution (into last).  done only where
+// the tolerance is met (b = 0 meets it): a not-a-number never does, so the
+// steps go on and carry it into x.
 __global__ __launch_bounds__(64) void k_gs_norm(const double* __restrict__ part, int nb, int what, double tol,
                                                 GmresState* st, double* __restrict__ scale, double* __restrict__ gv) {
   const double t = sqrt(wave_total(part, nb));
@@ -505,7 +507,7 @@ __global__ __launch_bounds__(64) void k_gs_norm(const double* __restrict__ part,
   if (what == 0) st->bnorm = t, st->it = 0;
   st->res = t;
   st->k = 0;
-  st->done = !(t > tol * st->bnorm);  // also when b = 0
+  st->done = t <= tol * st->bnorm;
   scale[0] = t > 0.0 ? 1.0 / t : 0.0;
   gv[0] = t;
 }
@@ -633,7 +635,7 @@ __global__ __launch_bounds__(256) void k_gs_givens(int k, int ld, const double* 
     st->res = fabs(s * g);
     st->k = k + 1;
     st->it++;
-    if (!(st->res > tol * st->bnorm) || hn == 0.0) st->done = 1;
+    if (st->res <= tol * st->bnorm || hn == 0.0) st->done = 1;
   }
   __syncthreads();
   for (int j = threadIdx.x; j <= k; j += 256) H[(int64_t)k * ld + j] = col[j];
@@ -901,7 +903,7 @@ int gmres(amps_ctx* c, const Work& W, double fpdt, double tol, int max_iter, int
       HIP_TRY(hipMemcpyAsync(W.yv, y.data(), sizeof(double) * k, hipMemcpyHostToDevice, c->stream));
     }
     hipLaunchKernelGGL(k_update_x, grid_of(n), dim3(256), 0, c->stream, nn, k, W.yv, W.V, W.xs, W.x);
-    if (!(h.res > tol * h.bnorm) || k == 0 || it >= max_iter) break;
+    if (h.res <= tol * h.bnorm || k == 0 || it >= max_iter) break;
   }
   // the true residual of the returned solution
   launch_sym(c, op, W.xs, W.ys, nullptr);

@@ -174,3 +174,29 @@ def test_gmres_packed_operator(gpu_ctx, level, restart, max_iter, kernel):
     # a zero right-hand side
     x0, it0, rr0 = st.EcsimSolve(p, np.zeros_like(b), tol=1e-9, max_iter=5, restart=2)
     assert it0 == 0 and rr0 == 0.0 and not x0.any()
+
+
+def test_gmres_not_a_number(gpu_ctx):
+    """One not-a-number in the right-hand side, or in B, makes the whole field
+    not a number after max_iter iterations (no residual ever meets the
+    tolerance), and an infinite one ends the solve at once, since then
+    ||r|| <= tol ||b||: the stopping rule as the sequential solver has it."""
+    c = _case(gpu_ctx)
+    st = c["st"]
+    dx = c["mesh"].cell_size()[0][0]
+    p = st.ecsim_params(c["dt"], theta=0.5, cDt=2 * dx)
+    rng = np.random.default_rng(8)
+    b = rng.normal(size=(st.nnodes, 3))
+    inside = np.flatnonzero(~np.asarray(c["bnd"], bool))[5]
+    b[inside, 1] = np.nan
+    for restart in (3, 40):
+        x, it, rr = st.EcsimSolve(p, b, tol=1e-9, max_iter=11, restart=restart)
+        assert np.isnan(x).all() and it == 11 and np.isnan(rr)
+    b[inside, 1] = np.inf
+    x, it, rr = st.EcsimSolve(p, b, tol=1e-9, max_iter=11, restart=3)
+    assert not x.any() and it == 0 and np.isnan(rr)
+    En = rng.normal(size=(st.nnodes, 3))
+    Bc = rng.normal(size=(c["mesh"].nblocks * 512, 3))
+    Bc[1234, 2] = np.nan
+    E1, Eth, B1, it, rr = st.EcsimTimeStep(p, En, Bc, tol=1e-9, max_iter=11, restart=3)
+    assert np.isnan(Eth).all() and np.isnan(E1).all() and it == 11 and np.isnan(rr)
