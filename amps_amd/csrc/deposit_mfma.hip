@@ -370,7 +370,10 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
       }
       double Bv[3] = {0.0, 0.0, 0.0};
       if constexpr (BC) {
-        center_B(m, Bc, xn, b, Bv);  // centre-based B, pic_field_solver_ecsim.cpp:2097-2129
+        // centre-based B, pic_field_solver_ecsim.cpp:2097-2129; not for an empty
+        // place, which lies in the block's first cell: a not-a-number there is
+        // not this cell's
+        if (s != MAX_SPEC) center_B(m, Bc, xn, b, Bv);
       } else {
         // the corner weights sum to 1 (InitStencil's normalization changes
         // them by rounding only)

@@ -119,3 +119,40 @@ def test_deposit_center_B(gpu_ctx, exact):
         nj = np.linalg.norm(J - Jo, axis=1) / np.maximum(np.linalg.norm(Jo, axis=1), 1e-300)
         nm = np.linalg.norm(Mm - Mo, axis=1) / np.maximum(np.linalg.norm(Mo, axis=1), 1e-300)
         assert nj.max() <= 1e-12 and nm.max() <= 1e-12, (nj.max(), nm.max())
+
+
+@pytest.mark.parametrize("paired", [0, 1])
+def test_deposit_center_B_reads_only_the_particles_own_cells(gpu_ctx, paired):
+    """A not-a-number in the first cell of every block reaches the nodes of the
+    particles that interpolate it and no others: cells of five particles, so
+    that the matrix-core pass fills up their last steps of four."""
+    from amps_amd import autotune
+
+    mesh = M.uniform_mesh(1)
+    E, Bk = M.corner_fields(mesh)
+    Bc = M.center_fields(mesh, lambda P: M.dipole_field(P))
+    Bc[:, 111] = np.nan  # cell (0, 0, 0) behind one layer of ghosts
+    parts = M.per_cell_particles(mesh, [3, 2], [0.05, 0.005], drift=(0.01, 0.0, 0.0))
+    dt = 0.1 / (np.max(np.linalg.norm(Bk, axis=-1)) / 0.01)
+    sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
+    st = PicState(mesh, E, Bk, sp, ctx=gpu_ctx)
+    st.set_center_fields(Bc)
+    st.set_particles(parts)
+    autotune.set_deposit_variant(gpu_ctx, 2, 12)
+    gpu_ctx.set_param("b_center", 1)
+    gpu_ctx.set_param("deposit_paired", paired)
+    try:
+        J, Mm = st.UpdateJMassMatrix(dt)
+        g, _ = st.get_particles()
+    finally:
+        gpu_ctx.set_param("b_center", 0)
+        gpu_ctx.set_param("deposit_paired", 0)
+    om = O.Mesh(mesh)
+    om.set_center_field(Bc)
+    noc, keys = om.build_nodes()
+    Jo, Mo = O.deposit(om, Bk, sp, dt, g, noc, len(keys))
+    ok = ~np.isnan(Mo).any(axis=1)
+    assert 0.5 < ok.mean() < 1.0
+    for a, b in ((J, Jo), (Mm, Mo)):
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert (np.linalg.norm(a[ok] - b[ok], axis=1) <= 1e-12 * np.linalg.norm(b[ok], axis=1)).all()
