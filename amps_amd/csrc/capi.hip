@@ -626,6 +626,7 @@ extern "C" int amps_gpu_get_node_map(amps_ctx* c, int32_t* node_of_corner, int64
 extern "C" int amps_gpu_set_fields(amps_ctx* c, const double* E, const double* B) {
   if (!c || !E || !B) return fail(AMPS_E_ARG, "amps_gpu_set_fields: null argument");
   if (!c->has_mesh) return fail(AMPS_E_STATE, "amps_gpu_set_fields: set the mesh first");
+  (void)hipSetDevice(c->device);
   const size_t nbytes = sizeof(double) * (size_t)c->mv.nb * NCORNER * 3;
   if (!c->d_E) HIP_TRY(hipMalloc(&c->d_E, nbytes));
   if (!c->d_B) HIP_TRY(hipMalloc(&c->d_B, nbytes));
@@ -804,6 +805,7 @@ extern "C" int64_t amps_gpu_particle_count(amps_ctx* c) {
 extern "C" int amps_gpu_get_particles(amps_ctx* c, double* x, double* v, int32_t* spec,
                                       int32_t* blk, int32_t* cell, int64_t* id, int32_t* code) {
   if (!c) return fail(AMPS_E_ARG, "null context");
+  (void)hipSetDevice(c->device);
   const std::lock_guard<std::mutex> lock(c->get_mutex);
   const int64_t n = amps_gpu_particle_count(c);
   if (n < 0) return fail(AMPS_E_HIP, "amps_gpu_get_particles: cannot read the particle count");

@@ -637,6 +637,7 @@ extern "C" int amps_gpu_mlp_grad(amps_ctx* c, int64_t n, float* grad_out, float*
   MlpState* s = mstate(c);
   if (!s || s->n == 0) return fail(AMPS_E_STATE, "mlp_grad: init and set_data first");
   if (n <= 0 || n % TB || n > s->n || n > (1 << 24)) return fail(AMPS_E_ARG, "mlp_grad: n must be a positive multiple of 64 <= data size");
+  (void)hipSetDevice(c->device);
   const int nwg = (int)(n / TS);
   if (int r = ensure_gpart(c, s, nwg)) return r;
   int64_t zero = 0;

@@ -2,6 +2,7 @@
 declares, and the Python binding declares each with the header's signature
 (no compute calls: this runs without a GPU)."""
 import ctypes
+import glob
 import os
 import re
 
@@ -29,6 +30,23 @@ def test_library_exports_every_declared_symbol():
     lib = ctypes.CDLL(LIB)
     missing = [n for n in declared("ampsgpu.h") if not hasattr(lib, n)]
     assert not missing, missing
+
+
+def test_entry_points_select_their_context_s_device():
+    """An entry point that launches, allocates or hands work to the copy threads
+    selects its context's device first (prepare() of the field solver does):
+    the calling thread's may be another."""
+    seen = 0
+    for f in sorted(glob.glob(os.path.join(ROOT, "amps_amd", "csrc", "*.hip"))):
+        with open(f) as fh:
+            src = fh.read()
+        for m in re.finditer(r'extern "C" [\w *]*?(amps_gpu_\w+)\(.*?\n}\n', src, re.S):
+            work = re.search(r"hipLaunchKernelGGL|hipMalloc|hipMemsetAsync|copy_to_\w+\(|\blaunch\w*\(", m.group(0))
+            if work:
+                seen += 1
+                first = re.search(r"hipSetDevice|\bprepare\(", m.group(0))
+                assert first and first.start() < work.start(), m.group(1)
+    assert seen > 20, seen
 
 
 @pytest.mark.skipif(not os.path.exists(LIB), reason="libampsgpu.so not built")
