@@ -51,12 +51,14 @@ __device__ __forceinline__ void load_geom_rcp(const MeshView& m, const BlockGeom
   }
 }
 
-// A species' constants of the push, staged in LDS.
+// A species' constants of the push, staged in LDS: the whole table, since
+// particles may carry species of a longer one that a shorter has replaced
+// (its further entries stay as they were).
 struct SpeciesPush {
   double q, mass, dt, qdt_m, q_m;  // qdt_m = (q dt) / mass, q_m = q / mass
 };
 __device__ __forceinline__ void stage_species(const Species& sp, SpeciesPush* s) {
-  if ((int)threadIdx.x < sp.n) {
+  if (threadIdx.x < MAX_SPEC) {
     const int i = threadIdx.x;
     s[i] = {sp.charge[i], sp.mass[i], sp.dt[i], sp.charge[i] * sp.dt[i] / sp.mass[i], sp.charge[i] / sp.mass[i]};
   }

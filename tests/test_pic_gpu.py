@@ -69,10 +69,31 @@ def test_push_waves4_variant(gpu_ctx, mover):
             st.set_particles(parts, precision=L.FP32)
             st.MoveParticles(mover=mover, bc_mode=L.BC_REFLECT, r_sphere=0.2, compact=False)
             res[w] = _by_id(*st.get_particles())
-    finally:
-        gpu_ctx.set_param("push_waves", 1)
+    finally:  # the default
+        gpu_ctx.set_param("push_waves", 4)
     (a, ca), (b, cb) = res[4], res[1]
     assert np.array_equal(ca, cb) and np.array_equal(a.x, b.x) and np.array_equal(a.v, b.v)
+
+
+@pytest.mark.parametrize("mover", [L.MOVER_LAPENTA, L.MOVER_BORIS, L.MOVER_RELATIVISTIC])
+def test_push_after_a_shorter_species_table(gpu_ctx, mover):
+    """A species table of one entry set over one of three leaves the further
+    entries' constants to the particles that carry them: bit-exact with the
+    oracle under the table of three."""
+    import ctypes
+
+    mesh = M.uniform_mesh(1)
+    E, B, parts, _ = _case(mesh, 20000, 0.5, 0.05, seed=13)
+    parts.spec = (np.arange(parts.n) % 3).astype(np.int32)
+    sp = Species([-1.0, 1.0, 2.0], [0.5, 1.0, 3.0], [0.05, 0.04, 0.03])
+    st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+    st.set_particles(parts)
+    one = [L._ptr(a[:1].copy(), ctypes.c_double) for a in (sp.charge, sp.mass, sp.dt, sp.weight)]
+    L.check(st.lib.amps_gpu_set_species(gpu_ctx.h, 1, *one))
+    st.MoveParticles(mover=mover, bc_mode=L.BC_REFLECT, compact=False)
+    g, gcode = _by_id(*st.get_particles())
+    o, ocode = _by_id(*O.push(O.Mesh(mesh), E, B, sp, parts, mover=mover, bc_mode=L.BC_REFLECT, r_sphere=0.0))
+    assert np.array_equal(gcode, ocode) and np.array_equal(g.x, o.x) and np.array_equal(g.v, o.v)
 
 
 @pytest.mark.parametrize("bc", [L.BC_REFLECT, L.BC_DELETE])
