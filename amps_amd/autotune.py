@@ -13,7 +13,9 @@ import numpy as np
 
 from . import _lib as L
 
-PUSH_TILES = (1024, 2048, 4096, 8192)
+# every size that the library's own rule picks from, so that a tuned run is not
+# slower than one left to the rule
+PUSH_TILES = (256, 512, 1024, 2048, 4096, 8192)
 # register budgets of the push: 1 = the compiler's allocation, 4 = held to
 # 128 VGPRs for four wavefronts per SIMD
 PUSH_WAVES = (1, 4)

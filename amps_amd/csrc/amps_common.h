@@ -164,6 +164,7 @@ struct amps_ctx {
   int* d_ntiles = nullptr;
   int* d_tcount = nullptr;     // per-block tile count / offsets [nb+1]
   int64_t max_tiles = 0;
+  int64_t tile_wgs = 0;        // most tiles of the current size: the push's workgroups
   int tile = 8192;             // particles per push tile when given, else push_tile()'s rule
   bool tile_given = false;
   bool offsets_valid = false;  // d_offset describes the current order

@@ -699,6 +699,7 @@ static int push_tile(const amps_ctx* c) {
 
 static int ensure_tiles(amps_ctx* c) {
   const int64_t need = c->mv.nb + c->cap / push_tile(c) + 2;
+  c->tile_wgs = need;
   if (need > c->max_tiles) {
     (void)hipFree(c->d_tiles);
     c->d_tiles = nullptr;
@@ -994,7 +995,7 @@ static int launch_push(amps_ctx* c, const amps_push_opts* o, int* count = nullpt
     c->pending_gather = false;
   }
 #define LAUNCH_PUSH32(MV, W)                                                                              \
-  hipLaunchKernelGGL((k_push_f32<MV, W>), dim3((unsigned)c->max_tiles), dim3(256), 0, c->stream, c->mv,     \
+  hipLaunchKernelGGL((k_push_f32<MV, W>), dim3((unsigned)c->tile_wgs), dim3(256), 0, c->stream, c->mv,     \
                      c->d_faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
                      c->d_x[k], (float*)c->d_v[k], c->d_spec[k], c->d_key[k], c->d_code, count, ps, pm)
   if (c->precision == AMPS_FP32) {
@@ -1010,7 +1011,7 @@ static int launch_push(amps_ctx* c, const amps_push_opts* o, int* count = nullpt
   }
 #undef LAUNCH_PUSH32
 #define LAUNCH_PUSH64(MV, BCV, W)                                                                       \
-  hipLaunchKernelGGL((k_push_f64<MV, BCV, W>), dim3((unsigned)c->max_tiles), dim3(256), 0, c->stream, c->mv,  \
+  hipLaunchKernelGGL((k_push_f64<MV, BCV, W>), dim3((unsigned)c->tile_wgs), dim3(256), 0, c->stream, c->mv,  \
                      c->d_faces, c->sp, c->d_E, c->d_B, c->d_tiles, c->d_ntiles, o->bc_mode, o->r_sphere, c->cap, \
                      c->d_x[k], c->d_v[k], c->d_spec[k], c->d_key[k], c->d_code, c->d_Bc, count, ps, pm)
   const bool bc = c->b_center != 0;

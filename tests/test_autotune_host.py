@@ -5,6 +5,8 @@ variant (a pass that cannot read a step's particles through the migration's
 source indices wins only if whole steps are faster with it), the node batch,
 the report fields and the cache."""
 import json
+import os
+import re
 
 import numpy as np
 import pytest
@@ -12,7 +14,7 @@ import pytest
 from amps_amd import _lib as L
 from amps_amd import autotune as A
 
-PUSH = {1024: 5.0, 2048: 4.5, 4096: 4.0, 8192: 4.2}
+PUSH = {256: 7.0, 512: 6.0, 1024: 5.0, 2048: 4.5, 4096: 4.0, 8192: 4.2}
 NODE = {4: 4.4, 8: 4.1, 16: 4.0}
 COMPACT = 0.45       # a step's migration that leaves the records for the next push
 SCATTER = 2.3        # the record scatter of a step whose cell pass cannot read through the indices
@@ -85,6 +87,7 @@ def _deposit_times(best=None):
 def _tune(tmp_path, deposit):
     ctx = FakeCtx()
     st = FakeState(ctx, deposit)
+    tmp_path.mkdir(exist_ok=True)
     cache = str(tmp_path / "tune.json")
     best, cached = A.tune_pic(ctx, st, {}, 0.1, "sig", cache=cache)
     return ctx, st, cache, best, cached
@@ -101,6 +104,20 @@ def test_fusable_deposit_winner_needs_no_step_comparison(tmp_path):
     assert best["push_ms"] == {str(t): PUSH[t] for t in A.PUSH_TILES}
     assert ctx.p["tile"] == 4096 and ctx.p["push_waves"] == 4 and ctx.p["node_batch"] == 16
     assert (ctx.p["deposit_kernel"], ctx.p["deposit_chunks"]) == (3, 8) and not ctx.on
+
+
+def test_tiles_of_the_library_s_rule_are_tried(tmp_path, monkeypatch):
+    """The library's rule goes down to small tiles for small runs: where one of
+    them is the fastest, the tuner takes it."""
+    with open(os.path.join(os.path.dirname(__file__), "..", "include", "ampsgpu.h")) as f:
+        lo, hi = re.search(r"power of two from (\d+) to (\d+)", f.read()).groups()
+    assert A.PUSH_TILES[0] == int(lo) and A.PUSH_TILES[-1] == int(hi)
+    assert all(b == 2 * a for a, b in zip(A.PUSH_TILES, A.PUSH_TILES[1:]))
+    for fastest in (256, 512):
+        monkeypatch.setitem(PUSH, fastest, 0.5)
+        ctx, _, _, best, _ = _tune(tmp_path / str(fastest), _deposit_times())
+        assert best["tile"] == fastest == ctx.p["tile"]
+        monkeypatch.undo()
 
 
 @pytest.mark.parametrize("margin,winner", [(1.0, (2, 4)), (3.0, (1, 4))])
