@@ -145,9 +145,12 @@ def tune_pic(ctx, state, opts_kw, deposit_dt, signature, cache=None, reps=2):
     return best, False
 
 
-def tune_tracer(ctx, run, n_cu, signature, cache=None):
+def tune_tracer(ctx, run, n_cu, signature, cache=None, grids=None):
     """Pick the persistent grid size and refill chunk for the tracer; run()
-    executes one representative tracing call."""
+    executes one representative tracing call.  grids: the grid sizes tried, by
+    default 2, 3, 4 and 8 workgroups per CU, which differ for the general
+    kernel only.  The Boris kernels take at most their own 1 or 2 per CU:
+    for those (0,), the library's choice, leaves the chunk alone to try."""
     from . import cutoff as CU
 
     db = _load(cache)
@@ -157,7 +160,7 @@ def tune_tracer(ctx, run, n_cu, signature, cache=None):
         CU.set_trace_param(ctx, "chunk", best["chunk"])
         return best, True
     res = {}
-    for wg in (2 * n_cu, 3 * n_cu, 4 * n_cu, 8 * n_cu):
+    for wg in grids or (2 * n_cu, 3 * n_cu, 4 * n_cu, 8 * n_cu):
         for ch in (16, 64):
             CU.set_trace_param(ctx, "workgroups", wg)
             CU.set_trace_param(ctx, "chunk", ch)

@@ -369,7 +369,8 @@ def cutoff_map_bench(ctx, n_cu, n_train=1 << 20, epochs=20, cpu_check_points=16,
     def run_sub():
         CU.cutoff_scan(ctx, P, x0[sub], dirs[sub], grid, mode=CU.SCAN_FULL, precision=L.FP32)
 
-    tune, cached = autotune.tune_tracer(ctx, run_sub, n_cu, f"trace|{n_cu}", cache=tune_cache)
+    # every scan here runs the Boris kernels, whose grid is their own
+    tune, cached = autotune.tune_tracer(ctx, run_sub, n_cu, f"trace|{n_cu}|boris", cache=tune_cache, grids=(0,))
     out["tracer_tune"] = {"workgroups": tune["workgroups"], "chunk": tune["chunk"], "cached": cached}
     # FP64 map (bit-exact with the CPU oracle): the reference map of this run
     t0 = time.perf_counter()

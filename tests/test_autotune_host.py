@@ -149,3 +149,29 @@ def test_cache_applies_the_stored_choice(tmp_path):
     assert ctx.p == {"tile": best["tile"], "push_waves": best["push_waves"],
                      "deposit_kernel": best["deposit_kernel"], "deposit_chunks": best["deposit_chunks"],
                      "node_batch": best["node_batch"]}
+
+
+@pytest.mark.parametrize("grids", [None, (0,)])
+def test_tracer_sweep(tmp_path, monkeypatch, grids):
+    """The tracer's sweep: the general kernel's four grids by two chunks, or the
+    chunks alone where the grid is the kernel's own; the fastest is set and
+    comes back from the cache."""
+    from amps_amd import cutoff as CU
+
+    cur, runs, clock = {}, [], [0.0]
+    monkeypatch.setattr(CU, "set_trace_param", lambda ctx, name, v: cur.__setitem__(name, v))
+    monkeypatch.setattr(A.time, "perf_counter", lambda: clock[0])
+
+    def run():
+        runs.append((cur["workgroups"], cur["chunk"]))
+        clock[0] += 2.0 - (cur["chunk"] == 64) - 0.5 * (cur["workgroups"] == 3 * 256)
+
+    cache = str(tmp_path / "t.json")
+    best, cached = A.tune_tracer(None, run, 256, "sig", cache=cache, grids=grids)
+    want = {(g, c) for g in (grids or (512, 768, 1024, 2048)) for c in (16, 64)}
+    assert len(runs) == len(want) and set(runs) == want and not cached
+    assert (best["workgroups"], best["chunk"]) == ((768, 64) if grids is None else (0, 64))
+    assert cur == {"workgroups": best["workgroups"], "chunk": 64}
+    cur.clear()
+    again, cached = A.tune_tracer(None, run, 256, "sig", cache=cache, grids=grids)
+    assert cached and again == best and cur == {"workgroups": best["workgroups"], "chunk": 64}
