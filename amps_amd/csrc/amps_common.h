@@ -189,7 +189,8 @@ struct amps_ctx {
   char* h_pin = nullptr;       // pinned slots of the copies to and from the caller's arrays
   hipEvent_t pin_ev[8] = {};   // their last use
   std::mutex pin_mutex;        // held by the copy that uses them
-  std::mutex get_mutex;        // held by amps_gpu_get_particles, which writes scratch
+  std::mutex read_mutex;       // held by the calls that hand particles, cell counts, J or M to the host: they
+                               // write scratch (d_pack, d_cursor, the idle particle buffer), which two readers share
   double* d_pack = nullptr;    // [PACK_DOUBLES] J or M columns on their way to the host
   int* d_ecsim_nbr = nullptr;  // [nnodes][27] neighbour nodes of the ECSIM stencil, -1 outside
   // ECSIM field equation (ecsim_field.hip)

@@ -807,7 +807,7 @@ extern "C" int amps_gpu_get_particles(amps_ctx* c, double* x, double* v, int32_t
                                       int32_t* blk, int32_t* cell, int64_t* id, int32_t* code) {
   if (!c) return fail(AMPS_E_ARG, "null context");
   (void)hipSetDevice(c->device);
-  const std::lock_guard<std::mutex> lock(c->get_mutex);
+  const std::lock_guard<std::mutex> lock(c->read_mutex);
   const int64_t n = amps_gpu_particle_count(c);
   if (n < 0) return fail(AMPS_E_HIP, "amps_gpu_get_particles: cannot read the particle count");
   if (n == 0) return AMPS_OK;
@@ -1171,6 +1171,7 @@ extern "C" int amps_gpu_update_j_mass_matrix(amps_ctx* c, double dt, double* J_o
   if (c->b_center && (!c->has_center || c->dep_kernel == 0))
     return fail(AMPS_E_STATE, "amps_gpu_update_j_mass_matrix: b_center needs the cell-centred B and deposit_kernel 1 or 2");
   (void)hipSetDevice(c->device);
+  const std::lock_guard<std::mutex> lock(c->read_mutex);
   if (int r = ensure_deposit_buffers(c)) return r;
   if (c->cap == 0) {
     HIP_TRY(hipMemsetAsync(c->d_nodeout, 0, sizeof(double) * (size_t)c->nnodes * NODE_STRIDE, c->stream));

@@ -165,6 +165,7 @@ extern "C" int amps_gpu_get_particles_restart(amps_ctx* c, const amps_aos_layout
   if (int r = check_layout(layout, L, aligned)) return r;
   if (!c->has_mesh) return fail(AMPS_E_STATE, "amps_gpu_get_particles_restart: no mesh");
   (void)hipSetDevice(c->device);
+  const std::lock_guard<std::mutex> lock(c->read_mutex);
   if (c->cap > 0 && !c->offsets_valid)
     if (int r = amps_gpu_compact(c)) return r;
   const int64_t n = c->cap > 0 ? amps_gpu_particle_count(c) : 0;

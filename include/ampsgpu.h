@@ -5,7 +5,9 @@
  * pointers and sizes.  Every function returns 0 on success and a nonzero
  * AMPS_E_* status otherwise; amps_gpu_last_error() returns the message of
  * the last failure on the calling thread.  One context per device; a context
- * is not re-entrant (calls on one context must not overlap).
+ * is not re-entrant (calls on one context must not overlap, but for those
+ * that hand particles, restart records, J or M to the host among themselves,
+ * which take turns).
  *
  * Each entry point names the reference interface it replaces.
  */

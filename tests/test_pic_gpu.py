@@ -841,6 +841,44 @@ def test_push_fp32_error_against_fp64_oracle(gpu_ctx, mover):
 
 
 @pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+def test_two_threads_read_one_context(gpu_ctx, precision):
+    """Particles, J and M, and restart records read by two threads at a time:
+    these calls share scratch on the device, and each gives what it gives
+    alone."""
+    import threading
+
+    mesh = M.uniform_mesh(2)
+    E, B = M.corner_fields(mesh)
+    dt = 0.05
+    st = PicState(mesh, E, B, Species([-1.0, 1.0], [0.01, 1.0], [dt, dt]), ctx=gpu_ctx)
+    st.generate_particles(mesh.ncells * 4, [0.1, 0.05], seed=6, precision=precision)
+
+    def particles():
+        g, code = st.get_particles()
+        return g.id, g.x, g.v, g.spec, g.blk, g.cell, code
+
+    reads = (particles, lambda: st.UpdateJMassMatrix(dt), lambda: st.get_restart(L.aos_layout_aligned()))
+    want = [r() for r in reads]
+    got, failed = {}, []
+
+    def run(t, r):
+        try:
+            for i in range(4):
+                got[t, i] = r, reads[r]()
+        except Exception as e:
+            failed.append(e)
+
+    for a in range(3):
+        for b in range(3):
+            ts = [threading.Thread(target=run, args=(t, r)) for t, r in enumerate((a, b))]
+            [t.start() for t in ts]
+            [t.join() for t in ts]
+            assert not failed, failed
+            for r, out in got.values():
+                assert all(np.array_equal(x, y) for x, y in zip(out, want[r])), (a, b, r)
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
 @pytest.mark.parametrize("n", [1, 131071, 131073, 600001])
 def test_particles_to_the_host(gpu_ctx, n, precision):
     """Columns on both sides of the size from which a copy goes through the
