@@ -96,7 +96,10 @@ int copy(amps_ctx* c, void* dst, const void* src, size_t bytes, bool to_host) {
   work(j, 0);
   for (auto& t : th)
     if (t.joinable()) t.join();
-  HIP_TRY((hipError_t)j.err.load());
+  const hipError_t e = (hipError_t)j.err.load();
+  // a copy whose event could not be recorded or waited for may still run
+  if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);
+  HIP_TRY(e);
   return 0;
 }
 }  // namespace
