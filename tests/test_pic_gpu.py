@@ -328,8 +328,75 @@ def test_migration_arrival_counts_at_the_sort_limits(tile, precision):
     assert b.n == n - ngone and per_key.max() > 1024 and (per_key > 16).sum() >= 10
 
 
+def _compacted_both_ways(ctx, mesh, E, B, sp, p, precision):
+    """The push with the compaction in the same call (it classifies) against
+    the push and a separate compaction, and both against the layout that the
+    arrays determine: each cell's stayers in their order, then its arrivals in
+    theirs.  Then a second push of the compacted arrays against the oracle."""
+    st = PicState(mesh, E, B, sp, ctx=ctx)
+    push = dict(mover=L.MOVER_BORIS, bc_mode=L.BC_DELETE)
+    st.set_particles(p, precision=precision)
+    st.MoveParticles(compact=False, **push)
+    st.compact()
+    c, _ = st.get_particles()
+    st.set_particles(p, precision=precision)
+    a, _ = st.get_particles()
+    st.MoveParticles(compact=True, **push)
+    b, _ = st.get_particles()
+    for k in ("id", "x", "v", "blk", "cell", "spec"):
+        assert np.array_equal(getattr(b, k), getattr(c, k)), k
+    pos = np.full(p.n, -1)
+    pos[a.id] = np.arange(a.n)
+    old = pos[b.id]
+    ka = a.blk.astype(np.int64) * 512 + a.cell
+    kb = b.blk.astype(np.int64) * 512 + b.cell
+    assert np.array_equal(np.lexsort((old, kb != ka[old], kb)), np.arange(b.n))
+    assert 0 < (kb != ka[old]).sum() < b.n < p.n
+    if precision == L.FP64:
+        st.MoveParticles(compact=True, **push)
+        g, _ = _by_id(*st.get_particles())
+        o, code = O.push(O.Mesh(mesh), E, B, sp, b, mover=L.MOVER_BORIS, bc_mode=L.BC_DELETE, r_sphere=0.0)
+        o, _ = _by_id(o.take(np.flatnonzero(code == L.CODE_FINISHED)), None)
+        for k in ("id", "x", "v", "blk", "cell"):
+            assert np.array_equal(getattr(g, k), getattr(o, k)), k
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("refined,n", [(1, 2047 * 256), (1, 2047 * 256 + 1), (2, 5000), (1, 300)])
+def test_compaction_at_the_one_launch_limits(refined, n, precision):
+    """15 blocks are 7,680 keys and 2,047 x 256 particles 8,188 mask words, the
+    most that the one-workgroup scan takes (eight entries a thread); one
+    particle or seven blocks more go the other way."""
+    mesh = M.uniform_mesh(1)
+    lv, ijk = M.refine(mesh.level, mesh.ijk, lambda lev, i, j, k: j == 0 and k == 0 and i < refined)
+    mesh = M.BlockMesh(lv, ijk, lmax=mesh.lmax)
+    assert mesh.nblocks == 8 + 7 * refined
+    E, B, parts, sp = _case(mesh, n, 1.5, 0.05, seed=3)
+    assert parts.n == n
+    with L.Context(0) as ctx:
+        _compacted_both_ways(ctx, mesh, E, B, sp, parts, precision)
+
+
+@pytest.mark.parametrize("tile", [None, 8192])
+def test_compaction_above_8192_blocks(tile):
+    """8,296 blocks (4.2 M keys): the push tiles from three launches in place
+    of one workgroup, and scans of more tile totals than every workgroup sums
+    for itself, for a plain compaction and for a classified one."""
+    mesh = M.uniform_mesh(4)
+    left = iter(range(600))
+    lv, ijk = M.refine(mesh.level, mesh.ijk, lambda lev, i, j, k: next(left, None) is not None)
+    mesh = M.BlockMesh(lv, ijk, lmax=mesh.lmax)
+    assert mesh.nblocks > 8192 and mesh.ncells > 2048 * 2048
+    E, B, parts, sp = _case(mesh, 100000, 0.2, 0.05, seed=9)
+    with L.Context(0) as ctx:
+        if tile:
+            ctx.set_param("tile", tile)
+        _compacted_both_ways(ctx, mesh, E, B, sp, parts, L.FP64)
+
+
+@pytest.mark.parametrize("waves,precision", [(4, L.FP64), (1, L.FP64), (4, L.FP32), (1, L.FP32)])
 @pytest.mark.parametrize("small,kernel", [(64, 2), (1, 2), (64, 1)])
-def test_step_migration_order_with_crowded_arrivals(gpu_ctx, small, kernel):
+def test_step_migration_order_with_crowded_arrivals(gpu_ctx, small, kernel, waves, precision):
     """The same layout from the step's own migration, whose push classifies
     the survivors and lists each cell's arrivals (16 per cell, the rest in
     an overflow list): about 200 particles per cell and fast ones, so that
@@ -345,8 +412,9 @@ def test_step_migration_order_with_crowded_arrivals(gpu_ctx, small, kernel):
     dt = 0.05
     sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
     st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
-    st.generate_particles(mesh.ncells * 100, [0.8, 0.8], seed=11)
+    st.generate_particles(mesh.ncells * 100, [0.8, 0.8], seed=11, precision=precision)
     gpu_ctx.set_param("migration_sort_small", small)
+    gpu_ctx.set_param("push_waves", waves)
     autotune.set_deposit_variant(gpu_ctx, kernel, 4)
     try:
         st.run_steps(1, dt, r_sphere=0.2, use_graph=False)
@@ -372,6 +440,7 @@ def test_step_migration_order_with_crowded_arrivals(gpu_ctx, small, kernel):
         print(f"cells with > 16 arrivals: {over16}, > 64: {over64}", flush=True)
         assert over16 > 100 and over64 > 0
     finally:  # the session context's defaults
+        gpu_ctx.set_param("push_waves", 4)
         gpu_ctx.set_param("migration_sort_small", 64)
         autotune.set_deposit_variant(gpu_ctx, 2, 12)
 
@@ -447,7 +516,7 @@ def test_deposit_parity(gpu_ctx, dep_case, exact, kernel, nch):
         nm = np.linalg.norm(Mm - Mo, axis=1) / np.maximum(np.linalg.norm(Mo, axis=1), 1e-300)
         assert nj.max() <= 1e-12 and nm.max() <= 1e-12, (nj.max(), nm.max())
     gpu_ctx.set_param("deposit_exact", 0)
-    set_deposit_variant(gpu_ctx, 1, 6)
+    set_deposit_variant(gpu_ctx, 2, 12)
 
 
 @pytest.mark.parametrize("kernel,nch", [(3, 8), (2, 12), (1, 6)])
@@ -464,7 +533,7 @@ def test_deposit_fp32_mode_error(gpu_ctx, dep_case, kernel, nch):
     try:
         J, Mm = st.UpdateJMassMatrix(dt)
     finally:
-        set_deposit_variant(gpu_ctx, 1, 6)
+        set_deposit_variant(gpu_ctx, 2, 12)
     g, _ = st.get_particles()  # device order, velocities widened from FP32
     om = O.Mesh(mesh)
     noc, keys = om.build_nodes()
@@ -507,6 +576,33 @@ def test_particle_energy_cfl_bitexact(gpu_ctx, dep_case, precision):
     print(f"energy {e!r} vs {eo!r}, cfl {cfl} vs {cflo}", flush=True)
     assert e == eo and np.array_equal(cfl, cflo)
     assert e > 0 and np.all(cfl > 0)
+
+
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("nspec", [1, 3, 8])
+def test_particle_energy_cfl_species_and_windows(gpu_ctx, nspec, precision):
+    """Up to two species and up to eight are two instantiations; a cell of
+    1,300 particles spans three windows of 512, among empty cells and cells of
+    a few: bit-exact with the oracle."""
+    mesh = M.uniform_mesh(1)
+    E, B = M.corner_fields(mesh)
+    parts = M.uniform_particles(mesh, 9000, 0.1)
+    key = parts.blk.astype(np.int64) * 512 + parts.cell
+    k, cnt = np.unique(key, return_counts=True)
+    assert len(k) < mesh.ncells  # some are empty
+    at = np.flatnonzero(key == k[np.argmax(cnt)])
+    parts = parts.take(np.concatenate([np.arange(parts.n), np.resize(at, 1300 - len(at))]))
+    rng = np.random.default_rng(nspec)
+    parts.v *= rng.uniform(0.5, 1.5, parts.n)
+    parts.id = np.arange(parts.n)
+    parts.spec = rng.integers(0, nspec, parts.n).astype(np.int32)
+    sp = Species(np.ones(nspec), 1.0 + np.arange(nspec), np.full(nspec, 0.01), 1.0 / (2.0 + np.arange(nspec)))
+    st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+    st.set_particles(parts, precision=precision)
+    e, cfl = st.ParticleEnergyCfl(0.02)
+    g, _ = st.get_particles()
+    eo, cflo, _, _ = O.energy_cfl(O.Mesh(mesh), sp, 0.02, g)
+    assert e == eo > 0 and np.array_equal(cfl, cflo) and np.all(cfl > 0)
 
 
 def test_node_gather_staged_matches_direct(gpu_ctx, dep_case):
@@ -553,7 +649,7 @@ def test_deposit_ragged_cells(gpu_ctx, kernel, paired, nch):
     try:
         J, Mm = st.UpdateJMassMatrix(dt)
     finally:
-        set_deposit_variant(gpu_ctx, 1, 6)
+        set_deposit_variant(gpu_ctx, 2, 12)
         gpu_ctx.set_param("deposit_paired", 0)
     g, _ = st.get_particles()
     om = O.Mesh(mesh)
@@ -608,7 +704,7 @@ def test_deposit_cells_per_wavefront(gpu_ctx, nblocks, precision):
             st.UpdateJMassMatrix(dt, copy_out=False)
             assert np.abs(fused).max() > 0 and np.array_equal(fused, st.MassMatrixApply(probe, 1.0))
     finally:
-        set_deposit_variant(gpu_ctx, 1, 6)
+        set_deposit_variant(gpu_ctx, 2, 12)
 
 
 @pytest.mark.parametrize("crowds", [1, 3, 20])
@@ -643,7 +739,7 @@ def test_deposit_crowded_subtiles(gpu_ctx, crowds):
             for a, b in ((J, Jo), (Mm, Mo)):
                 assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1)).all()
     finally:
-        set_deposit_variant(gpu_ctx, 1, 6)
+        set_deposit_variant(gpu_ctx, 2, 12)
 
 
 def test_deposit_after_push_and_migration(gpu_ctx, dep_case):
@@ -1012,22 +1108,24 @@ def test_ecsim_mass_apply_single_particle_closed_form(gpu_ctx):
     assert np.count_nonzero(np.abs(out).sum(1)) == 8
 
 
-def test_autotuner_weighs_whole_steps(gpu_ctx, monkeypatch):
+def test_autotuner_weighs_whole_steps(monkeypatch):
     """The tuner picks the deposit pass by the deposit's time, but a pass
     other than the matrix-core and lane ones (which read a step's particles
     where the migration left them) wins only if whole steps are faster with
     it too; the chosen configuration then runs steps."""
     from amps_amd import autotune
 
+    ctx = L.Context(0)  # its own: a tile once given stays
+
     mesh = M.central_octant_mesh()
     E, B = M.corner_fields(mesh)
     sp = Species([-1.0, 1.0], [0.01, 1.0], [0.05, 0.05])
-    st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+    st = PicState(mesh, E, B, sp, ctx=ctx)
     st.generate_particles(mesh.ncells * 8, [0.3, 0.3], seed=3)
     monkeypatch.setattr(autotune, "DEPOSIT_VARIANTS", ((1, 4), (2, 4)))
     opts = dict(mover=L.MOVER_LAPENTA, bc_mode=L.BC_REFLECT, r_sphere=0.2)
     try:
-        best, cached = autotune.tune_pic(gpu_ctx, st, opts, 0.05, "test", cache=None)
+        best, cached = autotune.tune_pic(ctx, st, opts, 0.05, "test", cache=None)
         print(f"tuned: {best}", flush=True)
         assert not cached and best["deposit_kernel"] in (1, 2)
         dep = best["deposit_ms"]
@@ -1041,13 +1139,9 @@ def test_autotuner_weighs_whole_steps(gpu_ctx, monkeypatch):
         st.run_steps(3, 0.05, **opts)
         assert 0 < st.particle_count() <= n0
         # the whole-step comparison itself
-        var, steps = autotune.weigh_steps(gpu_ctx, st, opts, 0.05, ((1, 4), (2, 4)))
+        var, steps = autotune.weigh_steps(ctx, st, opts, 0.05, ((1, 4), (2, 4)))
         print(f"steps: {steps}", flush=True)
         assert set(steps) == {(1, 4), (2, 4)} and all(t > 0 for t in steps.values())
         assert var == min(steps, key=steps.get)
-    finally:  # the session context's defaults
-        autotune.set_deposit_variant(gpu_ctx, 2, 12)
-        gpu_ctx.set_param("tile", 8192)
-        gpu_ctx.set_param("push_waves", 1)
-        gpu_ctx.set_param("node_batch", 8)
-        gpu_ctx.set_timing(False)
+    finally:
+        ctx.close()

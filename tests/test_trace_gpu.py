@@ -510,16 +510,17 @@ def _edge_tasks():
     dict(moment_scale=0.0, max_time=0.5), dict(moment_scale=1e-30, max_time=0.5, dist_limiter=False),
     dict(max_time=1e-3, dt_floor=False), dict(max_steps=3, retry=2), dict(dt_trace=1e-6, max_steps=50),
     dict(r_inner_Re=0.0), dict(adaptive=False), dict(mass_amu=1e-60), dict(charge_e=26, mass_amu=56.0)])
-def test_boris_kernels_agree(gpu_ctx, kw):
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+def test_boris_kernels_agree(gpu_ctx, kw, precision):
     """The lean Boris kernel (trace_batch) against the general one, which
     trace_batch_ex runs, over its options and at the edges of its ranges: the
     same bits in every field."""
     kw = dict(dict(max_steps=2000, max_time=60.0), **kw)
     P = CU.legacy_params(**kw)
     x, d, R = _edge_tasks()
-    print(f"trace options {kw} n={len(R)}", flush=True)
-    a, sa = CU.trace_batch(gpu_ctx, P, x, d, R)
-    b, _, sb = CU.trace_batch_ex(gpu_ctx, P, x, d, R)
+    print(f"trace options {kw} precision {precision} n={len(R)}", flush=True)
+    a, sa = CU.trace_batch(gpu_ctx, P, x, d, R, precision=precision)
+    b, _, sb = CU.trace_batch_ex(gpu_ctx, P, x, d, R, precision=precision)
     for f in a.dtype.names:
         assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype.kind == "f"), f
     assert sa == sb
