@@ -138,6 +138,20 @@ def test_other_deposit_winner_must_win_whole_steps(tmp_path, margin, winner):
     assert steps["k2c4"] == pytest.approx(push + RECORD_MOVE + COMPACT + 5.0 + margin + NODE[8])
 
 
+@pytest.mark.parametrize("in_steps", [1, 4])
+def test_register_budget_is_weighed_in_steps(tmp_path, monkeypatch, in_steps):
+    """The push of a step and that of MoveParticles may favour different
+    register budgets: the tuner goes by the step's."""
+    def push(self, move=False):
+        better = in_steps if move else 5 - in_steps
+        self.ctx.add(L.K_PUSH, PUSH[self.ctx.p["tile"]] - (0.1 if self.ctx.p["push_waves"] == better else 0.0))
+
+    monkeypatch.setattr(FakeState, "_push", push)
+    ctx, _, _, best, _ = _tune(tmp_path, _deposit_times())
+    assert best["push_waves"] == in_steps == ctx.p["push_waves"]
+    assert best["push_waves_ms"][str(in_steps)] < best["push_waves_ms"][str(5 - in_steps)]
+
+
 def test_cache_applies_the_stored_choice(tmp_path):
     dep = _deposit_times({(1, 4): 5.0, (2, 4): 6.0})
     _, _, cache, best, _ = _tune(tmp_path, dep)
