@@ -26,6 +26,7 @@ constexpr int NODE_VALS = 3 + 243;     // per-node J + mass-matrix row block
 constexpr int CELL_STRIDE_MOMENT = 272;  // 17 lines
 constexpr int NODE_STRIDE = 256;         // 16 lines
 constexpr int MAX_SPEC = 8;
+constexpr int TILE_WG = 8192;  // blocks up to which one workgroup makes the push tiles
 constexpr int64_t PACK_DOUBLES = (int64_t)1 << 23;  // staging of packed J and M columns (64 MiB)
 
 // Device view of the block mesh (leaf blocks of the AMR octree).
@@ -177,7 +178,7 @@ struct amps_ctx {
   int mig_small = 64;          // movers per key sorted by one lane (more: a workgroup merge sort)
   int dep_waves = 2;           // eight-lanes-per-cell pass: register budget in wavefronts per SIMD (2 or 3)
   int dep_paired = 0;          // matrix-core cell pass: two wavefronts per SIMD in opposite phases
-  int push_waves = 4;          // 4: push kernels built for 4 waves per SIMD (128 VGPRs); 1: unbounded
+  int push_waves = 4;          // 4: push kernels built for 4 waves per SIMD (128 VGPRs); 1: unbounded (k_push_f64)
   int dep_exact = 0;           // 1: unfused mul+add in the deposit (bit-exact order)
   int dep_kernel = 2;          // cell pass: 0 per-lane particle loop, 1 LDS record batches, 2 matrix cores,
                                // 3 eight lanes per cell

@@ -713,7 +713,7 @@ int amps::build_tiles(amps_ctx* c) {
   const int nb = c->mv.nb;
   const int tile = push_tile(c);
   if (int r = ensure_tiles(c)) return r;
-  if (nb <= 8192) {  // one launch where one workgroup keeps up (5-12 us; three launches above)
+  if (nb <= TILE_WG) {  // one launch where one workgroup keeps up (5-12 us; three launches above)
     hipLaunchKernelGGL(k_tiles, dim3(1), dim3(1024), 0, c->stream, nb, tile, c->d_offset, c->d_tiles, c->d_ntiles);
     c->tiles_valid = true;
     return AMPS_OK;

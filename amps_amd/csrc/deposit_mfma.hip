@@ -26,15 +26,17 @@
 // particles of the next two chunks, and the source indices of the one after,
 // are loaded while the current one is accumulated.
 //
-// What bounds it: the issue slots of a SIMD's two wavefronts (80 KB of LDS a
-// workgroup).  With counters (15.3 M particles, before): MFMA 38 % and other
-// vector instructions 31 % of the cycles, LDS 47 % busy.  So the inner loop is
+// What bounds it: what a wavefront issues, record by record and product by
+// product, with two of them to a SIMD (80 KB of LDS a workgroup) that overlap
+// in part: with counters (15.3 M particles, before) MFMA 38 % and other
+// vector instructions 31 % of the cycles, LDS 47 % busy, no unit saturated.
+// Fewer instructions a wavefront pay: the inner loop is
 // kept to the products and five address increments per four steps, with two
 // steps to an LDS read; 2^27 particles on 7,456 blocks 6.37 -> 5.88 ms, 15.3 M
-// in FP32 0.69 -> 0.62.  Three wavefronts per SIMD (records written in
-// halves of 32 particles, 47 KB) took 8.6 ms: the halves double the record stores.
+// in FP32 0.69 -> 0.62.  More wavefronts have not: three per SIMD (records written in
+// halves of 32 particles, 47 KB) took 8.6 ms, since the halves double the record stores.
 //
-// PAIRED: eight wavefronts, two per SIMD (a z-layer's two row pairs), run
+// PAIRED: eight wavefronts, two per SIMD (w and w + 4, in layers two apart), run
 // in opposite phases locked by workgroup barriers: while one builds the
 // records of its next chunk (VALU), the other issues the matrix products of
 // its current one (MFMA), so the two units overlap instead of taking turns.
@@ -76,8 +78,6 @@ __device__ __forceinline__ int corner_of(int bx, int by, int bz) { return 4 * bz
 template <bool PAIRED>
 constexpr int waves_of() { return PAIRED ? 8 : 4; }
 
-// VF32: FP32 velocities (widened when the record is built, not at the load:
-// a conversion there would wait for the prefetched data)
 // How the cells are split: ncw cells per wavefront; with `extra` workgroups
 // (four per list entry) in front of the others, the crowded sub-tiles take
 // one workgroup per layer and 4 cells per wavefront.
@@ -116,6 +116,8 @@ __global__ __launch_bounds__(256) void k_crowded(int ntiles, int64_t nkeys, int 
   crowded[t] = c;
 }
 
+// VF32: FP32 velocities (widened when the record is built, not at the load:
+// a conversion there would wait for the prefetched data)
 template <bool BC, bool PAIRED, bool FUSED, bool VF32>
 __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(MeshView m, Species sp, double dtTotal,
                                                                  const double* __restrict__ B,
@@ -463,8 +465,8 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
         // LDS latency under load exceeds one step's two MFMAs), two steps to
         // a ds_read2_b64; the factors are multiplied just before use.  The five
         // running LDS addresses are opaque to the compiler, which otherwise adds
-        // a common offset to each of them again for every pair of steps: vector
-        // instructions and MFMAs share the issue slots that bound this pass.
+        // a common offset to each of them again for every pair of steps, vector
+        // instructions in a wavefront's way to its next product.
         struct Ops {
           double a[2], x0[2], y0[2], x1[2], y1[2];
         };

@@ -15,9 +15,9 @@ struct BlockGeom {
 // 1 / b to full precision, and a / b with it: the instruction sequence of the
 // compiler's a / b less the operand scaling and special-case fix-up
 // (v_div_scale, v_div_fixup), which are the identity for finite operands
-// within 2^+-700 or so, a zero numerator among them; so the quotients are the
-// same bits, and divisions by one denominator share its reciprocal (3
-// instructions each instead of 11).
+// within 2^+-700 or so, a zero numerator among them but for its sign (-0 / b
+// comes out as +0); so the quotients are the same bits, and divisions by one
+// denominator share its reciprocal (3 instructions each instead of 11).
 __device__ __forceinline__ double rcp_full(double b) {
   const double y0 = __builtin_amdgcn_rcp(b);
   const double y1 = fma(y0, fma(-b, y0, 1.0), y0);

@@ -110,7 +110,14 @@ __device__ __forceinline__ void push_count(int* __restrict__ count, const PushMi
   pd.p = p;
 }
 
-// W: the occupancy the register allocation aims at (waves per SIMD).
+// W: the occupancy the register allocation aims at (waves per SIMD), 4 unless
+// "push_waves" says otherwise.  The push waits on loads, so the fourth
+// wavefront gains more than its few spills cost wherever the chip is full: the
+// push of a step, us, with 4 and with the compiler's own allocation (W = 1):
+// FP64 Lapenta 16,384 particles 21.6 and 20.9, 2^20 76 and 77, 2.0 M 141 and
+// 145, 15.3 M 796 and 821, 67 M 3,336 and 3,520, 2^27 5,103 and 5,524; FP32
+// 2.0 M 109 and 125, 67 M 2,500 and 2,754.  Cell-centred B and the relativistic
+// mover are built with W = 1 alone.
 template <int MOVER, bool BC, int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k_push_f64(MeshView m, const Faces* __restrict__ faces, Species sp,
                                                    const double* __restrict__ E,
@@ -783,7 +790,6 @@ __global__ __launch_bounds__(256) void k_mig_clear(int64_t nkeys, int* __restric
 
 // The push tiles in one workgroup (meshes of up to TILE_WG blocks): counts,
 // their scan and the tiles.
-constexpr int TILE_WG = 8192;
 // exclusive prefix of v over the workgroup's 1,024 threads
 __device__ __forceinline__ int wg_prefix(int v, int* s) {
   int incl = v;

@@ -1342,7 +1342,7 @@ static void launch_fast(amps_ctx* c, TraceState* t, const typename S::View& v, c
   }
   // a grid size that was set is a bound here: it is tuned on one mode and kept
   // for all, and these kernels only lose above their own (full FP64 map, 142
-  // ms with 512 workgroups, 178 with 1,024; bracketed, 145 with 256, 309 with
+  // ms with 512 workgroups, 178 with 1,024; bracketed, one set of directions, 145 with 256, 309 with
   // 1,024, in FP32 338)
   const int own = c->n_cu * fast_wgs_per_cu(a.mode, precision, a.nloc, c->n_cu);
   const int wgs = t->grid_waves > 0 ? std::min(t->grid_waves, own) : own;

@@ -18,7 +18,8 @@
 // Same bits.  div() and root() are the instruction sequences that the
 // compiler emits for a / b and sqrt(x) less v_div_scale, v_div_fixup, ldexp
 // and the class tests, which are the identity for finite operands well inside
-// the exponent range (quotient, operands and reciprocal within 2^+-700).  The
+// the exponent range (quotient, operands and reciprocal within 2^+-700; a zero
+// quotient comes out as +0, equal to the -0 that a / b may give).  The
 // host admits only launches whose constants keep every operand in that range
 // (fast64_view); what depends on the trajectory is checked in the step: a
 // step with an operand outside is made again with the compiler's own
@@ -491,8 +492,9 @@ __device__ __forceinline__ void open_rescan(const ScanWork& a, int loc) {
 // to open.  A location's rescan therefore fills neighbouring lanes of one or
 // two wavefronts, where holding one bin of each unresolved location a lane
 // spread every rescan over the whole grid, one active lane a wavefront
-// (32,768 pairs: 310 against 210 ms with two wavefronts per SIMD, 152 against
-// 145 ms with one; the longest trajectory alone takes 75).  A lane whose item has not opened waits; every bracket item
+// (32,768 pairs, one set of directions: 310 against 210 ms with two wavefronts
+// per SIMD, 152 against 145 with one; eight other sets take 147 to 190 with one;
+// the longest trajectory alone takes 75).  A lane whose item has not opened waits; every bracket item
 // has been drawn and is being traced by then, and when the last of them
 // retires no further rescan opens, so every wait ends.
 //
@@ -696,7 +698,7 @@ __global__ __launch_bounds__(256) void k_upper_read(ScanWork a) {
 // which end a launch (full FP64 map: 177, 142, 175, 220 ms with 1, 2, 3, 4;
 // FP32: 152, 95, 106, 128 ms).  One where trajectories follow one another or
 // are traced ahead of need, so that the longest come late: the bracketed mode
-// (32,768 pairs: 145, 210, 260, 260 ms) and FP64 downward scans of fewer
+// (32,768 pairs, one set of directions: 145, 210, 260, 260 ms) and FP64 downward scans of fewer
 // locations than two wavefronts per SIMD have lanes (16,384: 91, 170, 215,
 // 220 ms; FP32, 131,738: 195, 147, 158, 181 ms).
 int fast_wgs_per_cu(int mode, int precision, int64_t nloc, int n_cu) {
