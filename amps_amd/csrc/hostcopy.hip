@@ -2,10 +2,13 @@
 //
 // A pageable hipMemcpy stages through the runtime's pinned buffers with one
 // host thread, which on a fresh array also takes its page faults: 17 GB/s to
-// the host and 28 from it, where the bus moves 57.  Here a few threads that
-// live for the call copy between the array and a context's own pinned slots,
-// two per thread, while the other slots are on the bus.
+// the host (4 on a fresh array) and 26 to 35 from it, where the bus moves 57.  Here a
+// few threads that live for the call copy between the array and a context's own
+// pinned slots, two per thread, while the other slots are on the bus: 40 GB/s
+// (12 on a fresh array), less some 130 us to start and join them.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
@@ -22,8 +25,12 @@ using namespace amps;
 namespace {
 constexpr int THREADS = 4, SLOTS = 2 * THREADS;
 constexpr size_t SLOT_BYTES = (size_t)2 << 20;
-// below this the threads cost more than they save (10-20 us each to start)
-constexpr size_t MIN_BYTES = (size_t)1 << 20;
+// Sizes from which the slots are ahead (us, a plain copy and the slots): to the
+// host, 2 MiB 125 and 183, 4 MiB 248 and 237, 16 MiB 926 and 527, but where
+// the pages are not there yet 512 KiB 95 and 165, 1 MiB 259 and 200, 4 MiB 1,063 and
+// 487; to the device, of an array that the caches hold 16 MiB 458 and 483, 32 MiB
+// 904 and 900, of one that they don't 8 MiB 323 and 343, 16 MiB 630 and 532.
+constexpr size_t MIN_TO_HOST = (size_t)4 << 20, MIN_TO_FRESH = (size_t)1 << 20, MIN_TO_DEVICE = (size_t)16 << 20;
 
 struct Job {
   amps_ctx* c;
@@ -74,11 +81,34 @@ void work(Job& j, int t) {
   if (e != hipSuccess) j.err.store((int)e);
 }
 
+// the array's first, middle and last page are in memory
+bool resident(const void* p, size_t bytes) {
+  const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE), a = (uintptr_t)p;
+  for (const uintptr_t q : {a, a + bytes / 2, a + bytes - 1}) {
+    unsigned char in = 0;
+    if (mincore((void*)(q / page * page), 1, &in) != 0 || !(in & 1)) return false;
+  }
+  return true;
+}
+
+bool through_slots(const amps_ctx* c, const void* host, size_t bytes, bool to_host) {
+  if (!c->h_pin || bytes < (to_host ? MIN_TO_FRESH : MIN_TO_DEVICE)) return false;
+  // pinned memory takes the bus's rate by itself (32 MiB 597 us, through the
+  // slots 915); what is no host memory at all is the runtime's to resolve
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, host) != hipSuccess)
+    (void)hipGetLastError();  // a pointer that the runtime does not know
+  else if (a.type != hipMemoryTypeUnregistered)
+    return false;
+  return !to_host || bytes >= MIN_TO_HOST || !resident(host, bytes);
+}
+
 int copy(amps_ctx* c, void* dst, const void* src, size_t bytes, bool to_host) {
-  const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
-  if (bytes < MIN_BYTES || !c->h_pin) {
-    HIP_TRY(hipMemcpyAsync(dst, src, bytes, kind, c->stream));
-    if (to_host) HIP_TRY(hipStreamSynchronize(c->stream));  // a pageable source is read before the return
+  if (!through_slots(c, to_host ? dst : src, bytes, to_host)) {
+    // complete on return (12 us for a few bytes, an asynchronous copy and a wait 20)
+    if (to_host) HIP_TRY(hipMemcpyWithStream(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    // a pageable source is read before the return
+    else HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
     return 0;
   }
   const std::lock_guard<std::mutex> lock(c->pin_mutex);  // one call at a time on the slots
