@@ -975,10 +975,11 @@ def test_two_threads_read_one_context(gpu_ctx, precision):
 
 
 @pytest.mark.parametrize("precision", [L.FP64, L.FP32])
-@pytest.mark.parametrize("n", [1, 131071, 131073, 600001])
+@pytest.mark.parametrize("n", [1, 131071, 131073, 174763, 524288, 524289, 600001])
 def test_particles_to_the_host(gpu_ctx, n, precision):
     """Columns on both sides of the size from which a copy goes through the
-    pinned slots (1 MiB: 131,072 doubles, or twice as many ints) and of
+    pinned slots (4 MiB: 174,763 positions, 524,288 ids; 1 MiB on fresh pages),
+    of the number up to which the host widens the narrow columns (2^19), and of
     several chunks with a ragged last one: what was set comes back, and the
     cells' numbers in restart order are those of the columns."""
     import ctypes
