@@ -97,6 +97,15 @@ struct PushMig {
   uint64_t* wmask;
 };
 
+// The crowded sub-tiles (4x4x4 cells) of the current layout: their number, a
+// list of at most `slots`, a flag for each of the mesh's (list_crowded).
+constexpr int CROWD_MIN = 2048;  // fewest particles of one
+struct Crowd {
+  int ntiles, slots;
+  int *count, *list;
+  uint8_t* flag;
+};
+
 // Synthetic-population generator arguments (k_generate).
 struct GenArgs {
   int64_t ntotal, base, rem;
@@ -184,7 +193,7 @@ struct amps_ctx {
                                // 3 eight lanes per cell
   int b_center = 0;            // 1: B from the cell-centred field (mover and deposit)
   // deposit
-  int* d_crowd = nullptr;      // crowded sub-tiles: count, list [2 n_cu], a byte per sub-tile
+  int* d_crowd = nullptr;      // crowded sub-tiles: count, list [2 n_cu], a byte per sub-tile (crowd_view)
   double* d_cellpart = nullptr;
   double* d_nodeout = nullptr;
   char* h_pin = nullptr;       // pinned slots of the copies to and from the caller's arrays
@@ -274,6 +283,12 @@ int launch_deposit_cell_mfma(amps_ctx* c, double dt);
 int launch_deposit_cell_lanes(amps_ctx* c, double dt);
 int alloc_particles(amps_ctx* c, int64_t n);  // both particle sets for at least n
 int build_tiles(amps_ctx* c);                 // push tiles from the current offsets
+inline Crowd crowd_view(const amps_ctx* c) {
+  const int slots = 2 * c->n_cu;
+  return {c->mv.nb * 8, slots, c->d_crowd, c->d_crowd + 1, (uint8_t*)(c->d_crowd + 1 + slots)};
+}
+// the crowded sub-tiles of offsets that no compaction has made (a compaction lists them itself)
+int list_crowded_tiles(amps_ctx* c);
 // append the exits of the last push (codes AMPS_CODE_EXIT_FACE0..+5) to the
 // exit list (exits.hip); no host synchronisation, capturable
 int collect_exits(amps_ctx* c);

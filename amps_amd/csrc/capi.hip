@@ -27,8 +27,9 @@ __global__ void k_count_keys(const int*, const int*, const int8_t*, int*);
 __global__ void k_scatter(const int*, const int*, const int8_t*, const int*, int*, int64_t,
                           const double*, const double*, int, const uint8_t*, const int64_t*,
                           double*, double*, uint8_t*, int*, int64_t*);
-__global__ void k_mig_finish(int64_t, const int*, int*, int*, int64_t, int*);
-__global__ void k_mig_clear(int64_t, int*, int*, int64_t, uint64_t*, int*, int*);
+__global__ void k_mig_finish(int64_t, const int*, int*, int*, int64_t, int*, Crowd);
+__global__ void k_mig_clear(int64_t, int*, int*, int64_t, uint64_t*, int*, int*, int*);
+__global__ void k_crowded(Crowd, const int*);
 __global__ void k_mig_classify(const int*, const int*, const int8_t*, const int*, int, const int*, int*, int*,
                                uint64_t*);
 __global__ void k_mig_order(int64_t, int, int, const int*, const int*, int*, int*, int*, int, const int*,
@@ -50,8 +51,8 @@ template <int NCH, bool EXACT>
 __global__ void k_deposit_cell(MeshView, Species, double, const double*, const int*, int64_t,
                                const double*, const double*, int, const uint8_t*, double*);
 template <bool MOMENT>
-__global__ void k_deposit_node(int64_t, int, const int*, const int*, const double*, double*, int*);
-__global__ void k_deposit_node_staged(int64_t, int, const int*, const int*, const double*, double*, int*);
+__global__ void k_deposit_node(int64_t, int, const int*, const int*, const double*, double*);
+__global__ void k_deposit_node_staged(int64_t, int, const int*, const int*, const double*, double*);
 __global__ void k_generate(MeshView, GenArgs, int64_t, double*, double*, uint8_t*, int*, int64_t*, int8_t*);
 __global__ void k_copy_probe(const float4*, float4*, int64_t);
 template <int W>
@@ -518,6 +519,7 @@ extern "C" int amps_gpu_set_mesh(amps_ctx* c, const amps_mesh_desc* desc, const 
   HIP_TRY(hipMalloc(&c->d_big, sizeof(int) * (nkeys + 1)));
   HIP_TRY(hipMalloc(&c->d_kbase, sizeof(int) * std::max<int64_t>(nkeys, 1)));
   HIP_TRY(hipMalloc(&c->d_cursor, sizeof(int) * nkeys));
+  HIP_TRY(hipMalloc(&c->d_crowd, sizeof(int) * (1 + 2 * (size_t)c->n_cu) + (size_t)nb * 8));
   HIP_TRY(hipMalloc(&c->d_mig_slab, sizeof(int) * (nkeys * MIG_SLAB + 1)));
   c->layout_valid = false;
   HIP_TRY(hipMalloc(&c->d_tcount, sizeof(int) * (nb + 1)));
@@ -727,6 +729,14 @@ int amps::build_tiles(amps_ctx* c) {
   return AMPS_OK;
 }
 
+int amps::list_crowded_tiles(amps_ctx* c) {
+  const Crowd cr = crowd_view(c);
+  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, c->stream, cr.count, 1, 0);
+  hipLaunchKernelGGL(k_crowded, dim3((unsigned)((cr.ntiles + 15) / 16)), dim3(256), 0, c->stream, cr, c->d_offset);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 extern "C" int amps_gpu_set_particles(amps_ctx* c, int64_t n, const double* x, const double* v,
                                       const int32_t* spec, const int32_t* blk,
                                       const int32_t* cell, const int64_t* id, int32_t precision) {
@@ -790,6 +800,7 @@ extern "C" int amps_gpu_set_particles(amps_ctx* c, int64_t n, const double* x, c
   c->precision = precision;
   c->offsets_valid = true;
   if (int r = build_tiles(c)) return r;
+  if (int r = list_crowded_tiles(c)) return r;
   HIP_TRY(hipStreamSynchronize(c->stream));
   return AMPS_OK;
 }
@@ -895,7 +906,8 @@ static void clear_counts(amps_ctx* c, bool classify = false) {
   const int64_t most = std::max(nkeys, classify ? nw : 0);
   hipLaunchKernelGGL(k_mig_clear, dim3((unsigned)std::min<int64_t>(2048, (most + 255) / 256)), dim3(256), 0, c->stream,
                      nkeys, classify ? nullptr : c->d_offset, c->d_cursor, nw, classify ? c->d_wmask : nullptr,
-                     c->d_mig_slab + nkeys * MIG_SLAB, c->d_big + nkeys);
+                     c->d_mig_slab + nkeys * MIG_SLAB, c->d_big + nkeys, c->d_crowd);
+  c->offsets_valid = false;  // until the compaction that follows ends
 }
 
 // counted: the push has already counted the survivors into a cleared d_offset
@@ -975,10 +987,10 @@ static int compact_impl(amps_ctx* c, bool counted = false, bool defer = false, b
   c->offsets_valid = true;
   // all survivors carry a committed code
   std::swap(c->d_code, c->d_code2);
-  // the new layout, for the next compaction, and the codes
+  // the new layout, for the next compaction, the codes and the crowded sub-tiles
   hipLaunchKernelGGL(k_mig_finish, dim3((unsigned)std::min<int64_t>(2048, (std::max(nkeys, (cap + 3) / 4) + 256) / 256)),
                      dim3(256), 0, c->stream, nkeys, c->d_offset, c->d_off_layout, c->d_n, (cap + 3) / 4,
-                     (int*)c->d_code);
+                     (int*)c->d_code, crowd_view(c));
   c->layout_valid = true;
   if (small) {
     c->tiles_valid = true;
@@ -1158,13 +1170,13 @@ static int launch_deposit(amps_ctx* c, double dt) {
   // the record-batched and matrix-core cell passes write the moment form unless bit-exact
   if (c->dep_kernel >= 1 && !c->dep_exact && c->node_staged)
     hipLaunchKernelGGL(k_deposit_node_staged, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout, c->d_crowd);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout);
   else if (c->dep_kernel >= 1 && !c->dep_exact)
     hipLaunchKernelGGL(k_deposit_node<true>, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout, c->d_crowd);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8_oct, c->d_cellpart, c->d_nodeout);
   else
     hipLaunchKernelGGL(k_deposit_node<false>, dim3((unsigned)node_wgs), dim3(256), 0, c->stream,
-                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8, c->d_cellpart, c->d_nodeout, c->d_crowd);
+                       c->nnodes, nb_eff, c->d_node_order, c->d_inc8, c->d_cellpart, c->d_nodeout);
   HIP_TRY(hipGetLastError());
   tend(c, AMPS_K_DEPOSIT_NODE);
   return 0;
@@ -1178,10 +1190,6 @@ static int ensure_deposit_buffers(amps_ctx* c) {
     HIP_TRY(hipMalloc(&c->d_cellpart, sizeof(double) * n));
     HIP_TRY(hipMemset(c->d_cellpart + (size_t)c->zero_rec * CELL_STRIDE_MOMENT, 0,
                       sizeof(double) * CELL_STRIDE_MOMENT));
-  }
-  if (!c->d_crowd) {
-    HIP_TRY(hipMalloc(&c->d_crowd, sizeof(int) * (1 + 2 * (size_t)c->n_cu) + (size_t)c->mv.nb * 8));
-    HIP_TRY(hipMemset(c->d_crowd, 0, sizeof(int)));
   }
   if (!c->d_nodeout) HIP_TRY(hipMalloc(&c->d_nodeout, sizeof(double) * (size_t)c->nnodes * NODE_STRIDE));
   return 0;

@@ -18,7 +18,7 @@
 // cells of z-layer w (8 or 4 cells a wavefront, and fewer layers a workgroup, on
 // meshes of few blocks).  Its cells' particles are consecutive runs of the
 // key-sorted arrays; the wavefront walks their concatenation, each cell's run
-// rounded up to whole steps of 4, 64 places at a
+// rounded up to whole steps of 4 (but for SPARSE populations), 64 places at a
 // time: each lane turns one particle into its operand record (corner stencil,
 // B from the sub-tile's corners staged in LDS, alpha, alpha v) in LDS, then the
 // wavefront issues the MFMA steps cell by cell and writes a finished cell's
@@ -41,6 +41,8 @@
 // records of its next chunk (VALU), the other issues the matrix products of
 // its current one (MFMA), so the two units overlap instead of taking turns.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "amps_common.h"
 #include "center_device.h"
@@ -78,47 +80,32 @@ __device__ __forceinline__ int corner_of(int bx, int by, int bz) { return 4 * bz
 template <bool PAIRED>
 constexpr int waves_of() { return PAIRED ? 8 : 4; }
 
-// How the cells are split: ncw cells per wavefront; with `extra` workgroups
+// How the cells are split: 2^lw cells per wavefront; with `extra` workgroups
 // (four per list entry) in front of the others, the crowded sub-tiles take
 // one workgroup per layer and 4 cells per wavefront.
 struct Split {
-  int ncw, extra;
-  int* count;  // crowded sub-tiles; the node gather clears it for the next pass
+  int lw, extra;
+  const int* count;  // crowded sub-tiles of the layout
   const int* list;
   const uint8_t* crowded;  // per sub-tile
 };
 
-// The crowded sub-tiles, those with more particles than an equal share of
-// all of them for each workgroup the chip holds (so at most that many), which
-// alone would outlast the rest, and twice the mean (64 blocks are one
-// workgroup each: splitting those above the mean took 60 us instead of 41).
-// With drifted electrons standing at the walls (1,000 steps on the two-level
-// mesh, 2.0 M particles) the pass took 429 us, with the split 163, 131 at the
-// start of the run; the list takes 4.7 us.
-// 16 lanes a sub-tile, one row of 4 cells each.
-__global__ __launch_bounds__(256) void k_crowded(int ntiles, int64_t nkeys, int slots, const int* __restrict__ offset,
-                                                  int* __restrict__ count, int* __restrict__ list,
-                                                  uint8_t* __restrict__ crowded) {
-  const int t = blockIdx.x * 16 + (threadIdx.x >> 4), r = threadIdx.x & 15;
-  if (t >= ntiles) return;
-  const int st = t & 7, x = (st & 1) * 4, y = ((st >> 1) & 1) * 4 + (r & 3), z = (st >> 2) * 4 + (r >> 2);
-  const int k = (t >> 3) * NCELL + x + NC * (y + NC * z);
-  int n = offset[k + 4] - offset[k];
-  for (int d = 1; d < 16; d <<= 1) n += __shfl_xor(n, d);
-  if (r) return;
-  const int64_t total = offset[nkeys];
-  bool c = (int64_t)n * slots > total && (int64_t)n * ntiles > 2 * total;
-  if (c) {
-    const int at = atomicAdd(count, 1);
-    c = at < slots;  // always, unless a pass before was cut off by an error
-    if (c) list[at] = t;
-  }
-  crowded[t] = c;
-}
-
 // VF32: FP32 velocities (widened when the record is built, not at the load:
 // a conversion there would wait for the prefetched data)
-template <bool BC, bool PAIRED, bool FUSED, bool VF32>
+// SPARSE: cells of few particles (mean below SPARSE_MEAN).  There the rounding
+// to whole steps of 4 costs places, and with them chunks, and the loop's
+// start, which loads four steps, costs more than its pace gains: the cells' runs
+// stay as they are, one or two steps are issued without the loop and the
+// last 1-3 particles as a step of their own, and no chunk past the last is
+// looked for.  The pass at 1, 2, 4 and 8
+// particles per cell, us: 7,456 blocks 2,338, 2,470, 2,706 and 3,082 against
+// 2,459, 2,590, 2,787 and 3,116 in whole steps; 64 blocks, 1, 4 and 8: 22.5,
+// 26.0 and 31.5 against 26.5, 28.7 and 32.7.  At 35 a cell whole steps are ahead (7,456
+// blocks 5.94 ms against 6.03 with the short runs out of the loop, 6.4 with ragged
+// ones).
+constexpr int SPARSE_MEAN = 10;
+
+template <bool BC, bool PAIRED, bool FUSED, bool VF32, bool SPARSE>
 __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(MeshView m, Species sp, double dtTotal,
                                                                  const double* __restrict__ B,
                                                                  const int* __restrict__ offset,
@@ -140,15 +127,17 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   __shared__ int sfirst[MW][MCW], scum[MW][MCW + 1];
   __shared__ __align__(16) double sstage[MW][CS + 2];  // a finished cell's record, written out in full lines, and a spare place
   __shared__ int smaxchunks;
-  // cells per wavefront, wavefronts per layer, layers per workgroup
-  int ncw = PAIRED ? 8 : BC ? 16 : sp4.ncw;
-  int wpl = 16 / ncw, lz = MW / wpl;
+  // 2^lw cells per wavefront, 2^(4 - lw) wavefronts per layer, 2^lz layers per
+  // workgroup (logarithms: a division by a run-time value is some 30 instructions)
+  constexpr int LMW = PAIRED ? 3 : 2;
+  int lw = PAIRED ? 3 : BC ? 4 : sp4.lw, lz = LMW - 4 + lw;
   int b, st, sz;
+  bool skip = false;
   if (!PAIRED && !BC && (int)blockIdx.x < sp4.extra) {
     // a layer of a crowded sub-tile
     if ((int)(blockIdx.x >> 2) >= sp4.count[0]) return;
     const int tile = sp4.list[blockIdx.x >> 2];
-    ncw = 4, wpl = 4, lz = 1;
+    lw = 2, lz = 0;
     b = tile >> 3, st = tile & 7;
     sz = (st >> 2) * 4 + (blockIdx.x & 3);
   } else {
@@ -156,20 +145,20 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     const int extra = PAIRED || BC ? 0 : sp4.extra;
     const int bi = blockIdx.x - extra, ng = gridDim.x - extra;
     const int tile = (bi % N_XCD) * (ng / N_XCD) + bi / N_XCD;
-    if (extra && sp4.crowded[tile]) return;
-    const int tpb = 4 * (NC / lz);  // workgroups per block
-    b = tile / tpb, st = tile % tpb;
-    sz = (st >> 2) * lz;
+    if (extra) skip = sp4.crowded[tile];  // tested below, when the other loads are on their way
+    b = tile >> (5 - lz), st = tile & ((32 >> lz) - 1);
+    sz = (st >> 2) << lz;
   }
+  const int ncw = 1 << lw;
   const int sx = (st & 1) * 4, sy = ((st >> 1) & 1) * 4;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // wavefront w: layer w / wpl, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
-  const int zl = uniform(w / wpl), zc = sz + zl;
-  const int row0 = uniform((w % wpl) * (ncw / 4));
+  // wavefront w: layer zl, rows row0.. of it (cell c: x = c % 4, y = row0 + c / 4)
+  const int zl = uniform(w >> (4 - lw)), zc = sz + zl;
+  const int row0 = uniform((w & ((16 >> lw) - 1)) << (lw - 2));
   const int keybase = b * NCELL;
   if constexpr (!BC) {
     const double* Bb = B + (size_t)b * NCORNER * 3;
-    for (int i = threadIdx.x; i < 75 * (lz + 1); i += blockDim.x) {
+    for (int i = threadIdx.x; i < 75 * ((1 << lz) + 1); i += blockDim.x) {
       const int cidx = i / 3, d = i % 3;
       const int a0 = cidx % 5, a1 = (cidx / 5) % 5, a2 = cidx / 25;
       sB[i] = Bb[3 * ((sx + a0) + NN * ((sy + a1) + NN * (sz + a2))) + d];
@@ -197,14 +186,14 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   if (threadIdx.x < 3) sconst[MAX_SPEC][threadIdx.x] = 0.0;
   auto cellkey = [&](int c) { return keybase + (sx + (c & 3)) + NC * ((sy + row0 + (c >> 2)) + NC * zc); };
   // this wavefront's cells: first particle, running counts, each rounded up to
-  // whole steps of 4 particles
+  // whole steps of 4 particles (not SPARSE)
   int cntk = 0;
   {
     // counts of lanes' cells, then an inclusive scan across the lanes
     const int ck = cellkey(lane < ncw ? lane : 0);
     const int o0 = offset[ck];
     cntk = lane < ncw ? offset[ck + 1] - o0 : 0;
-    const int cnt = (cntk + 3) & ~3;
+    const int cnt = SPARSE ? cntk : (cntk + 3) & ~3;
     int incl = cnt;
 #pragma unroll
     for (int d = 1; d < MCW; d <<= 1) {
@@ -218,6 +207,7 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
     if (lane == ncw - 1) scum[w][ncw] = incl;
   }
   if (threadIdx.x == 0) smaxchunks = 0;
+  if (skip) return;  // the whole workgroup: its layers are in the list
   __syncthreads();
   const int* cum = scum[w];
   const int total = uniform(cum[ncw]);
@@ -447,8 +437,10 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
         for (int by = 0; by < 2; by++) FLD(F_WYZ + by + 2 * bz) = Lf[2 + by] * Lf[4 + bz];
 #undef FLD
     }
-    fetch(ix, nb);  // in flight while two chunks are accumulated
-    index(base + 192, ix);
+    if (!SPARSE || base + 128 < total) {
+      fetch(ix, nb);  // in flight while two chunks are accumulated
+      index(base + 192, ix);
+    }
   };
   // the matrix products of that chunk, cell by cell, and the finished cells' records
   auto accumulate = [&](int base) {
@@ -460,7 +452,17 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
       // steps of 4 particles
       const int nfull = (se - q) >> 2;
       const double* R = R0 + (q - base + slot);
-      if (nfull > 0) {
+      if (SPARSE && nfull > 0 && nfull <= 2) {
+        const double a0 = R[oa], a1 = R[oa + 4];
+        const double b00 = R[o0a] * R[o0b], b01 = R[o0a + 4] * R[o0b + 4];
+        const double b10 = R[o1a] * R[o1b], b11 = R[o1a + 4] * R[o1b + 4];
+        C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b00, C0, 0, 0, 0);
+        C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b10, C1, 0, 0, 0);
+        if (nfull == 2) {
+          C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b01, C0, 0, 0, 0);
+          C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b11, C1, 0, 0, 0);
+        }
+      } else if (nfull > 0) {
         // the raw operands of four steps in flight ahead of the products (the
         // LDS latency under load exceeds one step's two MFMAs), two steps to
         // a ds_read2_b64; the factors are multiplied just before use.  The five
@@ -514,6 +516,18 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
         if (t >= 2) step(pa, 1);
         if (t >= 3) step(pb, 0);
       }
+      if (SPARSE && q + 4 * nfull < se) {
+        // the cell's last 1-3 particles in this chunk: the other slots add zero
+        const double* Rt = R + 4 * nfull;
+        double a = 0.0, b0 = 0.0, b1 = 0.0;
+        if (q + 4 * nfull + slot < se) {
+          a = Rt[oa];
+          b0 = Rt[o0a] * Rt[o0b];
+          b1 = Rt[o1a] * Rt[o1b];
+        }
+        C0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, C0, 0, 0, 0);
+        C1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, C1, 0, 0, 0);
+      }
       q = se;
       if (q == ce) {
         flush(cur++);
@@ -558,21 +572,21 @@ __global__ __launch_bounds__(64 * waves_of<PAIRED>()) void k_deposit_cell_mfma(M
   }
 }
 
-template <bool BC, bool PAIRED, bool FUSED, bool VF32>
+template <bool BC, bool PAIRED, bool FUSED, bool VF32, bool SPARSE>
 void launch(amps_ctx* c, double dt, const Split& sp4) {
   const int k = c->cur;
   // FUSED: the particles are read from the previous buffer through the
   // migration's source indices
   const int r = FUSED ? 1 - k : k;
-  const unsigned grid = (unsigned)(c->mv.nb * (PAIRED || BC ? 8 : 8 * (16 / sp4.ncw)) + sp4.extra);
-  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32>), dim3(grid), dim3(64 * waves_of<PAIRED>()), 0,
+  const unsigned grid = (unsigned)(c->mv.nb * (PAIRED || BC ? 8 : 8 << (4 - sp4.lw)) + sp4.extra);
+  hipLaunchKernelGGL((k_deposit_cell_mfma<BC, PAIRED, FUSED, VF32, SPARSE>), dim3(grid), dim3(64 * waves_of<PAIRED>()), 0,
                      c->stream, c->mv, c->sp, dt, c->d_B, c->d_offset, c->cap, c->d_x[r], c->d_v[r],
                      c->precision == AMPS_FP32 ? 1 : 0, c->d_spec[r], c->d_cellpart, c->d_Bc, c->d_tmpsrc, sp4);
 }
 
 template <bool BC, bool PAIRED, bool FUSED>
 void launch_v(amps_ctx* c, double dt, bool vf32) {
-  Split s = {16, 0, nullptr, nullptr, nullptr};
+  Split s = {4, 0, nullptr, nullptr, nullptr};
   if constexpr (!PAIRED && !BC) {
     // fewer cells per wavefront where 16 would not give the chip its 8
     // wavefronts per CU (two workgroups): 8 blocks take 21, 13.6 and 10.5 us
@@ -580,19 +594,20 @@ void launch_v(amps_ctx* c, double dt, bool vf32) {
     // 40.9, 42.7 and 46.5 us, and on 7,456 blocks 5.88, 6.11 and 6.84 ms: each
     // wavefront pays once for its first loads
     const int64_t waves = (int64_t)c->mv.nb * 32, resident = (int64_t)c->n_cu * 8;
-    s.ncw = waves >= resident ? 16 : 2 * waves >= resident ? 8 : 4;
-    if (s.ncw == 16) {
-      const int slots = 2 * c->n_cu, nt = c->mv.nb * 8;
-      s.extra = 4 * slots;
-      s.count = c->d_crowd;
-      s.list = c->d_crowd + 1;
-      s.crowded = (const uint8_t*)(c->d_crowd + 1 + slots);
-      hipLaunchKernelGGL(k_crowded, dim3((unsigned)((nt + 15) / 16)), dim3(256), 0, c->stream, nt,
-                         (int64_t)c->mv.nb * NCELL, slots, c->d_offset, s.count, c->d_crowd + 1,
-                         (uint8_t*)(c->d_crowd + 1 + slots));
+    s.lw = waves >= resident ? 4 : 2 * waves >= resident ? 3 : 2;
+    if (s.lw == 4) {
+      const Crowd cr = crowd_view(c);
+      // fewer than half of them hold twice the mean
+      s.extra = 4 * (int)std::min<int64_t>(std::min(cr.slots, cr.ntiles / 2), c->n / CROWD_MIN);
+      s.count = cr.count, s.list = cr.list, s.crowded = cr.flag;
     }
   }
-  vf32 ? launch<BC, PAIRED, FUSED, true>(c, dt, s) : launch<BC, PAIRED, FUSED, false>(c, dt, s);
+  // by the host's count, which deletions since then can only have lowered
+  const bool sparse = !PAIRED && c->n < (int64_t)SPARSE_MEAN * c->mv.nb * NCELL;
+  if (sparse)
+    vf32 ? launch<BC, PAIRED, FUSED, true, !PAIRED>(c, dt, s) : launch<BC, PAIRED, FUSED, false, !PAIRED>(c, dt, s);
+  else
+    vf32 ? launch<BC, PAIRED, FUSED, true, false>(c, dt, s) : launch<BC, PAIRED, FUSED, false, false>(c, dt, s);
 }
 
 }  // namespace

@@ -64,6 +64,34 @@ __device__ __forceinline__ void stage_species(const Species& sp, SpeciesPush* s)
   }
 }
 
+// The crowded sub-tiles, those with more particles than an equal share of
+// all of them for each workgroup the chip holds (so at most that many), which
+// alone would outlast the rest of the deposit's cell pass, and twice the mean
+// (64 blocks are one workgroup each: splitting those above the mean took 60 us
+// instead of 41), and CROWD_MIN (46 us of its workgroup, at 5.8 us for 64
+// particles of a wavefront; 64 blocks half of which were empty took 29 us with
+// sub-tiles of 128 particles split and 23 without).  With drifted electrons standing at the walls (1,000 steps on
+// the two-level mesh, 2.0 M particles) the pass took 429 us, with the split 163, 131
+// at the start of the run.  The list belongs to the layout: the compaction's
+// last kernel makes it (in a launch of its own before every pass it took 5 us).
+// 16 lanes a sub-tile, one row of 4 cells each; i: the lane among all of them.
+__device__ __forceinline__ void list_crowded(const Crowd& cr, int64_t i, const int* __restrict__ offset) {
+  const int t = (int)(i >> 4), r = (int)(i & 15);
+  const int st = t & 7, x = (st & 1) * 4, y = ((st >> 1) & 1) * 4 + (r & 3), z = (st >> 2) * 4 + (r >> 2);
+  const int k = (t >> 3) * NCELL + x + NC * (y + NC * z);
+  int n = offset[k + 4] - offset[k];
+  for (int d = 1; d < 16; d <<= 1) n += __shfl_xor(n, d);
+  if (r) return;
+  const int64_t total = offset[cr.ntiles / 8 * (int64_t)NCELL];
+  bool c = n >= CROWD_MIN && (int64_t)n * cr.slots > total && (int64_t)n * cr.ntiles > 2 * total;
+  if (c) {
+    const int at = atomicAdd(cr.count, 1);
+    c = at < cr.slots;
+    if (c) cr.list[at] = t;
+  }
+  cr.flag[t] = c;
+}
+
 __device__ __forceinline__ void load_block_geom(const MeshView& m, int b, BlockGeom& g) {
 #pragma unroll
   for (int d = 0; d < 3; d++) {

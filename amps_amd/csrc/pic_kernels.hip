@@ -760,20 +760,26 @@ __global__ __launch_bounds__(256) void k_mig_scatter(const int* __restrict__ n_d
 }
 
 // The end of a compaction: the new layout and particle count for the next
-// one, and every survivor's code committed.
+// one, every survivor's code committed, the crowded sub-tiles listed.
 __global__ __launch_bounds__(256) void k_mig_finish(int64_t nkeys, const int* __restrict__ offset, int* __restrict__ lay,
-                                                     int* __restrict__ n_dev, int64_t ncode4, int* __restrict__ code) {
+                                                     int* __restrict__ n_dev, int64_t ncode4, int* __restrict__ code,
+                                                     Crowd cr) {
   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = i0; i <= nkeys; i += st) lay[i] = offset[i];
   for (int64_t i = i0; i < ncode4; i += st) code[i] = 0x03030303;
   if (i0 == 0) *n_dev = offset[nkeys];
+  for (int64_t i = i0; i < (int64_t)cr.ntiles * 16; i += st) list_crowded(cr, i, offset);  // whole wavefronts
+}
+__global__ __launch_bounds__(256) void k_crowded(Crowd cr, const int* __restrict__ offset) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < (int64_t)cr.ntiles * 16) list_crowded(cr, i, offset);
 }
 
 // What a step's counting starts from: zeroed counters (count null: not used),
 // stayer masks (wmask null likewise) and list lengths.
 __global__ __launch_bounds__(256) void k_mig_clear(int64_t nkeys, int* __restrict__ count, int* __restrict__ cursor,
                                                     int64_t nw, uint64_t* __restrict__ wmask, int* __restrict__ novf,
-                                                    int* __restrict__ nbig) {
+                                                    int* __restrict__ nbig, int* __restrict__ ncrowd) {
   const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, st = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = i0; i < nkeys; i += st) {
     cursor[i] = 0;
@@ -785,6 +791,7 @@ __global__ __launch_bounds__(256) void k_mig_clear(int64_t nkeys, int* __restric
     if (count) count[nkeys] = 0;
     *novf = 0;
     *nbig = 0;
+    *ncrowd = 0;
   }
 }
 
@@ -1114,8 +1121,7 @@ __global__ __launch_bounds__(256) void k_deposit_node(int64_t nnodes, int npw,
                                                        const int* __restrict__ node_order,
                                                        const int* __restrict__ inc8,
                                                        const double* __restrict__ cellpart,
-                                                       double* __restrict__ nodeout, int* clear) {
-  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // the cell pass's list, done with
+                                                       double* __restrict__ nodeout) {
   constexpr int STRIDE = MOMENT ? CELL_STRIDE_MOMENT : CELL_VALS;
   __shared__ __align__(16) short soff[8][256];
   static_assert(sizeof(soff) == 256 * 16, "one 16-byte row per thread");
@@ -1169,8 +1175,8 @@ __global__ __launch_bounds__(256) void k_deposit_node(int64_t nnodes, int npw,
   }
 }
 
-template __global__ void k_deposit_node<false>(int64_t, int, const int*, const int*, const double*, double*, int*);
-template __global__ void k_deposit_node<true>(int64_t, int, const int*, const int*, const double*, double*, int*);
+template __global__ void k_deposit_node<false>(int64_t, int, const int*, const int*, const double*, double*);
+template __global__ void k_deposit_node<true>(int64_t, int, const int*, const int*, const double*, double*);
 
 // Node gather for the moment record, staged.  The incidence rows come in
 // octant order (slot t: the cell on the node's side (t & 1, t >> 1 & 1,
@@ -1198,8 +1204,7 @@ __global__ __launch_bounds__(256) void k_deposit_node_staged(int64_t nnodes, int
                                                              const int* __restrict__ node_order,
                                                              const int* __restrict__ inc8,
                                                              const double* __restrict__ cellpart,
-                                                             double* __restrict__ nodeout, int* clear) {
-  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;  // the cell pass's list, done with
+                                                             double* __restrict__ nodeout) {
   __shared__ double G[4][8 * NODE_G + 1];  // the gathered values, then a zero
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;

@@ -286,6 +286,7 @@ extern "C" int amps_gpu_set_particles_restart(amps_ctx* c, const amps_aos_layout
   c->precision = precision;
   c->offsets_valid = true;
   if (int r = build_tiles(c)) return r;
+  if (int r = list_crowded_tiles(c)) return r;
   HIP_TRY(hipStreamSynchronize(c->stream));
   return AMPS_OK;
 }

@@ -122,17 +122,18 @@ def test_deposit_center_B(gpu_ctx, exact):
 
 
 @pytest.mark.parametrize("paired", [0, 1])
-def test_deposit_center_B_reads_only_the_particles_own_cells(gpu_ctx, paired):
+@pytest.mark.parametrize("ppc", [(3, 2), (7, 6)])
+def test_deposit_center_B_reads_only_the_particles_own_cells(gpu_ctx, ppc, paired):
     """A not-a-number in the first cell of every block reaches the nodes of the
-    particles that interpolate it and no others: cells of five particles, so
-    that the matrix-core pass fills up their last steps of four."""
+    particles that interpolate it and no others: cells of five (sparse) and of
+    thirteen particles, whose last step of four the matrix-core pass fills up."""
     from amps_amd import autotune
 
     mesh = M.uniform_mesh(1)
     E, Bk = M.corner_fields(mesh)
     Bc = M.center_fields(mesh, lambda P: M.dipole_field(P))
     Bc[:, 111] = np.nan  # cell (0, 0, 0) behind one layer of ghosts
-    parts = M.per_cell_particles(mesh, [3, 2], [0.05, 0.005], drift=(0.01, 0.0, 0.0))
+    parts = M.per_cell_particles(mesh, list(ppc), [0.05, 0.005], drift=(0.01, 0.0, 0.0))
     dt = 0.1 / (np.max(np.linalg.norm(Bk, axis=-1)) / 0.01)
     sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
     st = PicState(mesh, E, Bk, sp, ctx=gpu_ctx)

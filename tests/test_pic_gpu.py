@@ -707,6 +707,82 @@ def test_deposit_cells_per_wavefront(gpu_ctx, nblocks, precision):
         set_deposit_variant(gpu_ctx, 2, 12)
 
 
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+@pytest.mark.parametrize("per_cell", [0.4, 1, 3, 9.99, 10])
+def test_deposit_sparse_populations(gpu_ctx, per_cell, precision):
+    """Both sides of the mean of ten particles per cell below which the
+    matrix-core pass leaves the cells' runs ragged: cells of none to some fifty
+    (runs of one and two whole steps with every remainder, over chunk ends),
+    against the oracle, the bound of test_deposit_ragged_cells."""
+    mesh = M.uniform_mesh(2)
+    E, B = M.corner_fields(mesh)
+    dt = 0.05
+    sp = Species([-1.0, 1.0], [0.01, 1.0], [dt, dt])
+    n = int(per_cell * mesh.ncells)
+    parts = M.uniform_particles(mesh, n, 0.05, r_excl=0.0)
+    if per_cell > 1:  # denser towards one side
+        parts.x[0] = -1.0 + 2.0 * ((parts.x[0] + 1.0) / 2.0) ** 2
+        parts.blk = mesh.locate(parts.x.T).astype(np.int32)
+        parts.cell = M.cell_of(mesh, parts.x, parts.blk)
+    parts.spec = (np.arange(n) % 2).astype(np.int32)
+    st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+    st.set_particles(parts, precision=precision)
+    set_deposit_variant(gpu_ctx, 2, 12)
+    J, Mm = st.UpdateJMassMatrix(dt)
+    g, _ = st.get_particles()
+    om = O.Mesh(mesh)
+    noc, keys = om.build_nodes()
+    Jo, Mo = O.deposit(om, B, sp, dt, g, noc, len(keys))
+    cnt = np.bincount(g.blk.astype(np.int64) * 512 + g.cell, minlength=mesh.ncells)
+    print(f"{n} particles, at most {cnt.max()} in a cell, {(cnt == 0).sum()} empty", flush=True)
+    for a, b in ((J, Jo), (Mm, Mo)):
+        assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1)).all()
+    # a step's deposit reads through the source indices
+    probe = np.random.default_rng(3).standard_normal((len(keys), 3))
+    st.run_steps(1, dt, use_graph=False)
+    fused = st.MassMatrixApply(probe, 1.0)
+    st.UpdateJMassMatrix(dt, copy_out=False)
+    assert np.abs(fused).max() > 0 and np.array_equal(fused, st.MassMatrixApply(probe, 1.0))
+
+
+def test_crowded_subtiles_follow_the_layout(gpu_ctx):
+    """The list of crowded sub-tiles is made with the layout: J and M against
+    the oracle after a step that leaves a crowd where it is, after steps that
+    carry it to other sub-tiles, and from restart records."""
+    mesh = M.central_octant_mesh()
+    E, B = M.corner_fields(mesh)
+    E, B = np.zeros_like(E), np.zeros_like(B)
+    dt = 0.125
+    sp = Species([-1.0, 1.0], [1.0, 1.0], [dt, dt])
+    base = M.per_cell_particles(mesh, [2, 2], [1e-3, 1e-3])
+    key = base.blk.astype(np.int64) * 512 + base.cell
+    crowd = np.random.default_rng(5).choice(mesh.ncells, 3, replace=False)
+    many = base.take(np.repeat(np.arange(base.n), np.where(np.isin(key, crowd), 700, 1)))
+    many.id = np.arange(many.n)
+    moving = np.isin(many.blk.astype(np.int64) * 512 + many.cell, crowd)
+    om = O.Mesh(mesh)
+    noc, keys = om.build_nodes()
+    set_deposit_variant(gpu_ctx, 2, 12)
+
+    def check(st):
+        J, Mm = st.UpdateJMassMatrix(dt)
+        g, _ = st.get_particles()
+        Jo, Mo = O.deposit(om, B, sp, dt, g, noc, len(keys))
+        for a, b in ((J, Jo), (Mm, Mo)):
+            assert (np.linalg.norm(a - b, axis=1) <= 1e-12 * np.linalg.norm(b, axis=1)).all()
+
+    for speed in (0.0, 0.5):
+        many.v[:, moving] = np.array([speed, -speed, 0.7 * speed])[:, None]
+        st = PicState(mesh, E, B, sp, ctx=gpu_ctx)
+        st.set_particles(many)
+        for _ in range(3):
+            st.run_steps(2, dt, use_graph=False)
+            check(st)
+        counts, rec = st.get_restart(L.aos_layout_aligned())
+        st.set_restart(L.aos_layout_aligned(), counts, rec)
+        check(st)
+
+
 @pytest.mark.parametrize("crowds", [1, 3, 20])
 def test_deposit_crowded_subtiles(gpu_ctx, crowds):
     """Sub-tiles that hold more than an equal share of the particles, whose
