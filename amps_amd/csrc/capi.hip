@@ -691,10 +691,16 @@ int amps::alloc_particles(amps_ctx* c, int64_t n) {
 // the rule: 16,384 particles 0.072 and 0.023, 2^20 0.151 and 0.068, 2.0 M
 // 0.269 and 0.169, 15.3 M FP32 0.866 and 0.822); from 2^24 on it is the best,
 // since every tile reads its block's 35 KB of fields (2^27: 7.6 ms with 1024,
-// 6.4 with 8192).
+// 6.4 with 8192).  Where the blocks alone are a workgroup for every CU, a tile
+// takes a block's mean number, up to 1,024, before blocks are cut up (512 blocks,
+// us with 256, 512, 1024 and 2048: 2^18 particles 51, 44, 52 and 65, 2^19 74, 66,
+// 62 and 89, 2^20 127, 101, 97 and 103; with 8192 43, 63 and 101 in the build
+// before the rule).
 static int push_tile(const amps_ctx* c) {
   if (c->tile_given) return c->tile;
   int t = 256;
+  if (c->mv.nb >= c->n_cu)
+    while (t < 1024 && t < c->cap / c->mv.nb) t *= 2;
   while (t < 8192 && c->cap / (2 * t) >= 2048) t *= 2;
   return t;
 }

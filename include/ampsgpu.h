@@ -65,7 +65,8 @@ int amps_gpu_device_info(amps_ctx* ctx, char* name, int* n_cu, int64_t* hbm_byte
 
 /* Tuning parameters (no reference counterpart; set by the autotuner):
  * "tile" (particles per push workgroup, 64..2^20; until set, the largest
- * power of two from 256 to 8192 of which the capacity holds 2,048),
+ * power of two from 256 to 8192 of which the capacity holds 2,048, or, on
+ * meshes of a block for every CU, a block's mean number up to 1,024),
  * "deposit_chunks"
  * (waves per deposit workgroup: 2,3,4,6 for kernel 0, 4,6,12 for kernels 1
  * and 2; particles per cell per record batch, 4 or 8, for kernel 3),
