@@ -1334,7 +1334,8 @@ static void launch_fast(amps_ctx* c, TraceState* t, const typename S::View& v, c
   w.x0 = a.x0, w.dir = a.dir, w.R = a.R, w.grid = a.grid, w.lo = a.lo, w.hi = a.hi;
   w.out = a.out, w.states = a.states, w.cutoff = a.cutoff, w.pend = a.pend, w.status = a.status;
   w.stop = a.stop, w.item_steps = a.item_steps;
-  if (a.mode == TRACE_MODE_UPPER) w.nitems = a.nloc * a.nR;  // every bin an item, those outside a bracket skipped
+  // every bin an item, to the depth of the widest bracket, those outside a narrower one skipped
+  if (a.mode == TRACE_MODE_UPPER) w.nitems = a.nloc * a.nbin_item;
   if (a.mode == TRACE_MODE_BRACKET) {
     w.nitems = a.nloc * a.nbin_item;  // the rescans are handed out by ticket
     w.open_list = t->d_open;
@@ -1862,6 +1863,9 @@ extern "C" int amps_gpu_cutoff_scan(amps_ctx* c, const amps_trace_params* P, int
         if (bin_hi[i] - bin_lo[i] + 1 != w)
           return fail(AMPS_E_ARG, "cutoff_scan: FULL and BRACKETED modes need equal bracket widths");
       nbin_item = w;
+    } else {
+      nbin_item = 0;
+      for (int64_t i = 0; i < nloc; i++) nbin_item = std::max(nbin_item, bin_hi[i] - bin_lo[i] + 1);
     }
   }
   (void)hipSetDevice(c->device);
