@@ -27,6 +27,7 @@ constexpr int CELL_STRIDE_MOMENT = 272;  // 17 lines
 constexpr int NODE_STRIDE = 256;         // 16 lines
 constexpr int MAX_SPEC = 8;
 constexpr int TILE_WG = 8192;  // blocks up to which one workgroup makes the push tiles
+constexpr size_t PIN_BYTES = (size_t)16 << 20;      // pinned slots of the copies to and from the caller's arrays
 constexpr int64_t PACK_DOUBLES = (int64_t)1 << 23;  // staging of packed J and M columns (64 MiB)
 
 // Device view of the block mesh (leaf blocks of the AMR octree).

@@ -827,6 +827,7 @@ extern "C" int64_t amps_gpu_particle_count(amps_ctx* c) {
 // four integer columns 260 us against 552 there, 100 particles 92 us against 166
 // for all columns.
 constexpr int64_t GET_NARROW = (int64_t)1 << 19;
+static_assert(18 * GET_NARROW <= (int64_t)PIN_BYTES, "all narrow columns in the pinned slots");
 static int get_narrow(amps_ctx* c, int64_t n, double* v, int32_t* spec, int32_t* blk, int32_t* cell, int32_t* code) {
   const int k = c->cur;
   const std::lock_guard<std::mutex> lock(c->pin_mutex);

@@ -24,7 +24,7 @@ using namespace amps;
 
 namespace {
 constexpr int THREADS = 4, SLOTS = 2 * THREADS;
-constexpr size_t SLOT_BYTES = (size_t)2 << 20;
+constexpr size_t SLOT_BYTES = PIN_BYTES / SLOTS;
 // Sizes from which the slots are ahead (us, a plain copy and the slots): to the
 // host, 2 MiB 125 and 183, 4 MiB 248 and 237, 16 MiB 926 and 527, but where
 // the pages are not there yet 512 KiB 95 and 165, 1 MiB 259 and 200, 4 MiB 1,063 and
@@ -138,7 +138,7 @@ namespace amps {
 // pinned slots and their events; without them the copies are plain ones
 void host_copy_init(amps_ctx* c) {
   void* p = nullptr;
-  if (hipHostMalloc(&p, SLOTS * SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&p, PIN_BYTES, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     return;
   }
