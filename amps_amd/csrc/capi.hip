@@ -694,8 +694,8 @@ int amps::alloc_particles(amps_ctx* c, int64_t n) {
 // 6.4 with 8192).  Where the blocks alone are a workgroup for every CU, a tile
 // takes a block's mean number, up to 1,024, before blocks are cut up (512 blocks,
 // us with 256, 512, 1024 and 2048: 2^18 particles 51, 44, 52 and 65, 2^19 74, 66,
-// 62 and 89, 2^20 127, 101, 97 and 103; with 8192 43, 63 and 101 in the build
-// before the rule).
+// 62 and 89, 2^20 127, 101, 97 and 103; one
+// tile a block, before there was a rule, 43, 63 and 101).
 static int push_tile(const amps_ctx* c) {
   if (c->tile_given) return c->tile;
   int t = 256;
